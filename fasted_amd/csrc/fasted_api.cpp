@@ -286,7 +286,10 @@ void join_on_device(PointSet q, PointSet c, bool selfJoin, int d, double epsilon
     jl.nC = (int)c.n;
     jl.selfJoin = selfJoin;
     jl.forcedStride = forcedStride;
-    jl.symmetric = selfJoin && (flags & FASTED_SYMMETRIC);
+    if (selfJoin && (flags & FASTED_SYMMETRIC))
+        jl.triangle = fasted::Triangle::kUpper;
+    else if (selfJoin && !(flags & (FASTED_FULL_MATRIX | FASTED_NO_EPILOGUE)))
+        jl.triangle = fasted::Triangle::kAuto;
     jl.dPad = dPad;
     jl.halfQ = halfQ;
     jl.halfC = halfC;
@@ -329,7 +332,7 @@ void join_on_device(PointSet q, PointSet c, bool selfJoin, int d, double epsilon
     }
     cnt[1] = (jl.epilogue && cnt[0] > cap) ? cap : cnt[0];
     cnt[2] = fasted::tile_count(q.n, c.n);
-    if (jl.symmetric) {
+    if (jl.triangle == fasted::Triangle::kUpper) {
         const unsigned long long side = ((unsigned long long)q.n + fasted::kTile - 1) / fasted::kTile;
         cnt[2] = side * (side + 1) / 2;
     }
@@ -554,7 +557,7 @@ void self_join_blocked(const uint16_t* points, long long n, int d, double epsilo
             jl.nQ = nQ;
             jl.nC = (int)block_rows(j);
             jl.selfJoin = diagonal;
-            jl.symmetric = false;
+            jl.triangle = fasted::Triangle::kAuto;
             jl.dPad = dPad;
             jl.halfQ = halves + (size_t)i * rows;
             jl.halfC = halves + (size_t)j * rows;
@@ -807,9 +810,10 @@ Results find_pairs_resident(double epsilon, bool savePairs, bool skipUpload, con
     FastedJoinStats st{};
     const PointSet all{g_res.dPoints, tb.n, tb.dPad, nullptr};
     // a sort that fails (no memory for its buffers) is reported and the pairs leave unsorted, as the
-    // reference carries on after "Failed to sort pairs" (source/findPairs.cuh:701-718)
-    join_on_device(all, all, true, tb.dPad, epsilon, dPairs, maxPairs, FASTED_SORT_PAIRS, nullptr, &st, nullptr,
-                   /*sortMayFail=*/true);
+    // reference carries on after "Failed to sort pairs" (source/findPairs.cuh:701-718).  The whole matrix is
+    // computed: Results.TFLOPS divides 2*N*N*D by the kernel time and means operations that were executed.
+    join_on_device(all, all, true, tb.dPad, epsilon, dPairs, maxPairs, FASTED_SORT_PAIRS | FASTED_FULL_MATRIX, nullptr, &st,
+                   nullptr, /*sortMayFail=*/true);
     if (!quiet()) {
         std::printf("Number of pairs found %llu\n", st.pairsFound);
         std::printf("Number of pairs stored %llu\n", st.pairsStored);

@@ -10,6 +10,14 @@ constexpr int kTile = 256;       // points per tile side (queries x candidates)
 constexpr int kSlabK = 64;       // halves of K staged in LDS per pipeline stage
 constexpr int kSquareTiles = 256; // tiles of a super-square of the work queues: one per workgroup of a full chip
 
+// A self-join's distance matrix is bitwise symmetric, so the tiles on and above the diagonal hold every pair; the
+// pairs of the tiles above it are emitted in both orientations.
+enum class Triangle {
+    kFull,   // every tile
+    kUpper,  // tiles on and above the diagonal
+    kAuto    // whichever is the faster one at this size (launch_join)
+};
+
 struct JoinLaunch {
     const void* queries;         // FP16 rows
     const void* candidates;      // FP16 rows; the same buffer for a self-join
@@ -18,7 +26,7 @@ struct JoinLaunch {
     bool selfJoin;               // same set on both sides: (i, i) always counts as a pair
     int forcedStride = 0;        // two sets where query i IS candidate i * forcedStride (a sample of the
                                  // candidates joined against all of them): that pair always counts
-    bool symmetric;              // self-join: only tiles on/above the diagonal are computed, pairs mirrored
+    Triangle triangle = Triangle::kFull;  // self-join: which part of the distance matrix is computed
     int dPad;                    // K extent, multiple of kSlabK
     const float* halfQ;          // per query point: eps^2/4 - s/2 (s = squared norm), see launch_sum_squared
     const float* halfC;          // ... per candidate point

@@ -492,9 +492,12 @@ __global__ void __launch_bounds__(kThreads, 1) join_kernel(JoinParams p) {
             // A matrix of no more tiles than workgroups: one tile each, by workgroup number.  Through the queues,
             // every workgroup would reserve a second tile while it starts its first (the reservation runs one
             // tile ahead), and the workgroups of XCDs with short queues would find the work already taken.
-            r = blockIdx.x / p.raster.tileCols;
-            c = blockIdx.x % p.raster.tileCols;
-            if (p.symmetric && c < r) r = kNoTile;
+            if (p.symmetric) {
+                tile_order_upper_decode(blockIdx.x, &r, &c);
+            } else {
+                r = blockIdx.x / p.raster.tileCols;
+                c = blockIdx.x % p.raster.tileCols;
+            }
         } else {
             find_tile(atomicAdd(&p.counters[kQueueBase + home * kQueueStride], 1ull), &r, &c);
             if (kOneSlab && r != kNoTile) find_tile(atomicAdd(&p.counters[kQueueBase + home * kQueueStride], 1ull), &r1, &c1);
@@ -1100,7 +1103,8 @@ namespace {
 // One launch of the join kernel over the tile grid described by p.raster, in the queue or the direct mode, with
 // tiles of 256 or 128 query rows.
 hipError_t launch_join_grid(JoinParams p, bool rows128, bool tall, bool epilogue, int numCUs, hipStream_t stream) {
-    const unsigned long long realTiles = (unsigned long long)p.raster.tileRows * p.raster.tileCols;
+    const unsigned long long realTiles = p.symmetric ? (unsigned long long)p.raster.tileRows * (p.raster.tileRows + 1) / 2
+                                                     : (unsigned long long)p.raster.tileRows * p.raster.tileCols;
     // Up to two tiles per CU, workgroup b computes tile b and ends, one workgroup per tile (the hardware places
     // the second round as CUs fall free); from there on, one persistent workgroup per CU draws from the queues.
     p.direct = realTiles <= 2ull * (unsigned long long)numCUs ? 1 : 0;
@@ -1162,7 +1166,6 @@ hipError_t launch_join(const JoinLaunch& launch, hipStream_t stream) {
     p.nQ = l.nQ;
     p.nC = l.nC;
     p.selfStride = l.forcedStride > 0 ? l.forcedStride : (l.selfJoin ? 1 : 0);
-    p.symmetric = (l.selfJoin && l.symmetric) ? 1 : 0;
     p.nSlabs = l.dPad / kSlabK;
     p.halfQ = l.halfQ;
     p.halfC = l.halfC;
@@ -1170,18 +1173,24 @@ hipError_t launch_join(const JoinLaunch& launch, hipStream_t stream) {
     p.epoch = l.epoch;
     p.pairs = static_cast<int2*>(l.pairs);
     p.cap = l.cap;
-    // Tiles of 128 query rows when the matrix then still has no more tiles than the chip has workgroups (never
-    // in symmetric mode, whose diagonal logic assumes square tiles): twice as many workgroups work, each on half a
-    // tile.  A 128-row tile costs about 0.7 of a 256-row one (64 x 64 wave sub-tiles need a third more LDS fragment
-    // reads per MFMA), so the finer grid only pays while it fits one round: measured on Exp(40) data, 1000 and 2154
-    // points 1.1x - 1.4x faster, 3000 points (288 tiles of 128 rows: two rounds) 1.4x slower.
-    // FASTED_TILE_ROWS=256 or 128 in the environment overrides the choice (tests run both).
+    // What is computed, and in which tiles.  A self-join needs the tiles on and above the diagonal only (every pair of
+    // the others is the mirror image of one there, bit for bit): half the work as soon as the whole matrix would take
+    // more than one round of the workgroups.  Below that, time is set by the longest workgroup and not by the number
+    // of tiles, and a matrix whose tiles of 128 query rows (half the work of a 256-row tile per workgroup, on twice as
+    // many workgroups) still fit one round is computed in full in those: a 128-row tile costs about 0.7 of a 256-row
+    // one (64 x 64 wave sub-tiles need a third more LDS fragment reads per MFMA), measured on Exp(40) data 1.1x - 1.4x
+    // faster at 1000 and 2154 points, 1.4x slower at 3000 (288 tiles of 128 rows: two rounds).  (Never both: the
+    // diagonal logic assumes square tiles.)
+    // FASTED_TILE_ROWS=256 or 128 in the environment overrides the height (tests run both).
     const unsigned long long tiles128 = (unsigned long long)((l.nQ + 127) / 128) * ((l.nC + kTile - 1) / kTile);
-    bool rows128 = p.symmetric == 0 && tiles128 <= (unsigned long long)numCUs;
+    const bool mayMirror = l.selfJoin && l.triangle != Triangle::kFull;
+    bool rows128 = tiles128 <= (unsigned long long)numCUs;
     const char* const forced = getenv("FASTED_TILE_ROWS");  // read at every launch: a test sets it per case
     const int forcedRows = forced ? atoi(forced) : 0;
     if (forcedRows == 256) rows128 = false;
-    if (forcedRows == 128 && p.symmetric == 0) rows128 = true;
+    if (forcedRows == 128) rows128 = true;
+    if (mayMirror && l.triangle == Triangle::kUpper) rows128 = false;
+    p.symmetric = (mayMirror && !rows128) ? 1 : 0;
     const int tileRows = rows128 ? 128 : kTile;
     p.raster = make_raster(l.nQ, l.nC, p.symmetric != 0, tileRows);
     return launch_join_grid(p, rows128, tall_order(l.nQ, tileRows), l.epilogue, numCUs, stream);

@@ -88,6 +88,16 @@ FASTED_HD inline void tile_order_decode(const TileOrder& r, int subRows, int sub
     *tc = squareCol * width + (q & 1) * (unsigned)subCols + local % (unsigned)subCols;
 }
 
+// Number b of the upper triangle of a square tile matrix, column by column ((0,0), (0,1), (1,1), (0,2), ...): tile
+// (row, col), row <= col.  The square root is an estimate, then corrected.
+FASTED_HD inline void tile_order_upper_decode(unsigned b, unsigned* tr, unsigned* tc) {
+    unsigned c = (unsigned)((__builtin_sqrtf(8.0f * (float)b + 1.0f) - 1.0f) * 0.5f);
+    while (c > 0 && c * (c + 1) / 2 > b) --c;
+    while ((c + 1) * (c + 2) / 2 <= b) ++c;
+    *tc = c;
+    *tr = b - c * (c + 1) / 2;
+}
+
 // LDS placement of operand rows.  gfx950 serves a ds_read_b128 in four phases of 16 lanes --
 // {0-3,12-15,20-23,24-27}, {4-7,8-11,16-19,28-31} and the same two groups +32 -- and the fragment read
 // of v_mfma_f32_16x16x32_f16 has lane l on row l%16, 16-byte chunk l/16 of a 32-wide k-step.  A phase is

@@ -15,6 +15,7 @@ FASTED_NO_EPILOGUE = 2
 FASTED_SKIP_SUMS = 4
 FASTED_SYMMETRIC = 8
 FASTED_EVENT_TIMING = 16
+FASTED_FULL_MATRIX = 32
 
 
 def compute_selectivity(result_set_size: int, dataset_size: int) -> float:

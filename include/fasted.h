@@ -92,15 +92,19 @@ enum {
     FASTED_SORT_PAIRS = 1,  /* sort stored pairs row-major, as source/pair.cuh:151-158 */
     FASTED_NO_EPILOGUE = 2, /* measurement only: run the contraction, skip test + emit */
     FASTED_SKIP_SUMS = 4,   /* d_sums already holds the squared norms */
-    FASTED_SYMMETRIC = 8,   /* self-join only, off by default: dist(q,c) = dist(c,q), so compute only the tiles
-                               on and above the diagonal and emit both orientations of every pair found there.
-                               Same pair set, about half the matrix-core work; the reference always computes the
-                               full matrix (source/findPairs.cuh:650-653), which is also this library's default
-                               and what its TFLOPS figure assumes. */
-    FASTED_EVENT_TIMING = 16 /* time the kernels with HIP events and wait for the stream whatever the size of the
+    FASTED_SYMMETRIC = 8,   /* self-join only: compute the tiles on and above the diagonal whatever the size
+                               (dist(q,c) = dist(c,q), bit for bit) and emit both orientations of every pair found
+                               there; stats->tiles then counts those tiles.  Without it, and without
+                               FASTED_FULL_MATRIX, the library computes whichever is faster at the size: the upper
+                               triangle, except where the whole matrix fits one round of the chip's workgroups in
+                               smaller tiles.  Same pair set in every case. */
+    FASTED_EVENT_TIMING = 16, /* time the kernels with HIP events and wait for the stream whatever the size of the
                                join, as the reference does (source/findPairs.cuh:625-639,695-697): for joins of at
                                most 512 tiles this costs the call about 15 us and is what a profiler's kernel
                                durations compare with. */
+    FASTED_FULL_MATRIX = 32 /* self-join only: compute every tile of the matrix, all 2*N*N*D operations, as the
+                               reference always does (source/findPairs.cuh:650-653).  For measurements that divide
+                               2*N*N*D by the time, and for comparing the two. */
 };
 
 /* Host buffers in, host buffers out.  `points` is N x D row-major IEEE binary16 bit

@@ -155,6 +155,16 @@ static void check_tile_order() {
                 for (unsigned tc = tr; tc < o.tileCols; ++tc) CHECK(seen.count({tr, tc}) == 1);
         }
     }
+    // the upper triangle column by column, no tile left out: small matrices and the last numbers of large ones
+    for (unsigned side : {1u, 2u, 3u, 31u, 32u, 4000u}) {
+        unsigned b = 0;
+        for (unsigned c = 0; c < side; ++c)
+            for (unsigned r = 0; r <= c; ++r, ++b) {
+                unsigned tr, tc;
+                fasted::tile_order_upper_decode(b, &tr, &tc);
+                CHECK(tr == r && tc == c);
+            }
+    }
     // LDS swizzles: the 16 lanes of every ds_read_b128 phase touch all 64 banks once
     const int groups[2][16] = {{0, 1, 2, 3, 12, 13, 14, 15, 20, 21, 22, 23, 24, 25, 26, 27},
                                {4, 5, 6, 7, 8, 9, 10, 11, 16, 17, 18, 19, 28, 29, 30, 31}};

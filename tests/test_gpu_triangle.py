@@ -1,0 +1,40 @@
+"""GPU parity of the part of the distance matrix a self-join computes: the library's own choice, the upper triangle and
+the full matrix must give the same pairs record for record, at the sizes where the choice and the launch change."""
+import numpy as np
+import pytest
+
+import oracle
+from tests import datasets
+
+pytestmark = pytest.mark.gpu
+
+
+# one tile; the last size of 128-row tiles in one round (11 x 23 of 256 workgroups) and the next; one round of the full
+# matrix in 256-row tiles and the next; 31 tile rows (496 tiles above the diagonal: one workgroup each) and 32 (528: the
+# work queues); 64 tile rows (the tall order)
+@pytest.mark.parametrize("n,d", [(1, 3), (256, 64), (2816, 64), (2817, 130), (4096, 64), (4097, 130), (7936, 64),
+                                 (7937, 100), (16384, 64), (16385, 65)])
+def test_every_part_of_the_matrix_gives_the_same_pairs(n, d):
+    import torch
+
+    import fasted_amd as fasted
+    from fasted_amd import find_pairs as fp
+
+    ld = (d + 63) // 64 * 64
+    bits = np.zeros((n, ld), dtype=np.uint16)
+    bits[:, :d] = datasets.small_integers(n, d, high=3, seed=n + d)
+    sample = bits[:: max(1, n // 512)].view(np.float16).astype(np.float64)
+    d2 = np.sort(((sample[:, None, :] - sample[None, :, :]) ** 2).sum(-1), axis=1)
+    k = min(d2.shape[1] - 1, 1 + 8 * d2.shape[1] // n)
+    eps = float(np.sqrt(np.quantile(d2[:, k], 0.1).round() + 0.5))  # its square lies half-way between two integers
+    pts = torch.from_numpy(bits.view(np.int16).copy()).cuda()
+    cap = 200 * n + 1024
+    got = []
+    for flags in (fp.FASTED_FULL_MATRIX, 0, fp.FASTED_SYMMETRIC):
+        pairs = torch.full((cap, 2), -1, dtype=torch.int32, device="cuda")
+        st = fasted.self_join_device(pts.data_ptr(), n, d, ld, eps, pairs.data_ptr(), cap, flags=flags | fp.FASTED_SORT_PAIRS)
+        assert st.pairsFound == st.pairsStored
+        got.append(pairs[: st.pairsStored].cpu().numpy())
+    assert np.array_equal(got[0], got[1]) and np.array_equal(got[0], got[2])
+    if n <= 4097:
+        assert np.array_equal(got[0], oracle.self_join_f64(bits, eps))
