@@ -339,7 +339,7 @@ void join_on_device(PointSet q, PointSet c, bool selfJoin, int d, double epsilon
     float sortMs = 0.f;
     if ((flags & FASTED_SORT_PAIRS) && cnt[1] > 1) {
         const auto w0 = std::chrono::steady_clock::now();
-        const hipError_t e = fasted::sort_pairs_row_major(dPairs, cnt[1], stream, &g_sortWs, q.n, c.n);
+        const hipError_t e = fasted::sort_pairs_row_major(dPairs, cnt[1], stream, &g_sortWs, 0, q.n, c.n);
         if (e != hipSuccess) {
             (void)hipGetLastError();
             if (!sortMayFail) hip_check(e, "row-major sort of the pairs");
@@ -585,7 +585,7 @@ void self_join_blocked(const uint16_t* points, long long n, int d, double epsilo
         unsigned long long before = 0;
         HIP_CHECK(hipMemcpy(&before, g_ws.counters, sizeof before, hipMemcpyDeviceToHost));
         const unsigned long long kept = std::min(before, devCap);
-        if (kept > 1) HIP_CHECK(fasted::sort_pairs_row_major(dPairs, kept, dev.compute, &g_sortWs, n, n));
+        if (kept > 1) HIP_CHECK(fasted::sort_pairs_row_major(dPairs, kept, dev.compute, &g_sortWs, i * rows, nQ, n));
         HIP_CHECK(hipStreamSynchronize(dev.compute));
         const unsigned long long take = std::min(kept, cap - storedAll);
         if (take)

@@ -82,21 +82,26 @@ hipError_t launch_join(const JoinLaunch& p, hipStream_t stream);
 const char* build_tag();
 
 
-// Device buffers of the row-major sort (a second key buffer and the radix sort's own storage).  They only
-// grow; a caller that keeps a SortBuffers across calls sorts without allocating.
+// Device buffers of the row-major sort: keys on their way, the distribution's tables, the radix sort's own storage.  They
+// only grow; a caller that keeps a SortBuffers across calls sorts without allocating.
 struct SortBuffers {
     void* alt = nullptr;
     size_t altBytes = 0;
     void* temp = nullptr;
     size_t tempBytes = 0;
+    void* tables = nullptr;
+    size_t tableBytes = 0, cleanBytes = 0;  // the first cleanBytes hold no counts but zeros (where bins lie)
+    bool tablesDirty = false;               // a sort has not run to its end
+    unsigned long long* hostWord = nullptr;  // pinned: number of the last sort in which a bucket became too large
+    unsigned long long* hostWordDev = nullptr;
+    unsigned long long epoch = 0;            // number of the sort
     void release();
 };
-// Row-major sort of `count` stored pairs (pair_sort.hip); synchronises the stream.  With ws == nullptr the
-// buffers are allocated and freed inside the call.  On failure (no memory for the buffers) the pairs are left
-// as they were, unsorted.  nQueries / nCandidates bound the indices (0: unknown): the sort then only runs over
-// the bits the indices can occupy.
-hipError_t sort_pairs_row_major(void* pairs, unsigned long long count, hipStream_t stream, SortBuffers* ws = nullptr,
-                                long long nQueries = 0, long long nCandidates = 0);
+// Row-major sort (pair_sort.hip) of `count` distinct stored pairs whose indices lie in [firstQuery, firstQuery + nQueries)
+// and [0, nCandidates); synchronises the stream.  On failure (no memory for the buffers) the pairs are left as they
+// were, unsorted.
+hipError_t sort_pairs_row_major(void* pairs, unsigned long long count, hipStream_t stream, SortBuffers* ws,
+                                long long firstQuery, long long nQueries, long long nCandidates);
 // Device bytes a sort of `count` pairs needs beside the pairs themselves.
 size_t sort_scratch_bytes(unsigned long long count);
 
