@@ -1,0 +1,42 @@
+"""GPU parity of the distance column where the candidates are worked off in slices: every row length class of the sliced
+kernel, row-major and shuffled lists, with pairs that name no point."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+# dPad = 256, 320 ... 4096: 32, 40, 64, 72, 128, 136, 192, 200, 256, 264, 384, 392, 440, 512 chunks of 16 bytes; 520 (too long);
+# more than 8 slices; both batch sizes
+@pytest.mark.parametrize("n,d", [(9001, 256), (8001, 300), (5003, 512), (4500, 576), (3001, 1000), (2500, 1088), (2000, 1536),
+                                 (2000, 1600), (1500, 2048), (1400, 2112), (1300, 3071), (1300, 3136), (1200, 3500),
+                                 (1100, 4096), (1100, 4160), (20001, 4096), (40011, 260)])
+def test_sliced_distances_match_fp64(n, d):
+    import torch
+
+    import fasted_amd as fasted
+
+    gen = torch.Generator(device="cuda").manual_seed(n + d)
+    ld = (d + 63) // 64 * 64
+    count = max(8 * n + 7, (3 << 29) // (2 * ld) + 5)  # the smallest lists that go through the slices
+    pts = torch.zeros((n, ld), dtype=torch.float16, device="cuda")
+    pts[:, :d] = torch.randn((n, d), generator=gen, device="cuda").to(torch.float16)
+    pairs = torch.randint(0, n, (count, 2), generator=gen, device="cuda", dtype=torch.int32)
+    half = count // 2
+    pairs[:half] = pairs[:half][torch.argsort(pairs[:half, 0].long() * n + pairs[:half, 1])]
+    pairs[-1] = torch.tensor([n - 1, n - 1])
+    bad = torch.tensor([3, half, count - 2], device="cuda")
+    pairs[bad] = torch.tensor([[-1, 0], [0, n], [n, -1]], dtype=torch.int32, device="cuda")
+    got = torch.full((count + 1,), -2.0, dtype=torch.float32, device="cuda")
+    fasted.pair_distances_device(pts.data_ptr(), n, ld, pts.data_ptr(), n, ld, d, pairs.data_ptr(), count, got.data_ptr())
+    assert float(got[-1]) == -2.0
+    assert torch.isnan(got[bad]).all()
+    step = max(1, (1 << 26) // d)
+    for r in range(0, count, step):
+        i = pairs[r : r + step].long()
+        ok = (i >= 0).all(1) & (i < n).all(1)
+        i = i[ok]
+        want = (pts[i[:, 0]].double() - pts[i[:, 1]].double()).norm(dim=1)
+        # each of d products and additions rounds to half a unit of 2^-24 at most; the square root halves it
+        bound = 1e-7 + 0.5 * (ld / 16 + 20) * 2.0**-24
+        assert bool(((got[r : r + step][: len(ok)][ok].double() - want).abs() <= bound * want).all())
