@@ -65,6 +65,8 @@ hipError_t launch_sum_squared(const void* points, long long ld, int n, int dPad,
 // The same halves from norms that are already there.
 hipError_t launch_halves(const float* sums, int n, float eps2, float* halves, unsigned long long* counters,
                          hipStream_t stream, unsigned long long epoch = 1, bool reset = false);
+// rows x d halves, packed -> rows x dPad halves, the columns d .. dPad-1 zero.  dst is 16-byte aligned, src 2-byte.
+hipError_t launch_pad_rows(const void* src, int d, void* dst, int dPad, long long rows, hipStream_t stream);
 // *badRows += number of rows whose columns d .. dPad-1 are not all zeros.
 hipError_t launch_padding_check(const void* points, long long ld, int n, int d, int dPad, unsigned long long* badRows,
                                 hipStream_t stream);

@@ -902,7 +902,7 @@ hipError_t launch_pair_distances(const void* queries, long long ldQ, int nQ, con
     const u64 rowBytes = (u64)dPad * 2, bytes = rowBytes * (u64)nC, sliceBytes = 6ull << 20;
     const u64 slices = 8 * ((bytes + 8 * sliceBytes - 1) / (8 * sliceBytes));
     if (bytes <= 4ull << 20 || slices > rowBytes / 64 || count / 8 < (u64)nC || count * rowBytes < 3ull << 29 ||
-        count > 1ull << 30 || chunks > 64 * 8) {
+        count > 1ull << 30 || count / 2048 * slices >= 1ull << 23 || chunks > 64 * 8) {
         const u64 blocks = (count * 16 + 255) / 256;
         pair_distances_kernel<<<dim3((unsigned)(blocks > 16384ull ? 16384ull : blocks)), dim3(256), 0, stream>>>(
             q, ldQ / 8, nQ, c, ldC / 8, nC, chunks, list, count, out);
