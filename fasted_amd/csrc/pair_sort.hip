@@ -56,7 +56,7 @@ int index_bits(long long n) {  // bits of the largest index of n items; 32 when 
 // Bound by memory traffic: 32 bytes per record in one level, 44 in two, of which a key on its way is 4 (the radix sort
 // with its pack and unpack moves 120 at 36 key bits); below a million records by the launches.  Measured, join records,
 // radix sort -> this: 4 849 records 45 -> 18 us, 135 thousand 75 -> 34, 974 thousand 195 -> 55, 6.5 million 330 -> 160,
-// 200 million 7.5 -> 2.5 ms.  Where the lines between one workgroup, one level and two lie: one workgroup takes 8192
+// 200 million 7.5 -> 2.6 ms.  Where the lines between one workgroup, one level and two lie: one workgroup takes 8192
 // records in 22 us, two launches less than the 32 us of one level; one level takes 2^20 records in 60 us, and beyond
 // that its buckets grow past what a workgroup can tell apart.
 typedef unsigned int u32;
