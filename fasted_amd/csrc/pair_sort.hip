@@ -881,7 +881,10 @@ hipError_t sort_pairs_row_major(void* pairs, unsigned long long count, hipStream
     bool done = false;
     if (make_plan(count, lastKey, &p)) {
         const hipError_t e = distribute(records, (u32)count, p, lastKey, form, stream, ws, &done);
-        if (e != hipSuccess) return e;
+        if (e == hipErrorOutOfMemory)
+            (void)hipGetLastError();  // nothing was launched; the radix sort may need less
+        else if (e != hipSuccess)
+            return e;
     }
     return done ? hipSuccess : radix_sort(records, count, form, queryBits + candidateBits, stream, ws);
 }
