@@ -5,8 +5,8 @@
 // then candidate index; source/pair.cuh:39-45,151-158).  A pair is 8 bytes with the query
 // index in the low word; packed as (query << bits of a candidate index) | candidate that order is plain
 // unsigned order.  Two ways to it: distribution into buckets that fit a workgroup's LDS (see below), and, for what
-// that does not take (more than 2^29 records, keys of more than 42 bits, hundreds of thousands of pairs in a small
-// part of one row), rocPRIM's radix sort over the bits the indices can occupy: pack, sort, unpack.
+// that does not take (more than 2^29 records, keys of more than 42 bits, lists it breaks off because they crowd into
+// a few rows), rocPRIM's radix sort over the bits the indices can occupy: pack, sort, unpack.
 #include <cstring>
 #include <type_traits>
 
@@ -47,18 +47,24 @@ int index_bits(long long n) {  // bits of the largest index of n items; 32 when 
 // are distinct and, apart from clustering, spread evenly, so a record's place is found by counting instead of by
 // passes over all key bits:
 //   count_keys_kernel     how many records fall into each of at most 4096 equal key ranges (bins)
-//   plan_buckets_kernel   prefix sums over the bins; runs of bins become buckets of about `target` records (a bucket
-//                         never crosses a multiple of 2^32, so the low word of the key is enough from here on)
+//   plan_buckets_kernel   prefix sums over the bins; runs of bins become buckets of about `target` records, 512 to 1365
+//                         (a bucket never crosses a multiple of 2^32, so the low word of the key is enough from here on)
 //   scatter_keys_kernel   every record's low key word goes to its bucket, in any order inside the bucket
 //   sort_bucket_kernel    one workgroup orders a bucket of up to 4096 keys in LDS and writes the records out
 // From 2^20 records on the first three run twice, the second time on every bucket of the first by itself (1024 bins
-// each).  A few times 4096 records are ordered by one workgroup alone (sort_bucket_kernel on the records themselves).
+// each).  A bucket of more than 4096 keys is a bin that is crowded by itself; the last kernel orders it in windows
+// (order_windows).  Too many windows: one level breaks off after its plan and starts again with two, where a bin covers at
+// most 16 windows; lists of less than 2^18 records, and bins that two levels cannot cut small enough (millions of records
+// in 1/4096 of the key range), go to the radix sort.  A few times 4096 records are ordered by one workgroup alone (sort_bucket_kernel on the records themselves).
 // Bound by memory traffic: 32 bytes per record in one level, 44 in two, of which a key on its way is 4 (the radix sort
 // with its pack and unpack moves 120 at 36 key bits); below a million records by the launches.  Measured, join records,
-// radix sort -> this: 4 849 records 45 -> 18 us, 135 thousand 75 -> 34, 974 thousand 195 -> 55, 6.5 million 330 -> 160,
-// 200 million 7.5 -> 2.6 ms.  Where the lines between one workgroup, one level and two lie: one workgroup takes 8192
-// records in 22 us, two launches less than the 32 us of one level; one level takes 2^20 records in 60 us, and beyond
-// that its buckets grow past what a workgroup can tell apart.
+// radix sort -> this: 4 849 records 45 -> 18 us, 135 thousand 75 -> 34, 974 thousand 195 -> 40, 6.5 million 330 -> 160,
+// 200 million 7.5 -> 2.6 ms; 1.04 million in 200 000 rows 200 -> 54, 0.6 million of which 0.4 in 2000 of 100 000 rows 165
+// -> 75.  Slower where a list that breaks off is short, or one row holds most of a long one: 100 thousand records, half of
+// them in one row of a million, 71 -> 99 us, 3 million, half of them in one row of two million, 262 -> 324.
+// Where the lines between one workgroup, one level and two lie: one workgroup takes 8192 records in 22 us, two launches
+// less than the 32 us of one level; one level takes 1.04 million records in 53 us, two take 1.1 million in 65.  Where a list
+// breaks off, two levels took 500 thousand records in 150 us and the radix sort 180, 100 thousand in 140 and 100.
 typedef unsigned int u32;
 typedef unsigned long long u64;
 typedef u32 u32x4 __attribute__((ext_vector_type(4)));
@@ -68,14 +74,21 @@ constexpr int kBucketThreads = 512, kBucketCap = 4096; // a workgroup that order
 constexpr u32 kTargetMax = kBucketCap / 3;              // up to one target plus a bin of less than two share a bucket
 constexpr int kBins1 = 4096, kBins2Bits = 10, kBins2 = 1 << kBins2Bits;
 constexpr int kMaxIds = 2048;                         // buckets one workgroup of scatter_keys_kernel can tell apart
-constexpr int kWindowBits = 18;                       // bits of the LDS that sort_bucket_kernel uses as a bit map
-static_assert(1 << kWindowBits == 2 * kBucketCap * 32, "the bit map is the two key arrays");
+constexpr int kWindowBits = 18;                       // key range that a workgroup marks in a bit map in LDS
+static_assert(1 << kWindowBits == 2 * kBucketCap * 32, "the bit map is the two key arrays of sort_bucket_kernel");
+constexpr int kWindowWorkers = 256;                   // workgroups of sort_bucket_kernel that work on windows
+constexpr u32 kWindowsOneLevel = 1024;                // one level breaks off where there are more windows than this, or a
+constexpr u64 kReadsOneLevel = 1ull << 24;            // bucket's keys would be read more often than this
+constexpr int kWindowNumberBits = 12;                 // a window is stored as bucket << kWindowNumberBits | number
 constexpr u32 kCellMax = 48;                          // cells fuller than this: the bucket goes through the bitonic network
 
-// Can one workgroup order a bucket of `size` keys that lie within `range` of each other?  In LDS, or in a bit map that it
-// fills window by window, reading the keys every time: up to 4 million reads, about 50 us.
-__device__ __forceinline__ bool bucket_fits(u32 size, u64 range) {
-    return size <= (u32)kBucketCap || (u64)size * ((range >> kWindowBits) + 1) <= (1ull << 22);
+// What the kernels of a sort tell each other, in front of the tables.
+struct SortState {
+    u64 brokenOff[2];  // number of the last sort that the plan of the first, of the second level has broken off
+    u32 windows;       // windows of the buckets that are too large for the LDS
+};
+__device__ __forceinline__ bool broken_off(const SortState* s, u64 epoch) {
+    return s->brokenOff[0] == epoch || s->brokenOff[1] == epoch;
 }
 
 struct Bucket {
@@ -111,13 +124,17 @@ __device__ __forceinline__ u32 find_bucket(const Bucket* __restrict__ buckets, u
 template <bool kRecords>
 __global__ void __launch_bounds__(kSortThreads) count_keys_kernel(const void* __restrict__ in, u32 count, KeyForm form,
                                                                   int shift, const Bucket* __restrict__ parents,
-                                                                  u32 parentCount, u32 chunk, u32* __restrict__ bins) {
+                                                                  u32 parentCount, u32 chunk, u32* __restrict__ bins,
+                                                                  SortState* __restrict__ state, u64 epoch) {
     constexpr int kBins = kRecords ? kBins1 : kBins2;
     typedef std::conditional_t<kRecords, u64, u32> Key;
     __shared__ u32 local[kBins];
     __shared__ u32 which;
     u32 begin = blockIdx.x * chunk, end = min(count - begin, chunk) + begin, lo = 0;
-    if (!kRecords) {
+    if (kRecords) {
+        if (blockIdx.x == 0 && threadIdx.x == 0) state->windows = 0;
+    } else {
+        if (broken_off(state, epoch)) return;
         const u32 b = find_bucket(parents, parentCount, blockIdx.x, chunk, &which);
         if (b == ~0u) return;
         const Bucket p = parents[b];
@@ -177,10 +194,11 @@ __device__ __forceinline__ u32 block_exclusive_scan(u32 v, u32* waveSums) {
 template <bool kFirst>
 __global__ void __launch_bounds__(kSortThreads) plan_buckets_kernel(u32* __restrict__ bins, u32 count, int shift, u32 lastHigh,
                                                                     u32 lastLow, const Bucket* __restrict__ parents, u32 target,
-                                                                    u32 childCount, bool final, Bucket* __restrict__ children,
+                                                                    u32 childCount, u32 nextTarget, Bucket* __restrict__ children,
                                                                     unsigned short* __restrict__ childOfBin,
-                                                                    u32* __restrict__ cursors, u64 epoch,
-                                                                    u64* __restrict__ tooLarge, u64* tooLargeHost) {
+                                                                    u32* __restrict__ cursors, u32* __restrict__ windowList,
+                                                                    u32 maxWindows, SortState* __restrict__ state, u64 epoch,
+                                                                    u64* brokenOffHost) {
     constexpr int kBins = kFirst ? kBins1 : kBins2;
     constexpr int kPer = kBins / kSortThreads;
     __shared__ u32 waveSums[kSortThreads / 64];
@@ -188,6 +206,7 @@ __global__ void __launch_bounds__(kSortThreads) plan_buckets_kernel(u32* __restr
     Bucket p{0u, count, 0u, 0u, lastLow, 0u, {0u, 0u}};
     u32 firstChild = 0, ids = childCount;
     if (!kFirst) {
+        if (state->brokenOff[0] == epoch) return;  // (the other one may turn while this kernel runs)
         p = parents[blockIdx.x];
         shift = (int)p.shift;
         firstChild = p.start / target + blockIdx.x;
@@ -197,8 +216,6 @@ __global__ void __launch_bounds__(kSortThreads) plan_buckets_kernel(u32* __restr
         children += firstChild;
         cursors += firstChild;
     }
-    const bool tooMany = !kFirst && ids > (u32)kMaxIds;  // more than scatter_keys_kernel can tell apart
-    if (tooMany) ids = kMaxIds;
     for (u32 i = threadIdx.x; i < (u32)kMaxIds; i += kSortThreads) firstOf[i] = ~0u;
     u32 n[kPer], sum = 0;
 #pragma unroll
@@ -223,7 +240,7 @@ __global__ void __launch_bounds__(kSortThreads) plan_buckets_kernel(u32* __restr
         startOf[kBins] = p.end - p.start;
     }
     __syncthreads();
-    bool large = tooMany;
+    bool breakOff = false;
 #pragma unroll
     for (int e = 0; e < kPer; ++e) {
         const u32 i = threadIdx.x * kPer + e;
@@ -257,14 +274,25 @@ __global__ void __launch_bounds__(kSortThreads) plan_buckets_kernel(u32* __restr
             const u64 range = highest - lowest;
             const int bits = 64 - __clzll((long long)range);
             children[id].shift = (u32)(bits > kBins2Bits ? bits - kBins2Bits : 0);
-            large |= final && !bucket_fits(startOf[i + 1] - startOf[first], range);
+            const u32 size = startOf[i + 1] - startOf[first];
+            if (nextTarget) {
+                // cut into at most size / nextTarget + 2 at the next level: as many as scatter_keys_kernel can tell apart?
+                breakOff |= size / nextTarget + 2 > (u32)kMaxIds;
+            } else if (size > (u32)kBucketCap) {
+                const u64 windows = (range >> kWindowBits) + 1;
+                const bool few = windows <= min(maxWindows, 1u << kWindowNumberBits) && (!kFirst || size * windows <= kReadsOneLevel);
+                const u32 at = few ? atomicAdd(&state->windows, (u32)windows) : 0u;
+                breakOff |= !few || at + (u32)windows > maxWindows;
+                if (!breakOff)
+                    for (u32 w = 0; w < (u32)windows; ++w) windowList[at + w] = (firstChild + id) << kWindowNumberBits | w;
+            }
         }
     }
     if (threadIdx.x == kSortThreads - 1)
         for (u32 s = idOf[kBins - 1] + 1; s < ids; ++s) children[s] = Bucket{p.end, p.end, 0u, 0u, 0u, 0u, {0u, 0u}};
-    if (large) {
-        *tooLarge = epoch;
-        __hip_atomic_store(tooLargeHost, epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    if (breakOff) {
+        state->brokenOff[kFirst ? 0 : 1] = epoch;
+        __hip_atomic_store(brokenOffHost, epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
 }
 
@@ -278,7 +306,7 @@ __global__ void __launch_bounds__(kSortThreads) scatter_keys_kernel(const void* 
                                                                     u32 parentCount, u32 target, u32 childCount,
                                                                     const unsigned short* __restrict__ childOfBin,
                                                                     u32* __restrict__ cursors, u32* __restrict__ out, u64 epoch,
-                                                                    const u64* __restrict__ tooLarge) {
+                                                                    const SortState* __restrict__ state) {
     constexpr u32 kChunk = kPerThread * kSortThreads;
     constexpr int kBins = kRecords ? kBins1 : kBins2;
     typedef std::conditional_t<kRecords, u64, u32> Key;
@@ -287,7 +315,7 @@ __global__ void __launch_bounds__(kSortThreads) scatter_keys_kernel(const void* 
     __shared__ unsigned short child[kBins], keyChild[kChunk];
     __shared__ u32 waveSums[kSortThreads / 64];
     __shared__ u32 which;
-    if (*tooLarge == epoch) return;
+    if (broken_off(state, epoch)) return;
     u32 begin = blockIdx.x * kChunk, end = min(count - begin, kChunk) + begin, lo = 0, ids = childCount;
     if (!kRecords) {
         const u32 b = find_bucket(parents, parentCount, blockIdx.x, kChunk, &which);
@@ -356,17 +384,103 @@ __global__ void __launch_bounds__(kSortThreads) scatter_keys_kernel(const void* 
     for (u32 i = threadIdx.x; i < end - begin; i += kSortThreads) out[local[keyChild[i]] + i] = keys[i];
 }
 
+// Windows of the buckets that are too large for the LDS: a workgroup reads all keys of the bucket, marks those of its
+// window of 2^18 in a bit map and counts those below it, which is where the window's records begin; the windows of a
+// bucket know nothing of each other.  Bound by the instructions per key (read, compare, mark), about 10 keys a nanosecond
+// and workgroup.  Full chunks of a window leave in runs of up to 64 records (a lane's next records lie 256 bytes from its
+// neighbour's otherwise: 64 lines a store), thin ones record by record.
+// Measured, whole sorts, one workgroup that goes through all windows of a bucket -> this: a row of a million records, four
+// windows, 355 -> 167 us; 20 thousand records, half of them in one row of 300 000, 256 windows, 1450 -> 50; three million,
+// half of them in one row of two million, 2598 -> 324.
+template <int kThreads, int kWords>
+__device__ __forceinline__ void order_windows(const u32* __restrict__ in, const Bucket* __restrict__ buckets,
+                                              const u32* __restrict__ windowList, u32 windows, KeyForm form,
+                                              u64* __restrict__ records, u32* bits, u32* waveSums, u32* below) {
+    typedef u32 LooseU32x4 __attribute__((ext_vector_type(4), aligned(4)));
+    constexpr int kChunks = kWords / 64, kUnroll = 2;  // a wave writes out 64 words, a chunk, at a time
+    constexpr u32 kThin = 768;                         // records of a chunk that leave one by one
+    static_assert(kWords * 32 == 1 << kWindowBits && kWords % (4 * kThreads) == 0 && kChunks * 4 == kThreads, "window");
+    __shared__ u32 chunkAt[kChunks];
+    const u32 t = threadIdx.x, lane = t & 63;
+    for (u32 u = blockIdx.x; u < windows; u += kWindowWorkers) {
+        const u32 number = windowList[u] & ((1u << kWindowNumberBits) - 1u);
+        const Bucket b = buckets[windowList[u] >> kWindowNumberBits];
+        const u32* const keys = in + b.start;
+        const u32 m = b.end - b.start, fours = m / 4;
+        for (int i = 0; i < kWords / 4 / kThreads; ++i) reinterpret_cast<u32x4*>(bits)[i * kThreads + t] = u32x4{0u, 0u, 0u, 0u};
+        __syncthreads();
+        u32 less = 0;
+        auto mark = [&](u32 key) {
+            const u32 at = key - b.lo, w = at >> kWindowBits;
+            if (w == number) atomicOr(&bits[(at & ((1u << kWindowBits) - 1u)) >> 5], 1u << (at & 31u));
+            less += w < number ? 1u : 0u;
+        };
+        for (u32 base = 0; base < fours; base += kUnroll * kThreads) {
+            u32x4 four[kUnroll];
+#pragma unroll
+            for (int e = 0; e < kUnroll; ++e) four[e] = reinterpret_cast<const LooseU32x4*>(keys)[min(base + e * kThreads + t, fours - 1)];
+#pragma unroll
+            for (int e = 0; e < kUnroll; ++e)
+                if (base + e * kThreads + t < fours) {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) mark(four[e][i]);
+                }
+        }
+        if (t < m % 4) mark(keys[fours * 4 + t]);
+        const u32 lessBefore = block_exclusive_scan<kThreads>(less, waveSums);  // (its barrier: the bits are set)
+        if (t == kThreads - 1) *below = lessBefore + less;
+        // where the records of every chunk go: four threads count one, each 16 words (not all from the same bank)
+        u32 n = 0;
+#pragma unroll
+        for (u32 i = 0; i < 16; ++i) n += __popc(bits[t * 16 + ((i + t) & 15)]);
+        n += __shfl_xor(n, 1, 64);
+        n += __shfl_xor(n, 2, 64);
+        const u32 before = block_exclusive_scan<kThreads>(t % 4 == 0 ? n : 0u, waveSums);
+        if (t % 4 == 0) chunkAt[t / 4] = b.start + *below + before;
+        __syncthreads();
+        const u32 lowest = b.lo + (number << kWindowBits), candidates = (1u << form.candidateBits) - 1u;
+        auto put = [&](u64* record, u32 bit) {
+            const u32 low = lowest + bit;
+            *record = (u64)(low & candidates) << 32 | (__builtin_amdgcn_alignbit(b.window, low, form.candidateBits) + form.firstQuery);
+        };
+        for (u32 c = t / 64; c < (u32)kChunks; c += kThreads / 64) {
+            u32 word = bits[c * 64 + lane];
+            if (__builtin_amdgcn_ballot_w64(word != 0u) == 0ull) continue;
+            u64* out = records + __builtin_amdgcn_readfirstlane(chunkAt[c]);
+            u32 x = __popc(word);
+            const u32 mine = x;
+#pragma unroll
+            for (int off = 1; off < 64; off <<= 1) {
+                const u32 y = __shfl_up(x, off, 64);
+                if (lane >= (u32)off) x += y;
+            }
+            if (__builtin_amdgcn_readlane(x, 63) <= kThin) {
+                for (out += x - mine; word; word &= word - 1) put(out++, (c * 64 + lane) * 32 + (__ffs(word) - 1));
+            } else {
+                for (int j = 0; j < 64; j += 2) {
+                    const u32 even = __builtin_amdgcn_readlane(word, j), odd = __builtin_amdgcn_readlane(word, j + 1);
+                    if ((lane < 32 ? even : odd) >> (lane & 31) & 1)
+                        put(out + __builtin_amdgcn_mbcnt_hi(odd, __builtin_amdgcn_mbcnt_lo(even, 0u)), (c * 64 + j) * 32 + lane);
+                    out += __popc(even) + __popc(odd);
+                }
+            }
+        }
+        __syncthreads();  // the bits and where they go are read
+    }
+}
+
 // One bucket.  The key range is cut into at least as many cells as there are keys (half or all of the capacity): a key's cell gives its rank
 // up to the few keys that share the cell, which are then counted one by one.  Where keys crowd into few cells (runs of
 // consecutive candidates, say), a cell's own key range, from its smallest to its largest key, is cut once more, into as
-// many cells as it has keys; what is still crowded then goes through a bitonic network.  A bucket of more keys than
-// the LDS holds (see bucket_fits) is marked in a bit map, one window of 2^18 keys after the other.
+// many cells as it has keys; what is still crowded then goes through a bitonic network.  The first kWindowWorkers
+// workgroups see to the buckets of more keys than the LDS holds.
 // Bound by LDS latency between barriers, so four workgroups of 512 share a CU (64 registers; the spills lie on the
 // crowded path): 60 million keys 231 us, 380 us with 1024 threads and 8192 keys, two to a CU.
 template <bool kRecords, int kThreads, int kCap>
 __global__ void __launch_bounds__(kThreads, kRecords ? 4 : 8) sort_bucket_kernel(const void* in, const Bucket* __restrict__ buckets,
-                                                                   Bucket whole, KeyForm form, u64* records, u64 epoch,
-                                                                   const u64* __restrict__ tooLarge) {
+                                                                   Bucket whole, KeyForm form, u64* records,
+                                                                   const u32* __restrict__ windowList, u64 epoch,
+                                                                   const SortState* __restrict__ state) {
     __shared__ __align__(16) u32 lds[2 * kCap];
     __shared__ u32 waveSums[kThreads / 64];
     __shared__ u32 fullest, half;
@@ -375,9 +489,15 @@ __global__ void __launch_bounds__(kThreads, kRecords ? 4 : 8) sort_bucket_kernel
     u32* const cells = lds;
     u32* const keys = lds + kCap;
     Bucket b = whole;
-    if (!kRecords) {
-        if (*tooLarge == epoch) return;
-        b = buckets[blockIdx.x];
+    if constexpr (!kRecords) {
+        if (broken_off(state, epoch)) return;
+        if (blockIdx.x < (u32)kWindowWorkers) {
+            order_windows<kThreads, 2 * kCap>(static_cast<const u32*>(in), buckets, windowList, state->windows, form, records,
+                                              lds, waveSums, &half);
+            return;
+        }
+        b = buckets[blockIdx.x - kWindowWorkers];
+        if (b.end - b.start > (u32)kCap) return;
     }
     const u32 m = b.end - b.start;
     if (m == 0) return;
@@ -387,32 +507,6 @@ __global__ void __launch_bounds__(kThreads, kRecords ? 4 : 8) sort_bucket_kernel
         const u64 k = high | low;
         records[b.start + at] = ((k & mask) << 32) | (u32)((u32)(k >> form.candidateBits) + form.firstQuery);
     };
-    if (!kRecords && m > (u32)kCap) {
-        const u32* const all = static_cast<const u32*>(in) + b.start;
-        u32 written = 0;
-        for (u32 w = 0; w <= (b.last - b.lo) >> kWindowBits; ++w) {
-            for (int i = t; i < 2 * kCap; i += kThreads) lds[i] = 0;
-            __syncthreads();
-            for (u32 i = t; i < m; i += kThreads) {
-                const u32 at = all[i] - b.lo;
-                if (at >> kWindowBits == w) atomicOr(&lds[(at & ((1u << kWindowBits) - 1u)) >> 5], 1u << (at & 31u));
-            }
-            __syncthreads();
-            u32 sum = 0;
-            for (int e = 0; e < 2 * kPer; ++e) sum += __popc(lds[t * 2 * kPer + e]);
-            u32 before = block_exclusive_scan<kThreads>(sum, waveSums);
-            if (t == kThreads - 1) fullest = before + sum;  // keys of this window
-            for (int e = 0; e < 2 * kPer; ++e) {
-                const u32 word = t * 2 * kPer + e;
-                for (u32 bits = lds[word]; bits; bits &= bits - 1)
-                    put_record(written + before++, b.lo + (w << kWindowBits) + word * 32 + (__ffs(bits) - 1));
-            }
-            __syncthreads();
-            written += fullest;
-            __syncthreads();
-        }
-        return;
-    }
     const u32 nCells = m <= kCap / 2 ? kCap / 2 : kCap;
     const bool two = nCells == kCap;  // cells 4t .. 4t + 3 belong to thread t, and with all cells those half the capacity further on
     u32 key[kPer], cell[kPer];
@@ -719,26 +813,31 @@ struct SortPlan {
     int shift;               // first level: bin = key >> shift
     u32 target1, ids1, ids2; // two levels: records per first-level bucket; buckets of each level (one level: ids1 only)
     u32 target;              // records per bucket that is ordered in LDS
-    size_t cursors1, cursors2, buckets1, buckets2, bins2, childOf1, childOf2, bytes;  // byte offsets in `tables`
+    u32 maxWindows;          // room for windows of buckets that are too large for the LDS
+    size_t cursors1, cursors2, buckets1, buckets2, bins2, childOf1, childOf2, windowList, bytes;  // byte offsets in `tables`
 };
 constexpr u64 kTwoLevelsFrom = 1ull << 20;
+constexpr u64 kTwoLevelsAfterOneFrom = 1ull << 18;  // fewer records go from a distribution that broke off to the radix sort
 constexpr u64 kDistributeUpTo = 1ull << 29;
-constexpr size_t kBins1At = 64;  // word 0: the flag of a bucket that became too large; then the first level's bins
+constexpr size_t kBins1At = 64;  // the SortState, then the first level's bins
 
 // false: too many records, or keys of more than 42 bits (a first-level bin would cover more than 2^32 of them)
-bool make_plan(u64 count, u64 lastKey, SortPlan* p) {
+bool make_plan(u64 count, u64 lastKey, bool twoLevels, SortPlan* p) {
     if (count > kDistributeUpTo || lastKey >> 42) return false;
     p->shift = 0;
     while ((lastKey >> p->shift) >= (u64)kBins1) ++p->shift;
     const u32 windows = (u32)(lastKey >> 32) + 1;
-    p->twoLevels = count > kTwoLevelsFrom;
+    p->twoLevels = twoLevels;
     p->target = kTargetMax;
     if (!p->twoLevels) {
         // small joins: as many buckets as the chip has compute units to work on them, if that leaves them 512 records
         u64 target = (count + 255) / 256;
         if (target < 512) target = 512;
-        p->target = (u32)target;
+        if (target < p->target) p->target = (u32)target;
     }
+    // Two levels: a bucket too large for the LDS is a single bin of at most 2^32 / kBins2 keys, 16 windows, so there are
+    // fewer than count / 256 of them in all.
+    p->maxWindows = twoLevels ? (u32)(count >> 8) : kWindowsOneLevel;
     // two levels: about as many buckets in the first as in each of those in the second
     p->target1 = p->twoLevels ? (u32)__builtin_sqrt((double)count * p->target) : p->target;
     p->ids1 = (u32)(count / p->target1) + windows + 1;
@@ -758,6 +857,7 @@ bool make_plan(u64 count, u64 lastKey, SortPlan* p) {
     p->buckets2 = place(p->ids2 * sizeof(Bucket));
     p->childOf1 = place(kBins1 * sizeof(unsigned short));
     p->childOf2 = place(p->twoLevels ? (size_t)p->ids1 * kBins2 * sizeof(unsigned short) : 0);
+    p->windowList = place(p->maxWindows * sizeof(u32));
     p->bytes = at;
     return true;
 }
@@ -784,7 +884,7 @@ hipError_t distribute(u64* records, u32 count, const SortPlan& p, u64 lastKey, K
     }
     ws->tablesDirty = true;
     char* const base = static_cast<char*>(ws->tables);
-    u64* const flag = reinterpret_cast<u64*>(base);
+    auto* const state = reinterpret_cast<SortState*>(base);
     u32* const bins1 = reinterpret_cast<u32*>(base + kBins1At);
     u32* const bins2 = reinterpret_cast<u32*>(base + p.bins2);
     u32* const cursors1 = reinterpret_cast<u32*>(base + p.cursors1);
@@ -793,6 +893,7 @@ hipError_t distribute(u64* records, u32 count, const SortPlan& p, u64 lastKey, K
     Bucket* const buckets2 = reinterpret_cast<Bucket*>(base + p.buckets2);
     auto* const childOf1 = reinterpret_cast<unsigned short*>(base + p.childOf1);
     auto* const childOf2 = reinterpret_cast<unsigned short*>(base + p.childOf2);
+    u32* const windowList = reinterpret_cast<u32*>(base + p.windowList);
     const u64 epoch = ++ws->epoch;
     const u32 lastHigh = (u32)(lastKey >> 32), lastLow = (u32)lastKey;
     const dim3 threads(kSortThreads);
@@ -801,34 +902,38 @@ hipError_t distribute(u64* records, u32 count, const SortPlan& p, u64 lastKey, K
     u32* const keysB = keysA + count;
     const Bucket none{};
     if (!p.twoLevels) {
-        count_keys_kernel<true><<<blocks(count, 4096), threads, 0, stream>>>(records, count, form, p.shift, nullptr, 0u, 4096u, bins1);
-        plan_buckets_kernel<true><<<1, threads, 0, stream>>>(bins1, count, p.shift, lastHigh, lastLow, nullptr, p.target, p.ids1,
-                                                             true, buckets1, childOf1, cursors1, epoch, flag, ws->hostWordDev);
+        count_keys_kernel<true><<<blocks(count, 4096), threads, 0, stream>>>(records, count, form, p.shift, nullptr, 0u, 4096u, bins1, state, epoch);
+        plan_buckets_kernel<true><<<1, threads, 0, stream>>>(bins1, count, p.shift, lastHigh, lastLow, nullptr, p.target, p.ids1, 0u,
+                                                             buckets1, childOf1, cursors1, windowList, p.maxWindows, state, epoch,
+                                                             ws->hostWordDev);
         scatter_keys_kernel<true, 4><<<blocks(count, 4096), threads, 0, stream>>>(records, count, form, p.shift, nullptr, 0u, p.target,
-                                                                                  p.ids1, childOf1, cursors1, keysA, epoch, flag);
-        sort_bucket_kernel<false, kBucketThreads, kBucketCap><<<p.ids1, kBucketThreads, 0, stream>>>(keysA, buckets1, none, form, records, epoch, flag);
+                                                                                  p.ids1, childOf1, cursors1, keysA, epoch, state);
+        sort_bucket_kernel<false, kBucketThreads, kBucketCap><<<p.ids1 + kWindowWorkers, kBucketThreads, 0, stream>>>(
+            keysA, buckets1, none, form, records, windowList, epoch, state);
     } else {
         const u32 chunk1 = (u32)((count / 1024 + 4095) / 4096 * 4096 + 4096), chunk2 = 32768;
         constexpr u32 kScatter = 8 * kSortThreads;
-        count_keys_kernel<true><<<blocks(count, chunk1), threads, 0, stream>>>(records, count, form, p.shift, nullptr, 0u, chunk1, bins1);
-        plan_buckets_kernel<true><<<1, threads, 0, stream>>>(bins1, count, p.shift, lastHigh, lastLow, nullptr, p.target1, p.ids1, false,
-                                                             buckets1, childOf1, cursors1, epoch, flag, ws->hostWordDev);
+        count_keys_kernel<true><<<blocks(count, chunk1), threads, 0, stream>>>(records, count, form, p.shift, nullptr, 0u, chunk1, bins1, state, epoch);
+        plan_buckets_kernel<true><<<1, threads, 0, stream>>>(bins1, count, p.shift, lastHigh, lastLow, nullptr, p.target1, p.ids1, p.target,
+                                                             buckets1, childOf1, cursors1, windowList, 0u, state, epoch, ws->hostWordDev);
         scatter_keys_kernel<true, 8><<<blocks(count, kScatter), threads, 0, stream>>>(
-            records, count, form, p.shift, nullptr, 0u, p.target1, p.ids1, childOf1, cursors1, keysA, epoch, flag);
-        count_keys_kernel<false><<<count / chunk2 + p.ids1, threads, 0, stream>>>(keysA, count, form, 0, buckets1, p.ids1, chunk2, bins2);
-        plan_buckets_kernel<false><<<p.ids1, threads, 0, stream>>>(bins2, count, 0, 0u, 0u, buckets1, p.target, p.ids2, true,
-                                                                   buckets2, childOf2, cursors2, epoch, flag, ws->hostWordDev);
+            records, count, form, p.shift, nullptr, 0u, p.target1, p.ids1, childOf1, cursors1, keysA, epoch, state);
+        count_keys_kernel<false><<<count / chunk2 + p.ids1, threads, 0, stream>>>(keysA, count, form, 0, buckets1, p.ids1, chunk2, bins2, state, epoch);
+        plan_buckets_kernel<false><<<p.ids1, threads, 0, stream>>>(bins2, count, 0, 0u, 0u, buckets1, p.target, p.ids2, 0u,
+                                                                   buckets2, childOf2, cursors2, windowList, p.maxWindows, state, epoch,
+                                                                   ws->hostWordDev);
         scatter_keys_kernel<false, 8><<<count / kScatter + p.ids1, threads, 0, stream>>>(
-            keysA, count, form, 0, buckets1, p.ids1, p.target, p.ids2, childOf2, cursors2, keysB, epoch, flag);
-        sort_bucket_kernel<false, kBucketThreads, kBucketCap><<<p.ids2, kBucketThreads, 0, stream>>>(keysB, buckets2, none, form, records, epoch, flag);
+            keysA, count, form, 0, buckets1, p.ids1, p.target, p.ids2, childOf2, cursors2, keysB, epoch, state);
+        sort_bucket_kernel<false, kBucketThreads, kBucketCap><<<p.ids2 + kWindowWorkers, kBucketThreads, 0, stream>>>(
+            keysB, buckets2, none, form, records, windowList, epoch, state);
     }
     e = hipGetLastError();
     const hipError_t s = hipStreamSynchronize(stream);
     if (e == hipSuccess) e = s;
     if (e != hipSuccess) return e;
-    ws->tablesDirty = false;
-    ws->cleanBytes = binsEnd;
     *done = *static_cast<volatile u64*>(ws->hostWord) != epoch;
+    ws->tablesDirty = !*done;
+    ws->cleanBytes = binsEnd;
     return hipSuccess;
 }
 
@@ -860,7 +965,7 @@ size_t sort_scratch_bytes(unsigned long long count) {
     size_t needTemp = 0;
     if (radix_temp_bytes(count, &needTemp) != hipSuccess) return 0;
     SortPlan p{};
-    const size_t tables = make_plan(count, (1ull << 42) - 1, &p) ? p.bytes : 0;
+    const size_t tables = make_plan(count ? count : 1, (1ull << 42) - 1, true, &p) ? p.bytes : 0;
     return needTemp + tables + (size_t)count * sizeof(u64);
 }
 
@@ -873,18 +978,22 @@ hipError_t sort_pairs_row_major(void* pairs, unsigned long long count, hipStream
     const KeyForm form{candidateBits, (u32)firstQuery};
     if (count <= (u64)kAloneCap && lastKey >> 32 == 0) {
         const Bucket whole{0u, (u32)count, 0u, 0u, (u32)lastKey, 0u, {0u, 0u}};
-        sort_bucket_kernel<true, kSortThreads, kAloneCap><<<1, kSortThreads, 0, stream>>>(records, nullptr, whole, form, records, 0ull, nullptr);
+        sort_bucket_kernel<true, kSortThreads, kAloneCap><<<1, kSortThreads, 0, stream>>>(records, nullptr, whole, form, records, nullptr, 0ull,
+                                                                                                 nullptr);
         const hipError_t e = hipGetLastError(), s = hipStreamSynchronize(stream);
         return e == hipSuccess ? s : e;
     }
-    SortPlan p{};
     bool done = false;
-    if (make_plan(count, lastKey, &p)) {
+    for (bool twoLevels = count > kTwoLevelsFrom; !done; twoLevels = true) {
+        SortPlan p{};
+        if (!make_plan(count, lastKey, twoLevels, &p)) break;
         const hipError_t e = distribute(records, (u32)count, p, lastKey, form, stream, ws, &done);
-        if (e == hipErrorOutOfMemory)
+        if (e == hipErrorOutOfMemory) {
             (void)hipGetLastError();  // nothing was launched; the radix sort may need less
-        else if (e != hipSuccess)
-            return e;
+            break;
+        }
+        if (e != hipSuccess) return e;
+        if (twoLevels || count < kTwoLevelsAfterOneFrom) break;
     }
     return done ? hipSuccess : radix_sort(records, count, form, queryBits + candidateBits, stream, ws);
 }

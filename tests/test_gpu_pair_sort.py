@@ -47,22 +47,65 @@ CASES = {
 }
 
 
-@pytest.mark.parametrize("name", list(CASES))
-def test_sorted_pairs_are_row_major(name):
+def _check(qv, cv, calls=2):
+    """The sorted join of the coded sets against the pairs computed here; the shortest of its sorts, in milliseconds."""
     import torch
 
     import fasted_amd as fasted
     from fasted_amd.find_pairs import FASTED_SORT_PAIRS
 
-    qv, cv = (np.asarray(x).astype(np.int64) for x in CASES[name]())
+    qv, cv = np.asarray(qv).astype(np.int64), np.asarray(cv).astype(np.int64)
     (q, vq), (c, vc) = _coded(qv), _coded(cv)
     rows = max(1, (1 << 28) // len(cv))
     want = torch.cat([torch.nonzero(vq[r : r + rows, None] == vc[None, :]) + torch.tensor([r, 0], device="cuda")
                       for r in range(0, len(qv), rows)]).to(torch.int32)
     pairs = torch.zeros((len(want) + 1, 2), dtype=torch.int32, device="cuda")
-    for _ in range(2):  # the second call finds the tables as the first one left them
+    sort_ms = []
+    for _ in range(calls):  # a second call finds the tables as the first one left them
         st = fasted.join_device(q.data_ptr(), len(qv), 64, c.data_ptr(), len(cv), 64, 2, 0.5, pairs.data_ptr(), len(want) + 1,
                                 flags=FASTED_SORT_PAIRS)
         assert st.pairsFound == st.pairsStored == len(want)
         assert torch.equal(pairs[:-1], want)
         assert int(pairs[-1].abs().sum()) == 0
+        sort_ms.append(st.sortMs)
+    return min(sort_ms)
+
+
+@pytest.mark.parametrize("name", list(CASES))
+def test_sorted_pairs_are_row_major(name):
+    _check(*CASES[name]())
+
+
+def _groups(n, per):
+    """Two sets of n points in which every query has `per` candidates on average, anywhere."""
+    rng = np.random.default_rng(n)
+    small, large = int(per), int(per) + 1
+    split = int(n * (large - per))
+    v = np.concatenate([np.arange(split) // small, n + np.arange(n - split) // large])
+    return rng.permutation(v), rng.permutation(v)
+
+
+def _core():
+    """100 000 queries with two candidates each, but 2000 neighbouring ones with 200."""
+    rng = np.random.default_rng(1)
+    q = rng.permutation(np.arange(98000) // 2)
+    core = 100000 + np.arange(2000) % 10
+    return np.concatenate([q[:50000], core, q[50000:]]), rng.permutation(np.concatenate([q, core]))
+
+
+# lists on both sides of the line between one level and two, and one that crowds into a few rows
+SPARSE = {
+    "0.97 million in 130 000 rows": lambda: _groups(130000, 7.46),
+    "1.04 million in 130 000 rows": lambda: _groups(130000, 8.04),
+    "1.0 million in 200 000 rows": lambda: _groups(200000, 5.0),
+    "1.04 million in 250 000 rows": lambda: _groups(250000, 4.18),
+    "1.1 million in 250 000 rows": lambda: _groups(250000, 4.4),
+    "a crowded core": _core,
+}
+
+
+@pytest.mark.parametrize("name", list(SPARSE))
+def test_sparse_lists_are_sorted_at_the_rate_of_others(name):
+    # buckets that outgrow the LDS cost 30 to 100 times this; the lists here take 1.0 to 1.8 times as long
+    even = _check(*_groups(100000, 6.0), calls=6)
+    assert _check(*SPARSE[name](), calls=6) < 5 * even
