@@ -197,6 +197,8 @@ struct EventTimer {
     }
 };
 
+constexpr unsigned long long kMaxPairCapacity = 1ull << 45;  // 2^48 bytes of records
+
 // A NaN epsilon compares false with every distance in the reference (source/warpMma.cuh:257: no pairs at all);
 // here the accumulator start values are formed from epsilon, so it is refused before any launch.
 void validate_epsilon(double epsilon) {
@@ -1234,6 +1236,8 @@ int fasted_self_join(const uint16_t* points, long long n, int d, double epsilon,
         validate_epsilon(epsilon);
         const int dPad = round_up(d, fasted::kSlabK);
         validate_shape(n, d, dPad);
+        // (points and pairs share an allocation: its size must not wrap around to a small one)
+        if (cap > kMaxPairCapacity) throw std::invalid_argument("pair capacity exceeds what a device can address");
         // Points and pairs in one allocation.  Rows that need padding go up as they are, into the part that holds the pairs
         // later (at least 32 MB of it), and a kernel puts them in place: with rows packed on the host into new pinned
         // pages first, 30000 x 200 with 930 thousand pairs took 1.88 ms instead of 1.28 (8.2 where pinned pages were slow to touch).

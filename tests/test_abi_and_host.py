@@ -165,6 +165,16 @@ def test_raw_entry_rejects_bad_arguments_without_touching_a_gpu(lib):
     assert lib.fasted_pair_distances_device(None, 1, 64, None, 1, 64, 64, None, 0, None, None) != 0
 
 
+@pytest.mark.parametrize("cap", [2 ** 61 - 1, 2 ** 61 + 5, 2 ** 64 - 1])
+def test_pair_capacity_whose_bytes_wrap_around_is_refused_before_any_device_call(lib, cap):
+    buf = (ctypes.c_uint16 * 64)()
+    out = (ctypes.c_int32 * 2)()
+    found, stored = ctypes.c_ulonglong(), ctypes.c_ulonglong()
+    assert lib.fasted_self_join(ctypes.addressof(buf), 4, 8, 0.1, ctypes.addressof(out), cap, ctypes.byref(found),
+                                ctypes.byref(stored)) != 0
+    assert b"capacity" in lib.fasted_last_error()
+
+
 # ---------------------------------------------------------------- tile queues (host mirror)
 @pytest.mark.parametrize("n", [1, 256, 257, 4096, 5000, 100_000])
 def test_tile_queues_cover_every_tile_exactly_once(lib, n):
