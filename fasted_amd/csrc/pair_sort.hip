@@ -868,8 +868,8 @@ hipError_t distribute(u64* records, u32 count, const SortPlan& p, u64 lastKey, K
                       SortBuffers* ws, bool* done) {
     hipError_t e = grow(&ws->alt, &ws->altBytes, (size_t)count * sizeof(u32) * (p.twoLevels ? 2 : 1));
     if (e != hipSuccess) return e;
-    if (!ws->hostWord) {
-        e = hipHostMalloc(reinterpret_cast<void**>(&ws->hostWord), 64, hipHostMallocCoherent);
+    if (!ws->hostWordDev) {
+        if (!ws->hostWord) e = hipHostMalloc(reinterpret_cast<void**>(&ws->hostWord), 64, hipHostMallocCoherent);
         if (e != hipSuccess) return e;
         *ws->hostWord = 0;
         e = hipHostGetDevicePointer(reinterpret_cast<void**>(&ws->hostWordDev), ws->hostWord, 0);
