@@ -303,7 +303,7 @@ __global__ void __launch_bounds__(kSortThreads) plan_buckets_kernel(u32* __restr
 template <bool kRecords, int kPerThread>
 __global__ void __launch_bounds__(kSortThreads) scatter_keys_kernel(const void* __restrict__ in, u32 count, KeyForm form,
                                                                     int shift, const Bucket* __restrict__ parents,
-                                                                    u32 parentCount, u32 target, u32 childCount,
+                                                                    u32 parentCount, u32 target,
                                                                     const unsigned short* __restrict__ childOfBin,
                                                                     u32* __restrict__ cursors, u32* __restrict__ out, u64 epoch,
                                                                     const SortState* __restrict__ state) {
@@ -316,7 +316,7 @@ __global__ void __launch_bounds__(kSortThreads) scatter_keys_kernel(const void* 
     __shared__ u32 waveSums[kSortThreads / 64];
     __shared__ u32 which;
     if (broken_off(state, epoch)) return;
-    u32 begin = blockIdx.x * kChunk, end = min(count - begin, kChunk) + begin, lo = 0, ids = childCount;
+    u32 begin = blockIdx.x * kChunk, end = min(count - begin, kChunk) + begin, lo = 0;
     if (!kRecords) {
         const u32 b = find_bucket(parents, parentCount, blockIdx.x, kChunk, &which);
         if (b == ~0u) return;
@@ -326,7 +326,6 @@ __global__ void __launch_bounds__(kSortThreads) scatter_keys_kernel(const void* 
         lo = p.lo;
         shift = (int)p.shift;
         const u32 firstChild = p.start / target + b;
-        ids = (b + 1 < parentCount ? parents[b + 1].start / target + b + 1 : childCount) - firstChild;
         cursors += firstChild;
         childOfBin += (size_t)b * kBins2;
     }
@@ -907,7 +906,7 @@ hipError_t distribute(u64* records, u32 count, const SortPlan& p, u64 lastKey, K
                                                              buckets1, childOf1, cursors1, windowList, p.maxWindows, state, epoch,
                                                              ws->hostWordDev);
         scatter_keys_kernel<true, 4><<<blocks(count, 4096), threads, 0, stream>>>(records, count, form, p.shift, nullptr, 0u, p.target,
-                                                                                  p.ids1, childOf1, cursors1, keysA, epoch, state);
+                                                                                  childOf1, cursors1, keysA, epoch, state);
         sort_bucket_kernel<false, kBucketThreads, kBucketCap><<<p.ids1 + kWindowWorkers, kBucketThreads, 0, stream>>>(
             keysA, buckets1, none, form, records, windowList, epoch, state);
     } else {
@@ -917,13 +916,13 @@ hipError_t distribute(u64* records, u32 count, const SortPlan& p, u64 lastKey, K
         plan_buckets_kernel<true><<<1, threads, 0, stream>>>(bins1, count, p.shift, lastHigh, lastLow, nullptr, p.target1, p.ids1, p.target,
                                                              buckets1, childOf1, cursors1, windowList, 0u, state, epoch, ws->hostWordDev);
         scatter_keys_kernel<true, 8><<<blocks(count, kScatter), threads, 0, stream>>>(
-            records, count, form, p.shift, nullptr, 0u, p.target1, p.ids1, childOf1, cursors1, keysA, epoch, state);
+            records, count, form, p.shift, nullptr, 0u, p.target1, childOf1, cursors1, keysA, epoch, state);
         count_keys_kernel<false><<<count / chunk2 + p.ids1, threads, 0, stream>>>(keysA, count, form, 0, buckets1, p.ids1, chunk2, bins2, state, epoch);
         plan_buckets_kernel<false><<<p.ids1, threads, 0, stream>>>(bins2, count, 0, 0u, 0u, buckets1, p.target, p.ids2, 0u,
                                                                    buckets2, childOf2, cursors2, windowList, p.maxWindows, state, epoch,
                                                                    ws->hostWordDev);
         scatter_keys_kernel<false, 8><<<count / kScatter + p.ids1, threads, 0, stream>>>(
-            keysA, count, form, 0, buckets1, p.ids1, p.target, p.ids2, childOf2, cursors2, keysB, epoch, state);
+            keysA, count, form, 0, buckets1, p.ids1, p.target, childOf2, cursors2, keysB, epoch, state);
         sort_bucket_kernel<false, kBucketThreads, kBucketCap><<<p.ids2 + kWindowWorkers, kBucketThreads, 0, stream>>>(
             keysB, buckets2, none, form, records, windowList, epoch, state);
     }
