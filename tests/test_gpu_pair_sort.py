@@ -1,7 +1,12 @@
 """GPU parity of the row-major order of the stored pairs, at the counts and distributions where the sort takes another path:
-one workgroup, one and two levels of buckets, buckets too full for the LDS, keys of more than 32 bits, the radix sort."""
+one workgroup, one and two levels of buckets, buckets too full for the LDS, crowded cells, keys of more than 32 bits, lists
+that a level breaks off, the radix sort behind them.  tests/test_sort_routes.py holds the lists to these paths."""
+import ctypes
+
 import numpy as np
 import pytest
+
+from tests import sort_routes
 
 pytestmark = pytest.mark.gpu
 
@@ -109,3 +114,45 @@ def test_sparse_lists_are_sorted_at_the_rate_of_others(name):
     # buckets that outgrow the LDS cost 30 to 100 times this; the lists here take 1.0 to 1.8 times as long
     even = _check(*_groups(100000, 6.0), calls=6)
     assert _check(*SPARSE[name](), calls=6) < 5 * even
+
+
+@pytest.mark.parametrize("name", list(sort_routes.CASES))
+def test_crowded_lists_are_row_major_and_leave_the_sort_as_it_was(name):
+    import torch
+
+    import fasted_amd as fasted
+    from fasted_amd.find_pairs import FASTED_SORT_PAIRS
+
+    ordinary = _groups(20000, 10.0)
+    for qv, cv in (sort_routes.CASES[name][0](), ordinary, sort_routes.CASES[name][0]()):
+        want = torch.from_numpy(sort_routes.pairs_of(qv, cv)).cuda()
+        (q, _), (c, _) = _coded(qv), _coded(cv)
+        pairs = torch.zeros((len(want) + 1, 2), dtype=torch.int32, device="cuda")
+        st = fasted.join_device(q.data_ptr(), len(qv), 64, c.data_ptr(), len(cv), 64, 2, 0.5, pairs.data_ptr(), len(want) + 1,
+                                flags=FASTED_SORT_PAIRS)
+        assert st.pairsFound == st.pairsStored == len(want)
+        assert torch.equal(pairs[:-1], want)
+        assert int(pairs[-1].abs().sum()) == 0
+
+
+def test_crowded_rows_of_a_later_query_block_are_row_major():
+    # 24 blocks of query points; 4500 equal points, some in every block, whose rows are too full for the LDS
+    import fasted_amd as fasted
+
+    n, block = 24 * 4096, 4096
+    v = np.arange(n) + 1
+    v[np.random.default_rng(3).permutation(n)[:4500]] = 0
+    want = sort_routes.pairs_of(v, v)
+    bits = np.zeros((n, 64), dtype=np.float16)
+    bits[:, 0], bits[:, 1] = v // 2000, v % 2000
+    for r in range(0, n, block):
+        mine = want[(want[:, 0] >= r) & (want[:, 0] < r + block)] - np.array([r, 0])
+        assert {"one level", "windows"} <= sort_routes.route(mine, block, n)
+    lib = fasted.load_findpairs()
+    found, stored = ctypes.c_ulonglong(), ctypes.c_ulonglong()
+    out = np.full((len(want) + 1, 2), -1, dtype=np.int32)
+    rc = lib.fasted_self_join_blocked(bits.ctypes.data, n, 64, 0.5, block, out.ctypes.data, len(out), ctypes.byref(found),
+                                      ctypes.byref(stored))
+    assert rc == 0, lib.fasted_last_error()
+    assert found.value == stored.value == len(want)
+    assert np.array_equal(out[:-1], want) and (out[-1] == -1).all()
