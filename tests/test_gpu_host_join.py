@@ -1,10 +1,11 @@
 """GPU parity of the host-to-host join's way up: rows that need padding or none, odd dimensionalities, rows that go up in
-several pieces, the buffer kept from call to call, and a call that fails in between."""
+several pieces, and the buffer kept from call to call, for larger and smaller joins than the one that left it."""
 import ctypes
 
 import numpy as np
 import pytest
 
+import oracle
 from tests import datasets
 
 pytestmark = pytest.mark.gpu
@@ -21,29 +22,52 @@ def _self_join(bits, eps, cap):
     return rc, out[: stored.value], found.value
 
 
-# one row; odd, even and multiple-of-8 padding; no padding; more than 32 MB of packed rows (two pieces, as no pair list is longer)
+def _case(n, d):
+    """Integer coordinates and an epsilon with about eight neighbours a point whose square lies half-way between two integers."""
+    bits = datasets.small_integers(n, d, high=3, seed=n + d)
+    eps = datasets.epsilon_for_neighbours(bits, min(8, n - 1) or 1, sample=128) if n > 1 else 1.0
+    return bits, float(np.sqrt(np.floor(eps * eps) + 0.5))
+
+
+# one row; odd, even and multiple-of-8 padding; no padding; more than 32 MB of packed rows and fewer of pairs (two pieces)
 @pytest.mark.parametrize("n,d", [(1, 1), (300, 3), (2000, 63), (2000, 64), (2001, 66), (1500, 72), (1000, 129), (70001, 250)])
 def test_host_join_equals_device_join(n, d):
     import torch
 
     import fasted_amd as fasted
-    from fasted_amd.find_pairs import FASTED_SORT_PAIRS
+    from fasted_amd.find_pairs import FASTED_FULL_MATRIX, FASTED_SORT_PAIRS
 
-    bits = datasets.small_integers(n, d, high=3, seed=n + d)
+    bits, eps = _case(n, d)
     ld = (d + 63) // 64 * 64
     pts = torch.zeros((n, ld), dtype=torch.int16, device="cuda")
     pts[:, :d] = torch.from_numpy(bits.view(np.int16)).cuda()
-    eps = float(np.sqrt(max(1.0, d * 0.6) + 0.5))  # below the typical squared distance, half-way between two integers
-    cap = 2 * n + 1000
-    pairs = torch.zeros((cap, 2), dtype=torch.int32, device="cuda")
-    st = fasted.self_join_device(pts.data_ptr(), n, d, ld, eps, pairs.data_ptr(), cap, flags=FASTED_SORT_PAIRS)
+    count = int(fasted.self_join_device(pts.data_ptr(), n, d, ld, eps, None, 0, flags=0).pairsFound)
+    assert n == 1 or count > 2 * n  # what is checked is not the diagonal alone
+    pairs = torch.zeros((count + 1, 2), dtype=torch.int32, device="cuda")
+    st = fasted.self_join_device(pts.data_ptr(), n, d, ld, eps, pairs.data_ptr(), count + 1,
+                                 flags=FASTED_SORT_PAIRS | FASTED_FULL_MATRIX)
+    assert st.pairsFound == st.pairsStored == count
+    want = pairs[:-1].cpu().numpy()
+    if n <= 2001:
+        assert np.array_equal(want, oracle.self_join_f64(bits, eps))
+    small, small_eps = _case(200, 65)
+    small_want = oracle.self_join_f64(small, small_eps)
+    for release in (False, False, True):
+        if release:
+            fasted.load_findpairs().releaseResources()
+        rc, got, found = _self_join(bits, eps, count + 1)
+        assert rc == 0 and found == count and np.array_equal(got, want)
+        rc, got, found = _self_join(bits, eps, count // 2 or 1)  # room for some of them only
+        assert rc == 0 and found == count and len(got) == (count // 2 or 1)
+        rc, got, _ = _self_join(small, small_eps, len(small_want))
+        assert rc == 0 and np.array_equal(got, small_want)
+
+
+def test_host_join_after_one_that_was_refused():
+    bits, eps = _case(500, 70)
+    want = oracle.self_join_f64(bits, eps)
     for _ in range(2):
-        rc, got, found = _self_join(bits, eps, cap)
-        assert rc == 0 and found == st.pairsFound and len(got) == st.pairsStored
-        if st.pairsFound <= cap:
-            assert np.array_equal(got, pairs[: st.pairsStored].cpu().numpy())
-        rc, _, _ = _self_join(bits, float("nan"), cap)
+        rc, _, _ = _self_join(bits, float("nan"), len(want))
         assert rc != 0
-    fasted.load_findpairs().releaseResources()
-    rc, got, found = _self_join(bits, eps, cap)
-    assert rc == 0 and found == st.pairsFound
+        rc, got, found = _self_join(bits, eps, len(want))
+        assert rc == 0 and found == len(want) and np.array_equal(got, want)
