@@ -40,3 +40,37 @@ def test_sliced_distances_match_fp64(n, d):
         # each of d products and additions rounds to half a unit of 2^-24 at most; the square root halves it
         bound = 1e-7 + 0.5 * (ld / 16 + 20) * 2.0**-24
         assert bool(((got[r : r + step][: len(ok)][ok].double() - want).abs() <= bound * want).all())
+
+
+def test_sliced_distances_of_subnormal_large_and_infinite_coordinates():
+    # every difference of two halves is exact in FP32 but for the last bit; what no FP32 holds is what FP32 makes of it
+    import torch
+
+    import fasted_amd as fasted
+
+    n, d = 5003, 512
+    gen = torch.Generator(device="cuda").manual_seed(9)
+    count = max(8 * n + 7, (3 << 29) // (2 * d) + 5)
+    kind = torch.randint(0, 3, (n, 1), generator=gen, device="cuda")
+    tiny = torch.randint(-1023, 1024, (n, d), generator=gen, device="cuda").float() * 2.0**-24  # subnormal halves
+    large = torch.randint(-2047, 2048, (n, d), generator=gen, device="cuda").float() * 2.0**5   # up to 65504
+    mixed = torch.where(torch.rand((n, d), generator=gen, device="cuda") < 0.5, tiny, large)
+    pts = torch.where(kind == 0, tiny, torch.where(kind == 1, large, mixed)).to(torch.float16)
+    assert bool((pts.float() == torch.where(kind == 0, tiny, torch.where(kind == 1, large, mixed))).all())
+    pts[7, 3], pts[8, 500], pts[9, 511], pts[10, 0] = float("inf"), float("-inf"), float("inf"), float("nan")
+    pts[9, 3] = float("inf")
+    pairs = torch.randint(0, n, (count, 2), generator=gen, device="cuda", dtype=torch.int32)
+    some = torch.arange(0, 16, device="cuda", dtype=torch.int32)
+    pairs[:256] = torch.cartesian_prod(some, some)
+    got = torch.full((count,), -2.0, dtype=torch.float32, device="cuda")
+    fasted.pair_distances_device(pts.data_ptr(), n, d, pts.data_ptr(), n, d, d, pairs.data_ptr(), count, got.data_ptr())
+    for r in range(0, count, 1 << 17):
+        i = pairs[r : r + (1 << 17)].long()
+        want = (pts[i[:, 0]].double() - pts[i[:, 1]].double()).square().sum(1).sqrt()
+        mine = got[r : r + (1 << 17)].double()
+        assert torch.equal(torch.isnan(mine), torch.isnan(want)) and torch.equal(torch.isinf(mine), torch.isinf(want))
+        fine = torch.isfinite(want)
+        # as above; the square of the smallest difference, 2^-48, is far from the FP32 subnormals
+        bound = 1e-7 + 0.5 * (d / 16 + 20) * 2.0**-24
+        assert bool(((mine[fine] - want[fine]).abs() <= bound * want[fine]).all())
+    assert bool(torch.isinf(got[7 * 16 + 8])) and bool(torch.isnan(got[7 * 16 + 9])) and bool(torch.isnan(got[10 * 16 + 10]))
