@@ -228,12 +228,12 @@ def test_two_set_join_matches_the_checker(fasted, nq, nc, d):
 @pytest.mark.parametrize("n,d", [(700, 64), (2048, 128), (5000, 192)])
 def test_symmetric_option_gives_the_same_pair_set(fasted, n, d):
     """FASTED_SYMMETRIC computes only the tiles on and above the diagonal and mirrors the pairs: the
-    sorted pair list must be identical to the default full computation."""
+    sorted pair list must be identical to that of the full matrix."""
     from fasted_amd import find_pairs as fp
 
     bits = datasets.uniform_bytes(n, d, seed=3 * n + d)
     eps = datasets.epsilon_for_neighbours(bits, 12)
-    full, st_full, _ = device_join(fasted, bits, eps)
+    full, st_full, _ = device_join(fasted, bits, eps, flags=fp.FASTED_SORT_PAIRS | fp.FASTED_FULL_MATRIX)
     half, st_half, _ = device_join(fasted, bits, eps, flags=fp.FASTED_SORT_PAIRS | fp.FASTED_SYMMETRIC)
     assert st_half.pairsFound == st_full.pairsFound
     assert np.array_equal(half, full)
@@ -331,6 +331,8 @@ def test_points_with_infinite_coordinates_pair_with_nothing_but_themselves(faste
     """Values beyond the FP16 range quantise to infinity (source/DataLoader/PointListBuilder.hpp:57-73); the
     distances of such a point are NaN or infinite, every comparison with them is false
     (source/warpMma.cuh:257), so it has no neighbours; only its self pair is reported (forced here)."""
+    from fasted_amd import find_pairs as fp
+
     n, d = 1200, 64
     bits = datasets.uniform_bytes(n, d, seed=123)
     eps = datasets.epsilon_for_neighbours(bits, 25)
@@ -343,6 +345,8 @@ def test_points_with_infinite_coordinates_pair_with_nothing_but_themselves(faste
     keep = ~(np.isin(clean[:, 0], odd) | np.isin(clean[:, 1], odd))
     want = oracle.sort_pairs(np.vstack([clean[keep], [[i, i] for i in odd]]).astype(np.int32))
     assert np.array_equal(got, want)
+    triangle, _, _ = device_join(fasted, spoiled, eps, flags=fp.FASTED_SORT_PAIRS | fp.FASTED_SYMMETRIC)
+    assert np.array_equal(triangle, want)
 
 
 def test_padding_columns_are_checked(fasted):
@@ -365,9 +369,10 @@ def test_padding_columns_are_checked(fasted):
 
 def test_join_is_deterministic_over_many_tiles_per_workgroup(fasted):
     """Every workgroup walks hundreds of tiles here, with the next tile's operands in flight during each
-    epilogue: two runs must give the same pair set (a transfer that a barrier did not wait for shows up as a
-    few pairs that differ from run to run), and sampled rows must agree with FP64."""
+    epilogue: two runs of the full matrix and one of its triangle must give the same pair set (a transfer that a
+    barrier did not wait for shows up as a few pairs that differ from run to run), and sampled rows must agree with FP64."""
     import torch
+    from fasted_amd import find_pairs as fp
 
     n, d = 90000, 192
     g = torch.Generator(device="cuda")
@@ -380,14 +385,14 @@ def test_join_is_deterministic_over_many_tiles_per_workgroup(fasted):
     eps = float(torch.quantile(d2[d2 > 1e-6].flatten()[:1 << 20], 0.004).sqrt())
     cap = 400 * n
     keys = []
-    for _ in range(2):
+    for flags in (fp.FASTED_FULL_MATRIX, fp.FASTED_FULL_MATRIX, 0):
         pairs = torch.empty((cap, 2), dtype=torch.int32, device="cuda")
-        st = fasted.self_join_device(pts.view(torch.int16).data_ptr(), n, d, d, eps, pairs.data_ptr(), cap, flags=0)
+        st = fasted.self_join_device(pts.view(torch.int16).data_ptr(), n, d, d, eps, pairs.data_ptr(), cap, flags=flags)
         assert st.pairsFound == st.pairsStored > 10 * n
         got = pairs[: st.pairsStored]
         keys.append(torch.sort(got[:, 0].to(torch.int64) * n + got[:, 1].to(torch.int64)).values)
         del pairs
-    assert keys[0].shape == keys[1].shape and bool((keys[0] == keys[1]).all())
+    assert torch.equal(keys[0], keys[1]) and torch.equal(keys[0], keys[2])
     rows = torch.arange(0, n, n // 256, device="cuda")[:256]
     xs = pts[rows].double()
     d2 = ((xs * xs).sum(1)[:, None] + (pts.double() ** 2).sum(1)[None, :] - 2.0 * xs @ pts.double().T).clamp_min(0)
@@ -403,7 +408,7 @@ def test_join_is_deterministic_over_many_tiles_per_workgroup(fasted):
 
 def test_tall_tile_order_exact_pair_sets(fasted):
     """From 64 x 64 tiles on, the work queues walk super-squares of 32 x 8 tiles.  Integer coordinates make the
-    join exact, so on a ragged matrix of 65 x 65 tiles the default order, the symmetric option (upper part of
+    join exact, so on a ragged matrix of 65 x 65 tiles the full matrix, its upper triangle (upper part of
     the tall super-squares, mirrored) and a rectangular two-set join (65 x 3 tiles: most super-square positions
     are padding) must each give exactly the pair list of a blockwise FP64 computation."""
     import torch
@@ -428,7 +433,7 @@ def test_tall_tile_order_exact_pair_sets(fasted):
 
     want = truth(n)
     cap = int(want.shape[0]) + 1024
-    for flags in (fp.FASTED_SORT_PAIRS, fp.FASTED_SORT_PAIRS | fp.FASTED_SYMMETRIC):
+    for flags in (fp.FASTED_SORT_PAIRS | fp.FASTED_FULL_MATRIX, fp.FASTED_SORT_PAIRS | fp.FASTED_SYMMETRIC):
         pairs = torch.empty((cap, 2), dtype=torch.int32, device="cuda")
         st = fasted.self_join_device(pts.data_ptr(), n, d, d, eps, pairs.data_ptr(), cap, flags=flags)
         assert st.pairsFound == st.pairsStored == want.shape[0]
@@ -445,8 +450,10 @@ def test_both_tile_heights_give_the_exact_pair_set(fasted, n, d, monkeypatch):
     """Matrices of few tiles are cut into tiles of 128 query rows instead of 256 (FASTED_TILE_ROWS forces either).
     Integer coordinates make the join exact: both heights, on a self-join, on a two-set join with a ragged
     query count and with non-finite points present, must give exactly the FP64 pair list.  The last shape has
-    65 tile rows of 128: the tall tile order with that height."""
+    65 tile rows of 128: the tall tile order with that height.  Self-joins with the library's choice and of the
+    full matrix."""
     import torch
+    from fasted_amd import find_pairs as fp
 
     bits = datasets.small_integers(n, d, high=3, seed=3 * n + d)
     x = bits.view(np.float16).astype(np.float64)
@@ -459,8 +466,9 @@ def test_both_tile_heights_give_the_exact_pair_set(fasted, n, d, monkeypatch):
     pts = torch.from_numpy(bits.view(np.int16).copy()).cuda()
     for rows in ("256", "128"):
         monkeypatch.setenv("FASTED_TILE_ROWS", rows)
-        got, st, _ = device_join(fasted, bits, eps)
-        assert st.pairsFound == len(truth) and np.array_equal(got, truth), rows
+        for flags in (fp.FASTED_SORT_PAIRS, fp.FASTED_SORT_PAIRS | fp.FASTED_FULL_MATRIX):
+            got, st, _ = device_join(fasted, bits, eps, flags=flags)
+            assert st.pairsFound == len(truth) and np.array_equal(got, truth), (rows, flags)
         buf = torch.empty((len(truth2) + 64, 2), dtype=torch.int32, device="cuda")
         st2 = fasted.join_device(pts.data_ptr(), nq, d, pts.data_ptr(), nc, d, d, eps, buf.data_ptr(), buf.shape[0])
         assert st2.pairsFound == len(truth2) and np.array_equal(buf[: st2.pairsStored].cpu().numpy(), truth2), rows
@@ -472,8 +480,9 @@ def test_both_tile_heights_give_the_exact_pair_set(fasted, n, d, monkeypatch):
     want = want[np.lexsort((want[:, 1], want[:, 0]))]
     for rows in ("256", "128"):
         monkeypatch.setenv("FASTED_TILE_ROWS", rows)
-        got, st, _ = device_join(fasted, bad, eps)
-        assert np.array_equal(got, want), rows
+        for flags in (fp.FASTED_SORT_PAIRS, fp.FASTED_SORT_PAIRS | fp.FASTED_FULL_MATRIX):
+            got, st, _ = device_join(fasted, bad, eps, flags=flags)
+            assert np.array_equal(got, want), (rows, flags)
 
 
 def test_small_joins_time_themselves_with_the_device_clock(fasted):

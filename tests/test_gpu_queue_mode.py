@@ -30,10 +30,11 @@ def integer_case(n, d, seed, rank=10):
     return bits, eps
 
 
-@pytest.mark.parametrize("n,d", [(7000, 128), (7000, 320), (12000, 128), (12000, 320)])
+@pytest.mark.parametrize("n,d", [(7000, 128), (7000, 320), (12000, 128), (12000, 320), (6000, 1088)])
 def test_queue_mode_exact_pair_lists(fasted, n, d, monkeypatch):
-    """784 and 2209 tiles of 256 rows (1540 and 4418 of 128 rows, the latter in the tall order): default and
-    symmetric, both tile heights, with and without squared norms brought by the caller."""
+    """784 and 2209 tiles of 256 rows (1540 and 4418 of 128 rows, the latter in the tall order), and 17 slabs (hit bits
+    behind the k-loop): the library's choice, the full matrix and the triangle, both tile heights, with and without
+    squared norms brought by the caller."""
     import torch
     from fasted_amd import find_pairs as fp
 
@@ -47,8 +48,9 @@ def test_queue_mode_exact_pair_lists(fasted, n, d, monkeypatch):
     fasted.sum_squared_device(pts.data_ptr(), n, d, d, sums.data_ptr())
     for rows in ("256", "128"):
         monkeypatch.setenv("FASTED_TILE_ROWS", rows)
-        for flags in (fp.FASTED_SORT_PAIRS, fp.FASTED_SORT_PAIRS | fp.FASTED_SYMMETRIC,
-                      fp.FASTED_SORT_PAIRS | fp.FASTED_SKIP_SUMS):
+        for flags in (fp.FASTED_SORT_PAIRS, fp.FASTED_SORT_PAIRS | fp.FASTED_FULL_MATRIX,
+                      fp.FASTED_SORT_PAIRS | fp.FASTED_SYMMETRIC, fp.FASTED_SORT_PAIRS | fp.FASTED_SKIP_SUMS,
+                      fp.FASTED_SORT_PAIRS | fp.FASTED_FULL_MATRIX | fp.FASTED_SKIP_SUMS):
             pairs.fill_(-1)
             st = fasted.self_join_device(pts.data_ptr(), n, d, d, eps, pairs.data_ptr(), cap, sums_ptr=sums.data_ptr(),
                                          flags=flags)
@@ -87,7 +89,7 @@ def test_queue_mode_two_set_exact_pair_list(fasted, monkeypatch):
 
 def test_queue_mode_band_check_exponential_10000x1024(fasted):
     """Exp(40) data of the headline kind at 10 000 x 1024 (1600 tiles, 16 slabs): the whole pair set against the
-    FP64 checker under the relative 1e-3 band rule, default and symmetric."""
+    FP64 checker under the relative 1e-3 band rule, the full matrix and its triangle."""
     import torch
     from fasted_amd import find_pairs as fp
 
@@ -99,7 +101,7 @@ def test_queue_mode_band_check_exponential_10000x1024(fasted):
     cap = 4 * len(truth)
     pairs = torch.empty((cap, 2), dtype=torch.int32, device="cuda")
     lists = []
-    for flags in (fp.FASTED_SORT_PAIRS, fp.FASTED_SORT_PAIRS | fp.FASTED_SYMMETRIC):
+    for flags in (fp.FASTED_SORT_PAIRS | fp.FASTED_FULL_MATRIX, fp.FASTED_SORT_PAIRS | fp.FASTED_SYMMETRIC):
         st = fasted.self_join_device(pts.data_ptr(), n, d, d, eps, pairs.data_ptr(), cap, flags=flags)
         got = pairs[: st.pairsStored].cpu().numpy()
         rep = oracle.epsilon_band_report(bits, got, eps, truth_pairs=truth)

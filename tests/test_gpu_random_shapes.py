@@ -43,9 +43,9 @@ def test_random_shape(n, d, neighbours, seed, tile_rows, monkeypatch):
         pts = torch.from_numpy(bits.view(np.int16).copy()).cuda()
         cap = len(got) + 16
         buf = torch.empty((cap, 2), dtype=torch.int32, device="cuda")
-        st = fasted_amd.self_join_device(pts.data_ptr(), n, d, d, eps, buf.data_ptr(), cap,
-                                         flags=fp.FASTED_SORT_PAIRS | fp.FASTED_SYMMETRIC)
-        assert st.pairsFound == found and np.array_equal(buf[: st.pairsStored].cpu().numpy(), got)
+        for part in (fp.FASTED_SYMMETRIC, fp.FASTED_FULL_MATRIX):
+            st = fasted_amd.self_join_device(pts.data_ptr(), n, d, d, eps, buf.data_ptr(), cap, flags=fp.FASTED_SORT_PAIRS | part)
+            assert st.pairsFound == found and np.array_equal(buf[: st.pairsStored].cpu().numpy(), got)
         nq = max(1, n // 3)  # first third against the rest, as two sets
         st2 = fasted_amd.join_device(pts.data_ptr(), nq, d, pts[nq:].data_ptr(), n - nq, d, d, eps, buf.data_ptr(), cap)
         want = got[(got[:, 0] < nq) & (got[:, 1] >= nq)] - np.array([0, nq], dtype=np.int32)
