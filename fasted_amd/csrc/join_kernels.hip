@@ -306,8 +306,15 @@ __device__ __forceinline__ void static_for(F&& f) {
 // the mailbox that carries them runs one tile further ahead there (two slots).
 // kBitsInLastSlab: the hit bits of a tile are gathered between the MFMAs of its last slab instead of behind the
 // k-loop (tiles of up to 16 slabs; see slab_step).
-template <bool kEpilogue, bool kTall, int kTileRows, bool kOneSlab, bool kBitsInLastSlab = false>
+// kMirror: only tiles on and above the diagonal are computed, and pairs above it are written in both orientations.  Such
+// a pair is staged once and written twice when its region leaves: staged twice, the mirrored tile of a workgroup overflowed
+// its regions where the two tiles of the full matrix did not, and at 4096 x 64 with 128 neighbours the triangle took
+// 32.7 us, 27.9 the full matrix (now 28.3; 512 neighbours 90 -> 56, 100000 x 384 with 1000 3.67 -> 3.19 ms).  A variant of
+// its own because the full matrix became 1 - 2 % slower when the choice was made at run time (100000 x 128 2.18 -> 2.21 ms).
+template <bool kEpilogue, bool kTall, int kTileRows, bool kOneSlab, bool kBitsInLastSlab = false, bool kMirror = false>
 __global__ void __launch_bounds__(kThreads, 1) join_kernel(JoinParams p) {
+    static_assert(!kMirror || (kEpilogue && kTileRows == 256), "pairs are mirrored across the diagonal of square tiles");
+    const bool upperOnly = kEpilogue ? kMirror : p.symmetric != 0;
     static_assert(!kBitsInLastSlab || kEpilogue, "hit bits are gathered only when there is an epilogue");
     static_assert(kTileRows == 256 || kTileRows == 128, "tile rows");
     constexpr int kWaveRows = kTileRows / 2;    // rows of a wave's output sub-tile (2 x 4 waves)
@@ -400,7 +407,7 @@ __global__ void __launch_bounds__(kThreads, 1) join_kernel(JoinParams p) {
             if (pos < ras.perQueue) {
                 unsigned tr, tc;
                 tile_order_decode(ras, SubShape<kTall>::rows, SubShape<kTall>::cols, q, pos, &tr, &tc);
-                if (tr < ras.tileRows && tc < ras.tileCols && !(p.symmetric && tc < tr)) {
+                if (tr < ras.tileRows && tc < ras.tileCols && !(upperOnly && tc < tr)) {
                     *row = tr;
                     *col = tc;
                     home = q;  // the next reservation goes where this tile came from
@@ -419,6 +426,7 @@ __global__ void __launch_bounds__(kThreads, 1) join_kernel(JoinParams p) {
     // reservation on the global counter (same-address atomics serialise at about 12 ns each: one per pair,
     // or per wave and tile, is what would bound output-heavy joins) and coalesced 8-byte stores.
     int staged = 0;
+    bool doubled = false;  // a staged record stands for the pair and its mirror image
     // Pair records are written through to memory (a store at system scope) instead of staying dirty in the L2 of
     // the XCD until the kernel ends: the host may take a small join for finished as soon as the last workgroup
     // has reported, and a record is written once and not read again by this kernel.
@@ -427,15 +435,21 @@ __global__ void __launch_bounds__(kThreads, 1) join_kernel(JoinParams p) {
                            (unsigned long long)(unsigned)rec.x | ((unsigned long long)(unsigned)rec.y << 32),
                            __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     };
+    auto write_staged = [&](unsigned long long base, int ln) {
+        for (int i = ln; i < staged; i += 64) {
+            const int2 rec = sStage[i];
+            if (base + i < p.cap) store_pair(base + i, rec);  // past the capacity: counted, not stored
+            if (doubled && base + staged + i < p.cap) store_pair(base + staged + i, int2{rec.y, rec.x});
+        }
+    };
     auto flush_wave = [&]() {
         const int ln = lane_now();
         unsigned long long base = 0;
-        if (ln == 0) base = atomicAdd(&p.counters[kCounterFound], (unsigned long long)staged);
+        if (ln == 0) base = atomicAdd(&p.counters[kCounterFound], (unsigned long long)(staged << (doubled ? 1 : 0)));
         base = ((unsigned long long)__builtin_amdgcn_readfirstlane((unsigned)(base >> 32)) << 32) |
                __builtin_amdgcn_readfirstlane((unsigned)base);
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the staged records are in LDS
-        for (int i = ln; i < staged; i += 64)
-            if (base + i < p.cap) store_pair(base + i, sStage[i]);  // past the capacity: counted, not stored
+        write_staged(base, ln);
         staged = 0;
     };
 
@@ -512,7 +526,7 @@ __global__ void __launch_bounds__(kThreads, 1) join_kernel(JoinParams p) {
             // A matrix of no more tiles than workgroups: one tile each, by workgroup number.  Through the queues,
             // every workgroup would reserve a second tile while it starts its first (the reservation runs one
             // tile ahead), and the workgroups of XCDs with short queues would find the work already taken.
-            if (p.symmetric) {
+            if (upperOnly) {
                 tile_order_upper_decode(blockIdx.x, &r, &c);
             } else {
                 r = blockIdx.x / p.raster.tileCols;
@@ -844,7 +858,7 @@ __global__ void __launch_bounds__(kThreads, 1) join_kernel(JoinParams p) {
             const bool diagonal = p.selfStride != 0 && colBase <= (rowBase + kTileRows - 1) * p.selfStride &&
                                   rowBase * p.selfStride <= colBase + kTile - 1;
             const bool edge = nonFinite || diagonal || rowBase + kTileRows > p.nQ || colBase + kTile > p.nC;
-            const bool mirror = p.symmetric && tr != tc;  // a tile above the diagonal also stands for its mirror image
+            const bool mirror = kMirror && tr != tc;  // a tile above the diagonal also stands for its mirror image
 
             bool any;
             if (kFusedBits && !edge) {
@@ -939,6 +953,10 @@ __global__ void __launch_bounds__(kThreads, 1) join_kernel(JoinParams p) {
                 // lanes with a hit, lanes with more than one -- are formed together: a branch waits for the
                 // compare that forms its mask, and one wait serves both.
                 constexpr int kWords = kFragRows / 2;
+                if (kMirror && doubled != mirror) {
+                    if (staged != 0) flush_wave();
+                    doubled = mirror;
+                }
                 for (;;) {
                     unsigned first = ~0u, total = 0u;
 #pragma unroll
@@ -952,27 +970,21 @@ __global__ void __launch_bounds__(kThreads, 1) join_kernel(JoinParams p) {
                     unsigned long long again = __builtin_amdgcn_ballot_w64(total > 1u);
                     asm volatile("" : "+s"(lanes), "+s"(again));
                     if (lanes == 0ull) break;
-                    const int count = __builtin_popcountll(lanes) << (mirror ? 1 : 0);
+                    const int count = __builtin_popcountll(lanes);
                     if (staged + count > kWaveStagePairs) flush_wave();
                     if ((int)first >= 0) {
                         // element `first` of the lane: block row first / 16, block column (first / 4) % 4, row first % 4
                         const int q = qLane + (int)((first & ~15u) + (first & 3u));
                         const int c = cLane + (int)((first & 12u) << 2);
-                        const unsigned before = __builtin_amdgcn_mbcnt_hi(
-                            (unsigned)(lanes >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)lanes, 0u));
-                        const unsigned at = (unsigned)staged + (mirror ? 2u * before : before);
+                        const unsigned at = (unsigned)staged + __builtin_amdgcn_mbcnt_hi((unsigned)(lanes >> 32),
+                                                                                         __builtin_amdgcn_mbcnt_lo((unsigned)lanes, 0u));
+                        const unsigned long long rec = (unsigned long long)(unsigned)q | ((unsigned long long)(unsigned)c << 32);
                         // written as an instruction: for an ordinary LDS store the compiler first waits until
                         // this wave's global->LDS transfers of the next tile have landed
-                        auto put = [&](unsigned idx, int a0, int a1) {
-                            const unsigned long long rec =
-                                (unsigned long long)(unsigned)a0 | ((unsigned long long)(unsigned)a1 << 32);
-                            asm volatile("ds_write_b64 %0, %1" ::"v"(ldsBase + (unsigned)kLdsStage +
-                                                                     ((unsigned)wave * kWaveStagePairs + idx) * 8u),
-                                         "v"(rec)
-                                         : "memory");
-                        };
-                        put(at, q, c);
-                        if (mirror) put(at + 1, c, q);
+                        asm volatile("ds_write_b64 %0, %1" ::"v"(ldsBase + (unsigned)kLdsStage +
+                                                                 ((unsigned)wave * kWaveStagePairs + at) * 8u),
+                                     "v"(rec)
+                                     : "memory");
                     }
                     staged += count;
                     if (again == 0ull) break;
@@ -1003,7 +1015,7 @@ __global__ void __launch_bounds__(kThreads, 1) join_kernel(JoinParams p) {
         unsigned long long* const sBase = reinterpret_cast<unsigned long long*>(lds + 64);
         const int ln = lane_now();
         __syncthreads();  // every wave is past its last fragment read
-        if (ln == 0) sLeft[wave] = (unsigned)staged;
+        if (ln == 0) sLeft[wave] = (unsigned)(staged << (doubled ? 1 : 0));
         __syncthreads();
         unsigned before = 0, total = 0;
 #pragma unroll
@@ -1015,9 +1027,7 @@ __global__ void __launch_bounds__(kThreads, 1) join_kernel(JoinParams p) {
         if (total != 0) {
             if (wave == 0 && ln == 0) *sBase = atomicAdd(&p.counters[kCounterFound], (unsigned long long)total);
             __syncthreads();
-            const unsigned long long base = *sBase + before;
-            for (int i = ln; i < staged; i += 64)
-                if (base + i < p.cap) store_pair(base + i, sStage[i]);
+            write_staged(*sBase + before, ln);
         }
     }
     sign_off();
@@ -1146,7 +1156,17 @@ hipError_t launch_join_grid(JoinParams p, bool rows128, bool tall, bool epilogue
     // Tiles of up to 16 slabs gather their hit bits in their last slab; longer ones screen behind the k-loop.
     const bool bitsInLastSlab = epilogue && p.nSlabs <= 16;
     const int variant = (oneSlab ? 8 : 0) | (tall ? 2 : 0) | (rows128 ? 1 : 0);
-    if (bitsInLastSlab) {
+    if (epilogue && p.symmetric) {
+        const int mirrorVariant = (oneSlab ? 4 : bitsInLastSlab ? 2 : 0) | (tall ? 1 : 0);
+        switch (mirrorVariant) {
+            case 5: join_kernel<true, true, 256, true, true, true><<<g, b, 0, stream>>>(p); break;
+            case 4: join_kernel<true, false, 256, true, true, true><<<g, b, 0, stream>>>(p); break;
+            case 3: join_kernel<true, true, 256, false, true, true><<<g, b, 0, stream>>>(p); break;
+            case 2: join_kernel<true, false, 256, false, true, true><<<g, b, 0, stream>>>(p); break;
+            case 1: join_kernel<true, true, 256, false, false, true><<<g, b, 0, stream>>>(p); break;
+            default: join_kernel<true, false, 256, false, false, true><<<g, b, 0, stream>>>(p); break;
+        }
+    } else if (bitsInLastSlab) {
         switch (variant) {
             case 11: join_kernel<true, true, 128, true, true><<<g, b, 0, stream>>>(p); break;
             case 10: join_kernel<true, true, 256, true, true><<<g, b, 0, stream>>>(p); break;
@@ -1211,7 +1231,9 @@ hipError_t launch_join(const JoinLaunch& launch, hipStream_t stream) {
     // many workgroups) still fit one round is computed in full in those: a 128-row tile costs about 0.7 of a 256-row
     // one (64 x 64 wave sub-tiles need a third more LDS fragment reads per MFMA), measured on Exp(40) data 1.1x - 1.4x
     // faster at 1000 and 2154 points, 1.4x slower at 3000 (288 tiles of 128 rows: two rounds).  (Never both: the
-    // diagonal logic assumes square tiles.)
+    // diagonal logic assumes square tiles.)  Between the two, up to 4096 points, both run in one round of 256-row tiles and
+    // the triangle takes 0.7 to 1.02 of the full matrix's time: 2817 x 64 with 64 neighbours 26.8 against 27.3 us, 4096 x
+    // 1024 with 16 46.0 against 42.5, 4096 x 128 with 512 82.6 against 56.7.
     // FASTED_TILE_ROWS=256 or 128 in the environment overrides the height (tests run both).
     const unsigned long long tiles128 = (unsigned long long)((l.nQ + 127) / 128) * ((l.nC + kTile - 1) / kTile);
     const bool mayMirror = l.selfJoin && l.triangle != Triangle::kFull;
