@@ -635,21 +635,28 @@ typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 // next candidate row is on its way.  Measured, general -> sliced: 50021 x 384 with 5.1 million pairs 510 -> 368 us,
 // 20000 x 1024 with 1.0 million 258 -> 176, 5000 x 4096 with 0.5 million 498 -> 300.
 constexpr int kDistThreads = 256;
+constexpr u32 kTurnPairs = 8u << 20;  // (the list of a stretch, 64 MB, stays in the Infinity Cache for all XCDs)
 
 template <int kLanes, int kChunks, int kPer>
 __global__ void __launch_bounds__(kDistThreads) sliced_distances_kernel(const u32x4* __restrict__ ptsQ, long long ldQ16, int nQ,
                                                                       const u32x4* __restrict__ ptsC, long long ldC16, int nC,
                                                                       int chunksPerRow, const int2* __restrict__ pairs,
                                                                       u32 count, float* __restrict__ out,
-                                                                      u32 slices, int sliceRows) {
+                                                                      u32 slices, int sliceRows, u32 stretch) {
     constexpr u32 kBatch = kPer * kDistThreads;  // pairs a workgroup looks through
     __shared__ int2 found[kBatch];
     __shared__ unsigned short where[kBatch];
     __shared__ u32 total;
-    // workgroup number = ((pass * batches) + batch) * 8 + XCD, slice = pass * 8 + XCD
+    // workgroup number = ((pass * batches) + batch) * 8 + XCD, slice = pass * 8 + XCD; the XCDs go through every `stretch`
+    // batches from different ones on, each from where its slice lies in a list whose candidates ascend
     const u32 batches = gridDim.x / slices;
     const u32 slice = blockIdx.x / (8 * batches) * 8 + blockIdx.x % 8;
-    const u32 first = blockIdx.x / 8 % batches * kBatch;
+    u32 batch = blockIdx.x / 8 % batches;
+    if (stretch != 0) {
+        const u32 start = batch / stretch * stretch, length = min(stretch, batches - start);
+        batch = start + (batch - start + slice * length / slices) % length;
+    }
+    const u32 first = batch * kBatch;
     const u32 here = min(kBatch, count - first);
     const int lane = threadIdx.x & 63;
     if (threadIdx.x == 0) total = 0;
@@ -1008,32 +1015,45 @@ hipError_t launch_pair_distances(const void* queries, long long ldQ, int nQ, con
     // Slices pay where the candidates fit the eight L2 caches and not one of them (up to about 6 MB to a slice: at 4.8 to 6.7
     // MB eight slices were faster than sixteen), where a row is fetched often (8 pairs per candidate), and where looking
     // through the list once per slice, 8 bytes a pair, is little against a row (an eighth; 60000 x 128, 256 bytes a row:
-    // 143 us sliced, 143 without).  Below 1.6 GB of rows to fetch the chip is not busy for long enough (9000 x 3000 with 193
+    // 143 us sliced, 143 without).  A query row is fetched again in every slice, so a query needs two pairs in each: row-major
+    // lists of random candidates, without -> sliced, 50000 x 2048 (40 slices) 24 pairs a query 715 -> 1006 us, 100 a query
+    // 2840 -> 2730; 25000 x 2048 (24 slices) 24 a query 350 -> 423, 100 a query 1390 -> 950.  (Lists in no order fetch the
+    // query row for every pair either way and would gain 10 - 15 % in slices below that line as well.)  Below 1.6 GB of rows to fetch the chip is not busy for long enough (9000 x 3000 with 193
     // thousand pairs, 1.2 GB: 165 us sliced, 151 without).
     const u64 rowBytes = (u64)dPad * 2, bytes = rowBytes * (u64)nC, sliceBytes = 6ull << 20;
     const u64 slices = 8 * ((bytes + 8 * sliceBytes - 1) / (8 * sliceBytes));
-    if (bytes <= 4ull << 20 || slices > rowBytes / 64 || count / 8 < (u64)nC || count * rowBytes < 3ull << 29 ||
+    if (bytes <= 4ull << 20 || slices > rowBytes / 64 || count / 8 < (u64)nC || count / (2 * slices) < (u64)nQ || count * rowBytes < 3ull << 29 ||
         count > 1ull << 30 || count / 2048 * slices >= 1ull << 23 || chunks > 64 * 8) {
         const u64 blocks = (count * 16 + 255) / 256;
         pair_distances_kernel<<<dim3((unsigned)(blocks > 16384ull ? 16384ull : blocks)), dim3(256), 0, stream>>>(
             q, ldQ / 8, nQ, c, ldC / 8, nC, chunks, list, count, out);
         return hipGetLastError();
     }
+    const bool thin = count / (16 * slices) < (u64)nQ;
     const int sliceRows = (int)(((u64)nC + slices - 1) / slices);
-    auto launch = [&](auto kernel, u32 batch) {
+    auto launch = [&](auto kernel, u32 batch, bool turned) {
         const dim3 grid((unsigned)((count + batch - 1) / batch * slices));
         kernel<<<grid, dim3(kDistThreads), 0, stream>>>(q, ldQ / 8, nQ, c, ldC / 8, nC, chunks, list, (u32)count, out,
-                                                        (u32)slices, sliceRows);
+                                                        (u32)slices, sliceRows, turned ? kTurnPairs / batch : 0u);
     };
     // As few lanes per pair as hold the row in four chunks each, up to 64.  Only a lane's last chunk may lie beyond the
     // row, so a kernel serves more than kLanes * (kChunks - 1) and up to kLanes * kChunks chunks (the rule above leaves
     // no row of fewer than 32).  Lists of less than a million pairs go in smaller batches, so that every CU has work.
+    // Where the pairs of a query are few (`thin`: less than 16 to a slice) and its candidates are its neighbours in the set,
+    // whole batches belong to one slice: all XCDs but one would pass over them at the same time, and the one would have too
+    // few.  For longer rows, whose batches take long, the XCDs then start in different places and the batches are halved up to
+    // 2 or 8 million pairs.  100 candidates near the query, without slices / XCDs in step / this: 12000 x 2048 334 / 476 / 355
+    // us, 25000 x 2048 740 / 966 / 715, 12000 x 1024 182 / 231 / 176; random candidates 632 / 369 / 375, 1398 / 910 / 952, 302 /
+    // 171 / 177.  Left: 2500 x 4096 with 250 thousand pairs 145 / 170 / 172 near, 200 / 152 / 152 random.
     auto launch_for = [&](auto lanes, auto perLane) {
         constexpr int kLanes = decltype(lanes)::value, kChunks = decltype(perLane)::value;
+        const bool turned = kLanes >= 32 && thin;
         if (count < 1ull << 20)
-            launch(sliced_distances_kernel<kLanes, kChunks, 2>, 2 * kDistThreads);
+            launch(sliced_distances_kernel<kLanes, kChunks, 2>, 2 * kDistThreads, turned);
+        else if (turned && count < (kLanes == 64 ? 1ull << 23 : 1ull << 21))
+            launch(sliced_distances_kernel<kLanes, kChunks, 4>, 4 * kDistThreads, turned);
         else
-            launch(sliced_distances_kernel<kLanes, kChunks, 8>, 8 * kDistThreads);
+            launch(sliced_distances_kernel<kLanes, kChunks, 8>, 8 * kDistThreads, turned);
     };
     using std::integral_constant;
     integral_constant<int, 16> lanes16;

@@ -18,7 +18,8 @@ def test_sliced_distances_match_fp64(n, d):
 
     gen = torch.Generator(device="cuda").manual_seed(n + d)
     ld = (d + 63) // 64 * 64
-    count = max(8 * n + 7, (3 << 29) // (2 * ld) + 5)  # the smallest lists that go through the slices
+    slices = 8 * -(-2 * ld * n // (48 << 20))
+    count = max(8 * n + 7, 2 * slices * n + 7, (3 << 29) // (2 * ld) + 5)  # the smallest lists that go through the slices
     pts = torch.zeros((n, ld), dtype=torch.float16, device="cuda")
     pts[:, :d] = torch.randn((n, d), generator=gen, device="cuda").to(torch.float16)
     pairs = torch.randint(0, n, (count, 2), generator=gen, device="cuda", dtype=torch.int32)
@@ -40,6 +41,63 @@ def test_sliced_distances_match_fp64(n, d):
         # each of d products and additions rounds to half a unit of 2^-24 at most; the square root halves it
         bound = 1e-7 + 0.5 * (ld / 16 + 20) * 2.0**-24
         assert bool(((got[r : r + step][: len(ok)][ok].double() - want).abs() <= bound * want).all())
+
+
+
+# rows of more than 512 dimensions and fewer than 16 pairs per query and slice: batches of 512, 1024 and 2048 pairs that the
+# XCDs go through from different ones on, in one stretch of the list and in two
+@pytest.mark.parametrize("n,d,count", [(9001, 1024, 900001), (12001, 1024, 1200007), (25007, 1088, 2600003), (12001, 2049, 1200001),
+                                       (60001, 1024, 8 * 1024 * 1024 + 700001)])
+def test_sliced_distances_of_thin_lists_match_fp64(n, d, count):
+    import torch
+
+    import fasted_amd as fasted
+
+    gen = torch.Generator(device="cuda").manual_seed(n + d)
+    ld = (d + 63) // 64 * 64
+    pts = torch.zeros((n, ld), dtype=torch.float16, device="cuda")
+    pts[:, :d] = torch.randn((n, d), generator=gen, device="cuda").to(torch.float16)
+    q = torch.sort(torch.randint(0, n, (count,), generator=gen, device="cuda")).values
+    c = (q + torch.randint(-200, 200, (count,), generator=gen, device="cuda")) % n
+    c[count // 2 :] = torch.randint(0, n, (count - count // 2,), generator=gen, device="cuda")
+    pairs = torch.stack([q, c], 1).to(torch.int32)
+    got = torch.full((count + 1,), -2.0, dtype=torch.float32, device="cuda")
+    fasted.pair_distances_device(pts.data_ptr(), n, ld, pts.data_ptr(), n, ld, d, pairs.data_ptr(), count, got.data_ptr())
+    assert float(got[-1]) == -2.0
+    step = (1 << 26) // d
+    for r in range(0, count, step):
+        i = pairs[r : r + step].long()
+        want = (pts[i[:, 0]].double() - pts[i[:, 1]].double()).norm(dim=1)
+        bound = 1e-7 + 0.5 * (ld / 16 + 20) * 2.0**-24  # as above
+        assert bool(((got[r : r + step][: len(i)].double() - want).abs() <= bound * want).all())
+
+
+@pytest.mark.parametrize("near", [False, True])
+def test_thin_lists_take_no_longer_than_where_nothing_is_sliced(near):
+    # the same bytes in the same number of distinct rows: 50 000 x 2048 could go in slices (40, where a query has 24 pairs: 1.4
+    # and 2.0 times as long), 100 000 x 1024 does not
+    import torch
+
+    import fasted_amd as fasted
+
+    gen = torch.Generator(device="cuda").manual_seed(2)
+    times = []
+    for n, d in ((50000, 2048), (100000, 1024)):
+        pts = torch.randn((n, d), generator=gen, device="cuda").to(torch.float16)
+        q = torch.arange(n, device="cuda").repeat_interleave(24)
+        c = (q + torch.randint(-48, 48, q.shape, generator=gen, device="cuda")) % n if near else torch.randint(0, n, q.shape, generator=gen, device="cuda")
+        pairs = torch.stack([q, c], 1).to(torch.int32)
+        out = torch.empty(len(q), dtype=torch.float32, device="cuda")
+        best = 1e9
+        for _ in range(8):
+            begin, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            begin.record()
+            fasted.pair_distances_device(pts.data_ptr(), n, d, pts.data_ptr(), n, d, d, pairs.data_ptr(), len(q), out.data_ptr())
+            end.record()
+            torch.cuda.synchronize()
+            best = min(best, begin.elapsed_time(end))
+        times.append(best)
+    assert times[0] < 1.2 * times[1]
 
 
 def test_sliced_distances_of_subnormal_large_and_infinite_coordinates():
