@@ -308,9 +308,11 @@ __device__ __forceinline__ void static_for(F&& f) {
 // k-loop (tiles of up to 16 slabs; see slab_step).
 // kMirror: only tiles on and above the diagonal are computed, and pairs above it are written in both orientations.  Such
 // a pair is staged once and written twice when its region leaves: staged twice, the mirrored tile of a workgroup overflowed
-// its regions where the two tiles of the full matrix did not, and at 4096 x 64 with 128 neighbours the triangle took
-// 32.7 us, 27.9 the full matrix (now 28.3; 512 neighbours 90 -> 56, 100000 x 384 with 1000 3.67 -> 3.19 ms).  A variant of
-// its own because the full matrix became 1 - 2 % slower when the choice was made at run time (100000 x 128 2.18 -> 2.21 ms).
+// its region where the two tiles of the full matrix did not, and at 4096 x 64 with 128 neighbours the triangle took 32.7 us,
+// 27.9 the full matrix.  Join kernel alone, staged twice -> this: 4096 x 64 with 128 neighbours 24.6 -> 18.8 us, with 500
+// 80.9 -> 47.6, 20000 x 256 with 1000 705 -> 369, 100000 x 384 with 1000 3.65 -> 3.13 ms, 100000 x 128 with 64 1119 -> 1109 us.
+// A variant of its own because the full matrix became 1 - 2 % slower when the choice was made at run time (100000 x 128
+// 2.18 -> 2.21 ms).
 template <bool kEpilogue, bool kTall, int kTileRows, bool kOneSlab, bool kBitsInLastSlab = false, bool kMirror = false>
 __global__ void __launch_bounds__(kThreads, 1) join_kernel(JoinParams p) {
     static_assert(!kMirror || (kEpilogue && kTileRows == 256), "pairs are mirrored across the diagonal of square tiles");
@@ -435,11 +437,26 @@ __global__ void __launch_bounds__(kThreads, 1) join_kernel(JoinParams p) {
                            (unsigned long long)(unsigned)rec.x | ((unsigned long long)(unsigned)rec.y << 32),
                            __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     };
+    // (past the capacity: counted, not stored)
     auto write_staged = [&](unsigned long long base, int ln) {
-        for (int i = ln; i < staged; i += 64) {
-            const int2 rec = sStage[i];
-            if (base + i < p.cap) store_pair(base + i, rec);  // past the capacity: counted, not stored
-            if (doubled && base + staged + i < p.cap) store_pair(base + staged + i, int2{rec.y, rec.x});
+        if constexpr (kMirror) {
+            // All reads are issued before the first store: the other waves wait for this one at the next barrier (one record
+            // at a time, 100000 x 128 took 1130 us instead of 1104).  The two records of a pair lie side by side: the sort's
+            // LDS counters are what neighbouring records contend for (one orientation behind the other, the sort of 200
+            // million pairs took 0.27 ms longer).
+            int2 rec[kWaveStagePairs / 64];
+#pragma unroll
+            for (int k = 0; k < kWaveStagePairs / 64; ++k) rec[k] = sStage[ln + k * 64];
+#pragma unroll
+            for (int k = 0; k < kWaveStagePairs / 64; ++k) {
+                const int i = ln + k * 64;
+                const unsigned long long slot = base + (doubled ? 2 * i : i);
+                if (i < staged && slot < p.cap) store_pair(slot, rec[k]);
+                if (doubled && i < staged && slot + 1 < p.cap) store_pair(slot + 1, int2{rec[k].y, rec[k].x});
+            }
+        } else {
+            for (int i = ln; i < staged; i += 64)
+                if (base + i < p.cap) store_pair(base + i, sStage[i]);
         }
     };
     auto flush_wave = [&]() {

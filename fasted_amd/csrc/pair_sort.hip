@@ -125,7 +125,7 @@ template <bool kRecords>
 __global__ void __launch_bounds__(kSortThreads) count_keys_kernel(const void* __restrict__ in, u32 count, KeyForm form,
                                                                   int shift, const Bucket* __restrict__ parents,
                                                                   u32 parentCount, u32 chunk, u32* __restrict__ bins,
-                                                                  SortState* __restrict__ state, u64 epoch) {
+                                                                  SortState* __restrict__ state) {
     constexpr int kBins = kRecords ? kBins1 : kBins2;
     typedef std::conditional_t<kRecords, u64, u32> Key;
     __shared__ u32 local[kBins];
@@ -134,7 +134,6 @@ __global__ void __launch_bounds__(kSortThreads) count_keys_kernel(const void* __
     if (kRecords) {
         if (blockIdx.x == 0 && threadIdx.x == 0) state->windows = 0;
     } else {
-        if (broken_off(state, epoch)) return;
         const u32 b = find_bucket(parents, parentCount, blockIdx.x, chunk, &which);
         if (b == ~0u) return;
         const Bucket p = parents[b];
@@ -206,8 +205,8 @@ __global__ void __launch_bounds__(kSortThreads) plan_buckets_kernel(u32* __restr
     Bucket p{0u, count, 0u, 0u, lastLow, 0u, {0u, 0u}};
     u32 firstChild = 0, ids = childCount;
     if (!kFirst) {
-        if (state->brokenOff[0] == epoch) return;  // (the other one may turn while this kernel runs)
         p = parents[blockIdx.x];
+        if (state->brokenOff[0] == epoch) return;  // (the other one may turn while this kernel runs)
         shift = (int)p.shift;
         firstChild = p.start / target + blockIdx.x;
         ids = (blockIdx.x + 1 < gridDim.x ? parents[blockIdx.x + 1].start / target + blockIdx.x + 1 : childCount) - firstChild;
@@ -908,7 +907,7 @@ hipError_t distribute(u64* records, u32 count, const SortPlan& p, u64 lastKey, K
     u32* const keysB = keysA + count;
     const Bucket none{};
     if (!p.twoLevels) {
-        count_keys_kernel<true><<<blocks(count, 4096), threads, 0, stream>>>(records, count, form, p.shift, nullptr, 0u, 4096u, bins1, state, epoch);
+        count_keys_kernel<true><<<blocks(count, 4096), threads, 0, stream>>>(records, count, form, p.shift, nullptr, 0u, 4096u, bins1, state);
         plan_buckets_kernel<true><<<1, threads, 0, stream>>>(bins1, count, p.shift, lastHigh, lastLow, nullptr, p.target, p.ids1, 0u,
                                                              buckets1, childOf1, cursors1, windowList, p.maxWindows, state, epoch,
                                                              ws->hostWordDev);
@@ -919,12 +918,12 @@ hipError_t distribute(u64* records, u32 count, const SortPlan& p, u64 lastKey, K
     } else {
         const u32 chunk1 = (u32)((count / 1024 + 4095) / 4096 * 4096 + 4096), chunk2 = 32768;
         constexpr u32 kScatter = 8 * kSortThreads;
-        count_keys_kernel<true><<<blocks(count, chunk1), threads, 0, stream>>>(records, count, form, p.shift, nullptr, 0u, chunk1, bins1, state, epoch);
+        count_keys_kernel<true><<<blocks(count, chunk1), threads, 0, stream>>>(records, count, form, p.shift, nullptr, 0u, chunk1, bins1, state);
         plan_buckets_kernel<true><<<1, threads, 0, stream>>>(bins1, count, p.shift, lastHigh, lastLow, nullptr, p.target1, p.ids1, p.target,
                                                              buckets1, childOf1, cursors1, windowList, 0u, state, epoch, ws->hostWordDev);
         scatter_keys_kernel<true, 8><<<blocks(count, kScatter), threads, 0, stream>>>(
             records, count, form, p.shift, nullptr, 0u, p.target1, childOf1, cursors1, keysA, epoch, state);
-        count_keys_kernel<false><<<count / chunk2 + p.ids1, threads, 0, stream>>>(keysA, count, form, 0, buckets1, p.ids1, chunk2, bins2, state, epoch);
+        count_keys_kernel<false><<<count / chunk2 + p.ids1, threads, 0, stream>>>(keysA, count, form, 0, buckets1, p.ids1, chunk2, bins2, state);
         plan_buckets_kernel<false><<<p.ids1, threads, 0, stream>>>(bins2, count, 0, 0u, 0u, buckets1, p.target, p.ids2, 0u,
                                                                    buckets2, childOf2, cursors2, windowList, p.maxWindows, state, epoch,
                                                                    ws->hostWordDev);
