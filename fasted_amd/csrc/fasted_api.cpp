@@ -410,7 +410,7 @@ void upload_rows(void* dst, size_t pitch, const void* src, size_t rowBytes, size
 }
 
 // The largest pair count <= `want` whose records fit the free device memory together with what the sort of
-// that many records needs beside them (a second key buffer and the radix sort's storage), as Pairs::init
+// that many records needs beside them (the most any of its ways takes, see sort_scratch_bytes), as Pairs::init
 // shrinks the reference's buffer to the free memory (source/pair.cuh:69-85).
 unsigned long long fit_pairs_with_sort(unsigned long long want) {
     size_t freeB = 0, totalB = 0;
@@ -427,7 +427,8 @@ unsigned long long fit_pairs_with_sort(unsigned long long want) {
 
 // Device memory of one host-to-host join.  A buffer of up to 256 MB is kept when the call ends, for the next call (an
 // allocation costs 0.3 to 0.4 ms); there is at most one, releaseResources() frees it, and a call on another device
-// does not use it.  A caller takes it out while it works with it, so that calls of several threads do not share it.
+// does not use it.  A call takes it out while it works with it.  (The workspaces of the join and the sort are shared: calls
+// of several threads must not overlap.)
 class HostJoinBuffer {
 public:
     explicit HostJoinBuffer(size_t bytes) {
@@ -819,8 +820,8 @@ struct PairWorkspace {
 } g_pairWs;
 
 // Pair buffer of N*256 records (source/findPairs.cuh:644-647), shrunk to what the device can hold together
-// with what the sort of a full buffer needs (a second key buffer and the radix sort's storage), as
-// Pairs::init shrinks it to the free memory (source/pair.cuh:69-85).  Kept until a larger one is needed.
+// with what the sort of a full buffer needs, as Pairs::init shrinks it to the free memory (source/pair.cuh:69-85).
+// Kept until a larger one is needed.
 unsigned long long ensure_pair_buffer(int n) {
     const unsigned long long want = (unsigned long long)n * 256ull;
     if (g_pairWs.dPairs && g_pairWs.capPairs >= want) return want;

@@ -58,10 +58,10 @@ int index_bits(long long n) {  // bits of the largest index of n items; 32 when 
 // in 1/4096 of the key range), go to the radix sort.  A few times 4096 records are ordered by one workgroup alone (sort_bucket_kernel on the records themselves).
 // Bound by memory traffic: 32 bytes per record in one level, 44 in two, of which a key on its way is 4 (the radix sort
 // with its pack and unpack moves 120 at 36 key bits); below a million records by the launches.  Measured, join records,
-// radix sort -> this: 4 849 records 45 -> 18 us, 135 thousand 75 -> 34, 974 thousand 195 -> 40, 6.5 million 330 -> 160,
-// 200 million 7.5 -> 2.6 ms; 1.04 million in 200 000 rows 200 -> 54, 0.6 million of which 0.4 in 2000 of 100 000 rows 165
-// -> 75.  Slower where a list that breaks off is short, or one row holds most of a long one: 100 thousand records, half of
-// them in one row of a million, 71 -> 99 us, 3 million, half of them in one row of two million, 262 -> 324.
+// radix sort -> this: 4 849 records 45 -> 18 us, 135 thousand 75 -> 34, 974 thousand 195 -> 43, 6.5 million 330 -> 160,
+// 200 million 7.5 -> 2.6 ms; 1.04 million in 200 000 rows 200 -> 52, 0.6 million of which 0.4 in 2000 of 100 000 rows 165
+// -> 76.  Slower where a list that breaks off is short, or one row holds most of a long one: 100 thousand records, half of
+// them in one row of a million, 71 -> 102 us, 3 million, half of them in one row of two million, 262 -> 323.
 // Where the lines between one workgroup, one level and two lie: one workgroup takes 8192 records in 22 us, two launches
 // less than the 32 us of one level; one level takes 1.04 million records in 53 us, two take 1.1 million in 65.  Where a list
 // breaks off, two levels took 500 thousand records in 150 us and the radix sort 180, 100 thousand in 140 and 100.
@@ -631,8 +631,8 @@ typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 // one XCD -- workgroups are dealt to the XCDs in turn; nothing but time depends on it -- look through all pairs for those
 // of one slice, whose rows then stay in that XCD's L2.  kLanes lanes share a pair, kChunks chunks of 16 bytes of
 // either row each, all in registers; a query row stays there while the pairs that follow name the same query, and the
-// next candidate row is on its way.  Measured, general -> sliced: 50021 x 384 with 5.1 million pairs 510 -> 368 us,
-// 20000 x 1024 with 1.0 million 258 -> 176, 5000 x 4096 with 0.5 million 498 -> 300.
+// next candidate row is on its way.  Measured, general -> sliced: 50021 x 384 with 5.1 million pairs 506 -> 350 us,
+// 20000 x 1024 with 1.0 million 258 -> 176, 5000 x 4096 with 0.5 million 498 -> 304.
 constexpr int kDistThreads = 256;
 constexpr u32 kTurnPairs = 8u << 20;  // (the list of a stretch, 64 MB, stays in the Infinity Cache for all XCDs)
 

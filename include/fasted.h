@@ -64,7 +64,8 @@ Results runFromFile(const char* filename, double epsilon, bool savePairs);
 Results reRun(double epsilon, bool savePairs);
 
 /* source/main.cu:74,280 (there it recurses into itself; here it frees the resident
- * dataset as its comment intends, source/findPairs.cuh:766-776). */
+ * dataset as its comment intends, source/findPairs.cuh:766-776), and every buffer that the library keeps
+ * between calls: workspaces, pair and sort buffers, the buffer of fasted_self_join. */
 void releaseResources(void);
 
 /* ---- group 2: raw buffers ----------------------------------------------------------
@@ -111,7 +112,10 @@ enum {
  * patterns (what source/DataLoader/PointListBuilder.hpp:57-73 produces, before padding);
  * up to `cap` pairs are written to `out` sorted row-major; *found counts every pair
  * (source/pair.cuh:123-133), *stored = min(found, cap).  Replaces the body of
- * SimSearch::FindPairs (source/findPairs.cuh:615-764) for a caller that owns its data. */
+ * SimSearch::FindPairs (source/findPairs.cuh:615-764) for a caller that owns its data.
+ * Device memory: the padded points and `cap` records (at least 32 MB of them where D % 64 != 0), and what the sort
+ * needs.  A buffer of up to 256 MB for points and records stays allocated for the next call, one for the whole
+ * process; releaseResources() frees it.  `cap` of more than 2^45 is refused. */
 int fasted_self_join(const uint16_t* points, long long n, int d, double epsilon, FastedPair* out,
                      unsigned long long cap, unsigned long long* found, unsigned long long* stored);
 
@@ -119,7 +123,7 @@ int fasted_self_join(const uint16_t* points, long long n, int d, double epsilon,
  * points are streamed through the device in blocks of `block_rows` points (rounded up to a multiple of
  * 256).  Device memory used: three blocks, 4 bytes per point of the whole dataset (each point's squared norm
  * enters the join through one float, formed when its block is first uploaded), and a pair buffer of
- * min(cap, block_rows*256) records (about three times that while sorting).  Blocks that a later join still
+ * min(cap, block_rows*256) records (two to three times that while sorting).  Blocks that a later join still
  * needs stay on the device: with B blocks about B*(B-2)+2 block uploads instead of B*B.  Output as fasted_self_join: row-major, *found counts every pair,
  * at most `cap` are written; in addition the pairs of one block of query points beyond block_rows*256 are
  * counted but not written.  The reference has no such path: its dataset, twice, and N*256 pair records
@@ -142,9 +146,10 @@ int fasted_self_join_blocked(const uint16_t* points, long long n, int d, double 
  * count to the host (a few microseconds before the stream itself reports idle, a fifth of such a call).  Every
  * pair record and squared norm is in device memory by then, for any stream, copy or kernel that reads them next;
  * the stream may still answer hipStreamQuery with hipErrorNotReady for a moment.  With FASTED_SORT_PAIRS the sort's
- * device buffers (a second key buffer and the radix sort's storage, about twice the bytes of the stored
- * pairs) are allocated by the library and kept for the next sort; so are the counters and, without d_sums,
- * the squared norms.  releaseResources() frees all of it.  Replaces the
+ * device buffers are allocated by the library and kept for the next sort: none up to 8192 pairs, 4 bytes a pair up to
+ * 2^20 and 8 beyond, and tables of up to about 35 MB; lists that leave the distribution for the radix sort take 8 bytes
+ * a pair and its storage, about as much again.  The counters and, without d_sums, the squared norms are kept as well.
+ * releaseResources() frees all of it.  Replaces the
  * kernel launches of source/findPairs.cuh:632-687 (ComputeSquaredSums x2,
  * initOnDemandRasterizer, FindPairsKernel) and the sort of :703-704. */
 int fasted_self_join_device(const void* d_points, long long n, int d, long long ld, double epsilon, float* d_sums,
