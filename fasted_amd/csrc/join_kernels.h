@@ -107,8 +107,8 @@ hipError_t sort_pairs_row_major(void* pairs, unsigned long long count, hipStream
 // Device bytes a sort of `count` pairs needs beside the pairs themselves.
 size_t sort_scratch_bytes(unsigned long long count);
 
-// out[i] = Euclidean distance of pair i (FP32 sum of squared differences over dPad dimensions); NaN for a
-// pair that names a point outside [0, nQ) x [0, nC).
+// out[i] = Euclidean distance of pair i (FP32 sum of squared differences over dPad dimensions; pair_distances.hip); NaN for
+// a pair that names a point outside [0, nQ) x [0, nC).
 hipError_t launch_pair_distances(const void* queries, long long ldQ, int nQ, const void* candidates, long long ldC,
                                  int nC, int dPad, const void* pairs, unsigned long long count, float* out,
                                  hipStream_t stream);

@@ -1,5 +1,4 @@
-// pair_sort.hip -- what happens to the stored pairs on the device after the join: the row-major
-// ordering, and the optional distance of every pair.
+// pair_sort.hip -- row-major order of the stored pairs on the device after the join.
 //
 // The reference sorts its pair buffer with thrust::sort and Pair::operator< (query index,
 // then candidate index; source/pair.cuh:39-45,151-158).  A pair is 8 bytes with the query
@@ -621,160 +620,6 @@ __global__ void __launch_bounds__(kThreads, kRecords ? 4 : 8) sort_bucket_kernel
     for (u32 i = t; i < m; i += kThreads) put_record(i, result[i]);
 }
 
-typedef _Float16 half8 __attribute__((ext_vector_type(8)));
-
-// Euclidean distance of every listed pair, sum of squared differences in FP32 (no cancellation, unlike
-// the expansion the join itself tests).  Pairs that name a point outside its set get NaN.
-//
-// What bounds it is fetching the candidate rows, which come in no order: 768 bytes per pair at 384 dimensions from the
-// Infinity Cache, at 7 TB/s.  The sliced kernel cuts the candidates into 8 slices (or a multiple), and the workgroups of
-// one XCD -- workgroups are dealt to the XCDs in turn; nothing but time depends on it -- look through all pairs for those
-// of one slice, whose rows then stay in that XCD's L2.  kLanes lanes share a pair, kChunks chunks of 16 bytes of
-// either row each, all in registers; a query row stays there while the pairs that follow name the same query, and the
-// next candidate row is on its way.  Measured, general -> sliced: 50021 x 384 with 5.1 million pairs 506 -> 350 us,
-// 20000 x 1024 with 1.0 million 258 -> 176, 5000 x 4096 with 0.5 million 498 -> 304.
-constexpr int kDistThreads = 256;
-constexpr u32 kTurnPairs = 8u << 20;  // (the list of a stretch, 64 MB, stays in the Infinity Cache for all XCDs)
-
-template <int kLanes, int kChunks, int kPer>
-__global__ void __launch_bounds__(kDistThreads) sliced_distances_kernel(const u32x4* __restrict__ ptsQ, long long ldQ16, int nQ,
-                                                                      const u32x4* __restrict__ ptsC, long long ldC16, int nC,
-                                                                      int chunksPerRow, const int2* __restrict__ pairs,
-                                                                      u32 count, float* __restrict__ out,
-                                                                      u32 slices, int sliceRows, u32 stretch) {
-    constexpr u32 kBatch = kPer * kDistThreads;  // pairs a workgroup looks through
-    __shared__ int2 found[kBatch];
-    __shared__ unsigned short where[kBatch];
-    __shared__ u32 total;
-    // workgroup number = ((pass * batches) + batch) * 8 + XCD, slice = pass * 8 + XCD; the XCDs go through every `stretch`
-    // batches from different ones on, each from where its slice lies in a list whose candidates ascend
-    const u32 batches = gridDim.x / slices;
-    const u32 slice = blockIdx.x / (8 * batches) * 8 + blockIdx.x % 8;
-    u32 batch = blockIdx.x / 8 % batches;
-    if (stretch != 0) {
-        const u32 start = batch / stretch * stretch, length = min(stretch, batches - start);
-        batch = start + (batch - start + slice * length / slices) % length;
-    }
-    const u32 first = batch * kBatch;
-    const u32 here = min(kBatch, count - first);
-    const int lane = threadIdx.x & 63;
-    if (threadIdx.x == 0) total = 0;
-    __syncthreads();
-    {
-        const u32 waveFirst = threadIdx.x / 64 * (kBatch / (kDistThreads / 64)) + lane;
-        int2 pr[kPer];
-#pragma unroll
-        for (int e = 0; e < kPer; ++e) pr[e] = pairs[first + min(waveFirst + e * 64, here - 1)];
-        // the pairs of this slice, in order within a wave
-        u64 take[kPer];
-        u32 mine = 0;
-#pragma unroll
-        for (int e = 0; e < kPer; ++e) {
-            const bool valid = pr[e].x >= 0 && pr[e].x < nQ && pr[e].y >= 0 && pr[e].y < nC;
-            const bool real = waveFirst + e * 64 < here;
-            if (!valid && real && slice == 0) out[first + waveFirst + e * 64] = __builtin_nanf("");
-            take[e] = __builtin_amdgcn_ballot_w64(real && valid && (u32)pr[e].y - slice * (u32)sliceRows < (u32)sliceRows);
-            mine += __builtin_popcountll(take[e]);
-        }
-        u32 base = 0;
-        if (lane == 0) base = atomicAdd(&total, mine);
-        base = __builtin_amdgcn_readfirstlane(base);
-#pragma unroll
-        for (int e = 0; e < kPer; ++e) {
-            const u32 at = base + __builtin_amdgcn_mbcnt_hi((u32)(take[e] >> 32), __builtin_amdgcn_mbcnt_lo((u32)take[e], 0u));
-            if (take[e] >> lane & 1) {
-                found[at] = pr[e];
-                where[at] = (unsigned short)(waveFirst + e * 64);
-            }
-            base += __builtin_popcountll(take[e]);
-        }
-    }
-    __syncthreads();
-    constexpr u32 kGroups = kDistThreads / kLanes;
-    const u32 n = total, group = threadIdx.x / kLanes;
-    const int sub = threadIdx.x % kLanes;
-    const u32 per = (n + kGroups - 1) / kGroups, begin = min(group * per, n), end = min(begin + per, n);
-    const bool whole = sub + (kChunks - 1) * kLanes < chunksPerRow;  // this lane has a last chunk
-    auto load = [&](u32x4 (&r)[kChunks], const u32x4* row) {
-#pragma unroll
-        for (int k = 0; k < kChunks; ++k) r[k] = row[k + 1 < kChunks || whole ? sub + k * kLanes : 0];
-        if (!whole) r[kChunks - 1] = u32x4{0u, 0u, 0u, 0u};
-    };
-    auto distance2 = [&](const u32x4 (&a)[kChunks], const u32x4 (&b)[kChunks]) {
-        float acc = 0.0f;
-#pragma unroll
-        for (int k = 0; k < kChunks; ++k) {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                // the difference of two halves, widened and rounded once, in one instruction (the compiler widens both first)
-                float lo, hi;
-                asm("v_fma_mix_f32 %0, %1, 1.0, -%2 op_sel_hi:[1,0,1]" : "=v"(lo) : "v"(a[k][e]), "v"(b[k][e]));
-                asm("v_fma_mix_f32 %0, %1, 1.0, -%2 op_sel:[1,0,1] op_sel_hi:[1,0,1]" : "=v"(hi) : "v"(a[k][e]), "v"(b[k][e]));
-                acc = __builtin_fmaf(lo, lo, acc);
-                acc = __builtin_fmaf(hi, hi, acc);
-            }
-        }
-        // within 16 lanes by rotations in the vector unit, beyond that by permutes
-        acc += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, acc), 0x128, 0xf, 0xf, true));
-        acc += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, acc), 0x124, 0xf, 0xf, true));
-        acc += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, acc), 0x122, 0xf, 0xf, true));
-        acc += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, acc), 0x121, 0xf, 0xf, true));
-        if (kLanes >= 32) acc += __shfl_xor(acc, 16, 64);
-        if (kLanes >= 64) acc += __shfl_xor(acc, 32, 64);
-        return acc;
-    };
-    if (begin >= end) return;
-    u32x4 a[kChunks], a1[kChunks], b0[kChunks], b1[kChunks];
-    int2 pr = found[begin];
-    load(a, ptsQ + (long long)pr.x * ldQ16);
-    load(b0, ptsC + (long long)pr.y * ldC16);
-    for (u32 i = begin; i < end; ++i) {
-        const int2 next = found[min(i + 1, end - 1)];
-        load(b1, ptsC + (long long)next.y * ldC16);
-        const bool turn = next.x != pr.x;
-        if (turn) load(a1, ptsQ + (long long)next.x * ldQ16);
-        const float d2 = distance2(a, b0);
-        if (sub == 0) out[first + where[i]] = __builtin_sqrtf(d2);
-#pragma unroll
-        for (int k = 0; k < kChunks; ++k) b0[k] = b1[k];
-        if (turn) {
-#pragma unroll
-            for (int k = 0; k < kChunks; ++k) a[k] = a1[k];
-        }
-        pr = next;
-    }
-}
-
-// The general kernel: 16 lanes walk the two rows of a pair, chunk by chunk.
-__global__ void __launch_bounds__(256) pair_distances_kernel(const u32x4* __restrict__ ptsQ, long long ldQ16, int nQ,
-                                                                  const u32x4* __restrict__ ptsC, long long ldC16, int nC,
-                                                                  int chunksPerRow, const int2* __restrict__ pairs,
-                                                                  unsigned long long count, float* __restrict__ out) {
-    const int sub = threadIdx.x & 15;
-    const unsigned long long groups = ((unsigned long long)gridDim.x * blockDim.x) >> 4;
-    for (unsigned long long g = ((unsigned long long)blockIdx.x * blockDim.x + threadIdx.x) >> 4; g < count; g += groups) {
-        const int2 pr = pairs[g];
-        const bool valid = pr.x >= 0 && pr.x < nQ && pr.y >= 0 && pr.y < nC;
-        float acc = 0.0f;
-        if (valid) {
-            const u32x4* a = ptsQ + (long long)pr.x * ldQ16;
-            const u32x4* b = ptsC + (long long)pr.y * ldC16;
-            for (int c = sub; c < chunksPerRow; c += 16) {
-                const half8 x = __builtin_bit_cast(half8, a[c]);
-                const half8 y = __builtin_bit_cast(half8, b[c]);
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const float diff = (float)x[e] - (float)y[e];
-                    acc = __builtin_fmaf(diff, diff, acc);
-                }
-            }
-        }
-#pragma unroll
-        for (int off = 8; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
-        if (sub == 0) out[g] = valid ? __builtin_sqrtf(acc) : __builtin_nanf("");
-    }
-}
-
 unsigned grid_for(unsigned long long count) {
     unsigned long long blocks = (count + 255) / 256;
     return (unsigned)(blocks > 65536ull ? 65536ull : (blocks ? blocks : 1));
@@ -1001,80 +846,6 @@ hipError_t sort_pairs_row_major(void* pairs, unsigned long long count, hipStream
         if (twoLevels || count < kTwoLevelsAfterOneFrom) break;
     }
     return done ? hipSuccess : radix_sort(records, count, form, queryBits + candidateBits, stream, ws);
-}
-
-hipError_t launch_pair_distances(const void* queries, long long ldQ, int nQ, const void* candidates, long long ldC,
-                                 int nC, int dPad, const void* pairs, unsigned long long count, float* out,
-                                 hipStream_t stream) {
-    if (count == 0) return hipSuccess;
-    const auto* const q = static_cast<const u32x4*>(queries);
-    const auto* const c = static_cast<const u32x4*>(candidates);
-    const auto* const list = static_cast<const int2*>(pairs);
-    const int chunks = dPad / 8;
-    // Slices pay where the candidates fit the eight L2 caches and not one of them (up to about 6 MB to a slice: at 4.8 to 6.7
-    // MB eight slices were faster than sixteen), where a row is fetched often (8 pairs per candidate), and where looking
-    // through the list once per slice, 8 bytes a pair, is little against a row (an eighth; 60000 x 128, 256 bytes a row:
-    // 143 us sliced, 143 without).  A query row is fetched again in every slice, so a query needs two pairs in each: row-major
-    // lists of random candidates, without -> sliced, 50000 x 2048 (40 slices) 24 pairs a query 715 -> 1006 us, 100 a query
-    // 2840 -> 2730; 25000 x 2048 (24 slices) 24 a query 350 -> 423, 100 a query 1390 -> 950.  (Lists in no order fetch the
-    // query row for every pair either way and would gain 10 - 15 % in slices below that line as well.)  Below 1.6 GB of rows to fetch the chip is not busy for long enough (9000 x 3000 with 193
-    // thousand pairs, 1.2 GB: 165 us sliced, 151 without).
-    const u64 rowBytes = (u64)dPad * 2, bytes = rowBytes * (u64)nC, sliceBytes = 6ull << 20;
-    const u64 slices = 8 * ((bytes + 8 * sliceBytes - 1) / (8 * sliceBytes));
-    if (bytes <= 4ull << 20 || slices > rowBytes / 64 || count / 8 < (u64)nC || count / (2 * slices) < (u64)nQ || count * rowBytes < 3ull << 29 ||
-        count > 1ull << 30 || count / 2048 * slices >= 1ull << 23 || chunks > 64 * 8) {
-        const u64 blocks = (count * 16 + 255) / 256;
-        pair_distances_kernel<<<dim3((unsigned)(blocks > 16384ull ? 16384ull : blocks)), dim3(256), 0, stream>>>(
-            q, ldQ / 8, nQ, c, ldC / 8, nC, chunks, list, count, out);
-        return hipGetLastError();
-    }
-    const bool thin = count / (16 * slices) < (u64)nQ;
-    const int sliceRows = (int)(((u64)nC + slices - 1) / slices);
-    auto launch = [&](auto kernel, u32 batch, bool turned) {
-        const dim3 grid((unsigned)((count + batch - 1) / batch * slices));
-        kernel<<<grid, dim3(kDistThreads), 0, stream>>>(q, ldQ / 8, nQ, c, ldC / 8, nC, chunks, list, (u32)count, out,
-                                                        (u32)slices, sliceRows, turned ? kTurnPairs / batch : 0u);
-    };
-    // As few lanes per pair as hold the row in four chunks each, up to 64.  Only a lane's last chunk may lie beyond the
-    // row, so a kernel serves more than kLanes * (kChunks - 1) and up to kLanes * kChunks chunks (the rule above leaves
-    // no row of fewer than 32).  Lists of less than a million pairs go in smaller batches, so that every CU has work.
-    // Where the pairs of a query are few (`thin`: less than 16 to a slice) and its candidates are its neighbours in the set,
-    // whole batches belong to one slice: all XCDs but one would pass over them at the same time, and the one would have too
-    // few.  For longer rows, whose batches take long, the XCDs then start in different places and the batches are halved up to
-    // 2 or 8 million pairs.  100 candidates near the query, without slices / XCDs in step / this: 12000 x 2048 334 / 476 / 355
-    // us, 25000 x 2048 740 / 966 / 715, 12000 x 1024 182 / 231 / 176; random candidates 632 / 369 / 375, 1398 / 910 / 952, 302 /
-    // 171 / 177.  Left: 2500 x 4096 with 250 thousand pairs 145 / 170 / 172 near, 200 / 152 / 152 random.
-    auto launch_for = [&](auto lanes, auto perLane) {
-        constexpr int kLanes = decltype(lanes)::value, kChunks = decltype(perLane)::value;
-        const bool turned = kLanes >= 32 && thin;
-        if (count < 1ull << 20)
-            launch(sliced_distances_kernel<kLanes, kChunks, 2>, 2 * kDistThreads, turned);
-        else if (turned && count < (kLanes == 64 ? 1ull << 23 : 1ull << 21))
-            launch(sliced_distances_kernel<kLanes, kChunks, 4>, 4 * kDistThreads, turned);
-        else
-            launch(sliced_distances_kernel<kLanes, kChunks, 8>, 8 * kDistThreads, turned);
-    };
-    using std::integral_constant;
-    integral_constant<int, 16> lanes16;
-    integral_constant<int, 32> lanes32;
-    integral_constant<int, 64> lanes64;
-    const int perLane = chunks <= 64 ? (chunks + 15) / 16 : chunks <= 128 ? (chunks + 31) / 32 : (chunks + 63) / 64;
-    if (chunks <= 64) {
-        if (perLane == 2) launch_for(lanes16, integral_constant<int, 2>{});
-        if (perLane == 3) launch_for(lanes16, integral_constant<int, 3>{});
-        if (perLane == 4) launch_for(lanes16, integral_constant<int, 4>{});
-    } else if (chunks <= 128) {
-        if (perLane == 3) launch_for(lanes32, integral_constant<int, 3>{});
-        if (perLane == 4) launch_for(lanes32, integral_constant<int, 4>{});
-    } else {
-        if (perLane == 3) launch_for(lanes64, integral_constant<int, 3>{});
-        if (perLane == 4) launch_for(lanes64, integral_constant<int, 4>{});
-        if (perLane == 5) launch_for(lanes64, integral_constant<int, 5>{});
-        if (perLane == 6) launch_for(lanes64, integral_constant<int, 6>{});
-        if (perLane == 7) launch_for(lanes64, integral_constant<int, 7>{});
-        if (perLane == 8) launch_for(lanes64, integral_constant<int, 8>{});
-    }
-    return hipGetLastError();
 }
 
 }  // namespace fasted

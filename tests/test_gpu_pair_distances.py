@@ -132,3 +132,76 @@ def test_sliced_distances_of_subnormal_large_and_infinite_coordinates():
         bound = 1e-7 + 0.5 * (d / 16 + 20) * 2.0**-24
         assert bool(((mine[fine] - want[fine]).abs() <= bound * want[fine]).all())
     assert bool(torch.isinf(got[7 * 16 + 8])) and bool(torch.isnan(got[7 * 16 + 9])) and bool(torch.isnan(got[10 * 16 + 10]))
+
+
+# the kernel that goes through the list in its order: every row length class (1 to 6 chunks for each of 8, 4 to 6 for 16 and 32
+# lanes), fewer pairs than lanes, one, two and four pairs to a group, one past a full batch, pairs that name no point, and
+# queries that change at every place of a group's run
+@pytest.mark.parametrize("n,d", [(700, 1), (900, 65), (800, 190), (700, 256), (600, 300), (500, 384), (400, 385), (400, 640), (300, 768),
+                                 (300, 769), (300, 1280), (300, 1535), (200, 1537)])
+@pytest.mark.parametrize("count", [1, 7, 129, 4099, 140001, 300001])
+def test_listed_distances_match_fp64(n, d, count):
+    import torch
+
+    import fasted_amd as fasted
+
+    gen = torch.Generator(device="cuda").manual_seed(n + d + count)
+    ld = (d + 63) // 64 * 64 + 8
+    pts = torch.zeros((n, ld), dtype=torch.float16, device="cuda")
+    pts[:, :d] = torch.randn((n, d), generator=gen, device="cuda").to(torch.float16)
+    other = torch.zeros((n + 3, ld + 56), dtype=torch.float16, device="cuda")
+    other[:, :d] = torch.randn((n + 3, d), generator=gen, device="cuda").to(torch.float16)
+    q = torch.sort(torch.randint(0, n, (count,), generator=gen, device="cuda")).values
+    c = torch.randint(0, n + 3, (count,), generator=gen, device="cuda")
+    pairs = torch.stack([q, c], 1).to(torch.int32)
+    pairs[-1] = torch.tensor([n - 1, n + 2])
+    if count > 5:
+        pairs[torch.tensor([0, 2, count // 2], device="cuda")] = torch.tensor([[-1, 0], [n, 0], [0, n + 3]], dtype=torch.int32, device="cuda")
+    got = torch.full((count + 1,), -2.0, dtype=torch.float32, device="cuda")
+    fasted.pair_distances_device(pts.data_ptr(), n, ld, other.data_ptr(), n + 3, ld + 56, d, pairs.data_ptr(), count, got.data_ptr())
+    assert float(got[-1]) == -2.0
+    i = pairs.long()
+    ok = (i >= 0).all(1) & (i[:, 0] < n) & (i[:, 1] < n + 3)
+    assert bool(torch.isnan(got[:-1][~ok]).all())
+    i, mine = i[ok], got[:-1][ok].double()
+    step = max(1, (1 << 26) // d)
+    for r in range(0, len(i), step):
+        j = i[r : r + step]
+        want = (pts[j[:, 0], :d].double() - other[j[:, 1], :d].double()).norm(dim=1)
+        bound = 1e-7 + 0.5 * (ld / 8 + 20) * 2.0**-24  # as above, with 8 lanes to a row
+        assert bool(((mine[r : r + step] - want).abs() <= bound * want).all())
+
+
+# the smallest sets and lists that go through the slices: every row length class (2 to 6 chunks for each of 8 lanes, 4 to 6 for
+# 16 and 32, 4 to 8 for 64), with and without lanes that have no last chunk; an unordered piece of the list, invalid pairs
+@pytest.mark.parametrize("d", [128, 190, 256, 320, 384, 450, 576, 640, 768, 1000, 1088, 1280, 1536, 1600, 2048, 2112, 2560, 3072, 3136,
+                               3584, 4096])
+def test_smallest_sliced_lists_match_fp64(d):
+    import torch
+
+    import fasted_amd as fasted
+
+    gen = torch.Generator(device="cuda").manual_seed(d)
+    ld = (d + 63) // 64 * 64
+    n = (8 << 20) // (2 * ld) + 1
+    count = max(24 * n, 96 * 1024 - 1023) + 5
+    pts = torch.zeros((n, ld), dtype=torch.float16, device="cuda")
+    pts[:, :d] = torch.randn((n, d), generator=gen, device="cuda").to(torch.float16)
+    pairs = torch.randint(0, n, (count, 2), generator=gen, device="cuda", dtype=torch.int32)
+    pairs = pairs[torch.argsort(pairs[:, 0].long() * n + pairs[:, 1])]
+    pairs[1000:5000] = pairs[1000:5000][torch.randperm(4000, generator=gen, device="cuda")]
+    pairs[-1] = torch.tensor([n - 1, n - 1])
+    bad = torch.tensor([0, 1023, count - 2], device="cuda")
+    pairs[bad] = torch.tensor([[-1, 0], [0, n], [n, -1]], dtype=torch.int32, device="cuda")
+    got = torch.full((count + 1,), -2.0, dtype=torch.float32, device="cuda")
+    fasted.pair_distances_device(pts.data_ptr(), n, ld, pts.data_ptr(), n, ld, d, pairs.data_ptr(), count, got.data_ptr())
+    assert float(got[-1]) == -2.0
+    assert torch.isnan(got[bad]).all()
+    step = (1 << 26) // d
+    for r in range(0, count, step):
+        i = pairs[r : r + step].long()
+        ok = (i >= 0).all(1) & (i < n).all(1)
+        i = i[ok]
+        want = (pts[i[:, 0]].double() - pts[i[:, 1]].double()).norm(dim=1)
+        bound = 1e-7 + 0.5 * (ld / 8 + 20) * 2.0**-24  # as above, with 8 lanes to a row
+        assert bool(((got[r : r + step][: len(ok)][ok].double() - want).abs() <= bound * want).all())
