@@ -292,6 +292,7 @@ void join_on_device(PointSet q, PointSet c, bool selfJoin, int d, double epsilon
         jl.triangle = fasted::Triangle::kUpper;
     else if (selfJoin && !(flags & (FASTED_FULL_MATRIX | FASTED_NO_EPILOGUE)))
         jl.triangle = fasted::Triangle::kAuto;
+    jl.d = d;
     jl.dPad = dPad;
     jl.halfQ = halfQ;
     jl.halfC = halfC;
@@ -610,6 +611,7 @@ void self_join_blocked(const uint16_t* points, long long n, int d, double epsilo
             jl.nC = (int)block_rows(j);
             jl.selfJoin = diagonal;
             jl.triangle = fasted::Triangle::kAuto;
+            jl.d = d;
             jl.dPad = dPad;
             jl.halfQ = halves + (size_t)i * rows;
             jl.halfC = halves + (size_t)j * rows;

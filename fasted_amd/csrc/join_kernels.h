@@ -27,6 +27,7 @@ struct JoinLaunch {
     int forcedStride = 0;        // two sets where query i IS candidate i * forcedStride (a sample of the
                                  // candidates joined against all of them): that pair always counts
     Triangle triangle = Triangle::kFull;  // self-join: which part of the distance matrix is computed
+    int d;                       // dimensions; the columns d .. dPad-1 of every row are zeros
     int dPad;                    // K extent, multiple of kSlabK
     const float* halfQ;          // per query point: eps^2/4 - s/2 (s = squared norm), see launch_sum_squared
     const float* halfC;          // ... per candidate point

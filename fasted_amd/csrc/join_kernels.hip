@@ -313,10 +313,15 @@ __device__ __forceinline__ void static_for(F&& f) {
 // 80.9 -> 47.6, 20000 x 256 with 1000 705 -> 369, 100000 x 384 with 1000 3.65 -> 3.13 ms, 100000 x 128 with 64 1119 -> 1109 us.
 // A variant of its own because the full matrix became 1 - 2 % slower when the choice was made at run time (100000 x 128
 // 2.18 -> 2.21 ms).
-template <bool kEpilogue, bool kTall, int kTileRows, bool kOneSlab, bool kBitsInLastSlab = false, bool kMirror = false>
+// kHalfTail: no more than 32 dimensions reach into a tile's last slab, so its second k-step would multiply padding.  Join
+// kernel, with that k-step -> without: 100000 x 24 795 -> 696 us, 60000 x 80 428 -> 396, 60000 x 150 572 -> 542, 10007 x 250000
+// x 200 988 -> 938, 50000 x 544 1015 -> 986.
+template <bool kEpilogue, bool kTall, int kTileRows, bool kOneSlab, bool kBitsInLastSlab = false, bool kMirror = false,
+          bool kHalfTail = false>
 __global__ void __launch_bounds__(kThreads, 1) join_kernel(JoinParams p) {
     static_assert(!kMirror || (kEpilogue && kTileRows == 256), "pairs are mirrored across the diagonal of square tiles");
     const bool upperOnly = kEpilogue ? kMirror : p.symmetric != 0;
+    static_assert(!kHalfTail || kBitsInLastSlab, "only the last slab that gathers the hit bits leaves its second k-step out");
     static_assert(!kBitsInLastSlab || kEpilogue, "hit bits are gathered only when there is an epilogue");
     static_assert(kTileRows == 256 || kTileRows == 128, "tile rows");
     constexpr int kWaveRows = kTileRows / 2;    // rows of a wave's output sub-tile (2 x 4 waves)
@@ -660,9 +665,10 @@ __global__ void __launch_bounds__(kThreads, 1) join_kernel(JoinParams p) {
                 // a hit behind the k-loop, where nothing hides them.  Only the last row's 16 shifts are exposed.
                 // (Both k-steps visit the candidate blocks in ascending order, so that the blocks of a row become
                 // final in the order in which their bits are gathered.)
+                constexpr int kSteps = kHalfTail ? 1 : 2;  // (the order of an element's products stays: zeros are left out)
                 half8 a[2][2];
 #pragma unroll
-                for (int ks = 0; ks < 2; ++ks) {
+                for (int ks = 0; ks < kSteps; ++ks) {
                     a[0][ks] = fragment(buf + aOff[ks]);
 #pragma unroll
                     for (int fj = 0; fj < kFragCols; ++fj) b[ks][fj] = fragment(buf + bOff[ks] + fj * 16 * kRowBytes);
@@ -696,21 +702,21 @@ __global__ void __launch_bounds__(kThreads, 1) join_kernel(JoinParams p) {
                     __builtin_amdgcn_sched_barrier(0);
                     if constexpr (fi + 1 < kFragRows) {
                         a[(fi + 1) & 1][0] = fragment(buf + aOff[0] + (fi + 1) * 16 * kRowBytes);
-                        a[(fi + 1) & 1][1] = fragment(buf + aOff[1] + (fi + 1) * 16 * kRowBytes);
+                        if constexpr (kSteps == 2) a[(fi + 1) & 1][1] = fragment(buf + aOff[1] + (fi + 1) * 16 * kRowBytes);
                     }
 #pragma unroll
-                    for (int ks = 0; ks < 2; ++ks)
+                    for (int ks = 0; ks < kSteps; ++ks)
 #pragma unroll
                         for (int fj = 0; fj < kFragCols; ++fj)
                             acc[fi][fj] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[fi & 1][ks], b[ks][fj], acc[fi][fj], 0, 0, 0);
                     if constexpr (fi >= 1) {
                         gather_row(fi - 1);
                         // the order asked of the scheduler: the fragment reads, then MFMA, 2 shifts, MFMA, 2 shifts ...
-                        if constexpr (fi + 1 < kFragRows) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+                        if constexpr (fi + 1 < kFragRows) __builtin_amdgcn_sched_group_barrier(0x100, kSteps, 0);
 #pragma unroll
-                        for (int k = 0; k < 8; ++k) {
+                        for (int k = 0; k < 4 * kSteps; ++k) {
                             __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                            __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);
+                            __builtin_amdgcn_sched_group_barrier(0x002, 4 / kSteps, 0);
                         }
                     }
                 });
@@ -1160,7 +1166,7 @@ namespace {
 
 // One launch of the join kernel over the tile grid described by p.raster, in the queue or the direct mode, with
 // tiles of 256 or 128 query rows.
-hipError_t launch_join_grid(JoinParams p, bool rows128, bool tall, bool epilogue, int numCUs, hipStream_t stream) {
+hipError_t launch_join_grid(JoinParams p, bool rows128, bool tall, bool epilogue, bool halfTail, int numCUs, hipStream_t stream) {
     const unsigned long long realTiles = p.symmetric ? (unsigned long long)p.raster.tileRows * (p.raster.tileRows + 1) / 2
                                                      : (unsigned long long)p.raster.tileRows * p.raster.tileCols;
     // Up to two tiles per CU, workgroup b computes tile b and ends, one workgroup per tile (the hardware places
@@ -1173,7 +1179,20 @@ hipError_t launch_join_grid(JoinParams p, bool rows128, bool tall, bool epilogue
     // Tiles of up to 16 slabs gather their hit bits in their last slab; longer ones screen behind the k-loop.
     const bool bitsInLastSlab = epilogue && p.nSlabs <= 16;
     const int variant = (oneSlab ? 8 : 0) | (tall ? 2 : 0) | (rows128 ? 1 : 0);
-    if (epilogue && p.symmetric) {
+    // (128-row tiles run in one round of the workgroups, whose time is latency: 1000 x 30 is the same without the k-step)
+    if (bitsInLastSlab && halfTail && !rows128) {
+        const int halfVariant = (p.symmetric ? 4 : 0) | (oneSlab ? 2 : 0) | (tall ? 1 : 0);
+        switch (halfVariant) {
+            case 7: join_kernel<true, true, 256, true, true, true, true><<<g, b, 0, stream>>>(p); break;
+            case 6: join_kernel<true, false, 256, true, true, true, true><<<g, b, 0, stream>>>(p); break;
+            case 5: join_kernel<true, true, 256, false, true, true, true><<<g, b, 0, stream>>>(p); break;
+            case 4: join_kernel<true, false, 256, false, true, true, true><<<g, b, 0, stream>>>(p); break;
+            case 3: join_kernel<true, true, 256, true, true, false, true><<<g, b, 0, stream>>>(p); break;
+            case 2: join_kernel<true, false, 256, true, true, false, true><<<g, b, 0, stream>>>(p); break;
+            case 1: join_kernel<true, true, 256, false, true, false, true><<<g, b, 0, stream>>>(p); break;
+            default: join_kernel<true, false, 256, false, true, false, true><<<g, b, 0, stream>>>(p); break;
+        }
+    } else if (epilogue && p.symmetric) {
         const int mirrorVariant = (oneSlab ? 4 : bitsInLastSlab ? 2 : 0) | (tall ? 1 : 0);
         switch (mirrorVariant) {
             case 5: join_kernel<true, true, 256, true, true, true><<<g, b, 0, stream>>>(p); break;
@@ -1263,7 +1282,7 @@ hipError_t launch_join(const JoinLaunch& launch, hipStream_t stream) {
     p.symmetric = (mayMirror && !rows128) ? 1 : 0;
     const int tileRows = rows128 ? 128 : kTile;
     p.raster = make_raster(l.nQ, l.nC, p.symmetric != 0, tileRows);
-    return launch_join_grid(p, rows128, tall_order(l.nQ, tileRows), l.epilogue, numCUs, stream);
+    return launch_join_grid(p, rows128, tall_order(l.nQ, tileRows), l.epilogue, l.dPad - l.d >= kSlabK / 2, numCUs, stream);
 }
 
 }  // namespace fasted

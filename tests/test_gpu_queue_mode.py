@@ -146,3 +146,33 @@ def test_skip_sums_needs_the_buffers_and_gives_the_same_list(fasted):
     with pytest.raises(fp.FastedError):
         fasted.self_join_device(pts.data_ptr(), n, d, d, eps, pairs.data_ptr(), cap, sums_ptr=None,
                                 flags=fp.FASTED_SKIP_SUMS)
+
+
+@pytest.mark.parametrize("d", [1, 32, 33, 65, 96, 97, 160, 992, 993])
+@pytest.mark.parametrize("n", [2900, 7001, 16500])
+def test_last_slab_with_one_and_two_steps(fasted, n, d):
+    """Dimensions that reach 32 columns or more into a tile's last slab, and fewer: one workgroup per tile, the queues, the
+    tall order; the triangle, the full matrix and two sets.  Integer coordinates: every sum is exact, the lists are equal."""
+    import torch
+    from fasted_amd import find_pairs as fp
+
+    gen = torch.Generator(device="cuda").manual_seed(n + d)
+    ld, high = (d + 63) // 64 * 64, 2000 if d == 1 else 8 if d < 64 else 3
+    pts = torch.zeros((n, ld), dtype=torch.float16, device="cuda")
+    pts[:, :d] = torch.randint(0, high, (n, d), generator=gen, device="cuda").to(torch.float16)
+    x = pts.float()
+    sq = (x * x).sum(1)
+    d2 = torch.cat([sq[r : r + 2048, None] + sq[None, :] - 2.0 * (x[r : r + 2048] @ x.T) for r in range(0, n, 2048)])
+    eps2 = float(torch.kthvalue(d2[:256].flatten(), 256 * 12).values) + 0.5
+    want = torch.nonzero(d2 <= eps2).to(torch.int32)
+    m = n // 3
+    cap = len(want) + 64
+    pairs = torch.empty((cap, 2), dtype=torch.int32, device="cuda")
+    for flags in (0, fp.FASTED_FULL_MATRIX):
+        pairs.fill_(-1)
+        st = fasted.self_join_device(pts.data_ptr(), n, d, ld, eps2**0.5, pairs.data_ptr(), cap, flags=flags | fp.FASTED_SORT_PAIRS)
+        assert st.pairsFound == len(want) and torch.equal(pairs[: len(want)], want), flags
+    st = fasted.join_device(pts.data_ptr(), m, ld, pts[m:].data_ptr(), n - m, ld, d, eps2**0.5, pairs.data_ptr(), cap,
+                            flags=fp.FASTED_SORT_PAIRS)
+    two = want[(want[:, 0] < m) & (want[:, 1] >= m)] - torch.tensor([0, m], dtype=torch.int32, device="cuda")
+    assert st.pairsFound == len(two) and torch.equal(pairs[: len(two)], two)
