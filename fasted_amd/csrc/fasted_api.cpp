@@ -70,6 +70,27 @@ struct Workspace {
     unsigned long long* hostCount = nullptr;
     unsigned long long* hostCountDev = nullptr;  // the same words as the device addresses them
     double clockRate = 0.0;
+    // hit bits of joins of few points whose pairs are wanted in order (at most 31.5 MiB)
+    unsigned* bits = nullptr;
+    size_t bitsBytes = 0;
+
+    // null if there is no memory for them
+    unsigned* ensure_bits(size_t bytes) {
+        if (bytes > bitsBytes) {
+            if (bits) HIP_CHECK(hipFree(bits));
+            bits = nullptr;
+            bitsBytes = 0;
+            size_t room = (size_t)1 << 20;
+            while (room < bytes) room *= 2;
+            if (hipMalloc(&bits, room) != hipSuccess) {
+                (void)hipGetLastError();
+                bits = nullptr;
+                return nullptr;
+            }
+            bitsBytes = room;
+        }
+        return bits;
+    }
 
     // ticks per millisecond of the clock the kernels read (a constant-rate counter, independent of the shader clock)
     double clockKHz() {
@@ -113,6 +134,9 @@ struct Workspace {
         if (sums) (void)hipFree(sums);
         if (halves) (void)hipFree(halves);
         if (hostCount) (void)hipHostFree(hostCount);
+        if (bits) (void)hipFree(bits);
+        bits = nullptr;
+        bitsBytes = 0;
         for (auto& e : ev) {
             if (e) (void)hipEventDestroy(e);
             e = nullptr;
@@ -260,13 +284,18 @@ void join_on_device(PointSet q, PointSet c, bool selfJoin, int d, double epsilon
     // squared norms and, from them, each point's accumulator start value eps^2/4 - s/2
     // (the first of these launches also clears the pair counter and the queue heads)
     const unsigned long long epoch = ++g_epoch;
+    // Few points and pairs in order: the join leaves its hit bits, and one kernel behind it makes the list of them.
+    unsigned* const bits = (flags & FASTED_SORT_PAIRS) && !(flags & FASTED_NO_EPILOGUE) && cap > 0 && !fixed &&
+                                   q.n <= fasted::kMaxBitRows && c.n <= fasted::kMaxBitRows
+                               ? g_ws.ensure_bits(fasted::bits_bytes((int)q.n, (int)c.n))
+                               : nullptr;
     // Timing.  Three event records cost a call about 10 us, a third of a join of a few thousand points, so a
     // join of at most two tiles per compute unit is timed by the kernels themselves instead: the first norm
     // kernel and the join kernel note the device's constant-rate clock when they start, and the join kernel's
     // last workgroup when it hands the pair count to the host.  Larger joins, and the entry
     // that owns no pinned memory, are timed with events on the stream as the reference is
     // (source/findPairs.cuh:625-639,695-697,728-736).
-    const bool stamped = !fixed && !(flags & FASTED_EVENT_TIMING) && fasted::tile_count(q.n, c.n) <= 512;
+    const bool stamped = !fixed && !(flags & FASTED_EVENT_TIMING) && (bits || fasted::tile_count(q.n, c.n) <= 512);
     const bool events = !stamped && stats != nullptr;
     if (events) HIP_CHECK(hipEventRecord(t.ev[0], stream));
     if (!(flags & FASTED_SKIP_SUMS)) {
@@ -302,8 +331,11 @@ void join_on_device(PointSet q, PointSet c, bool selfJoin, int d, double epsilon
     jl.cap = cap;
     jl.epilogue = !(flags & FASTED_NO_EPILOGUE);
     if (!fixed) static_cast<volatile unsigned long long*>(g_ws.hostCount)[3] = 0;  // the kernel's report turns it non-zero
-    HIP_CHECK(fasted::launch_join(jl, stream));
+    jl.bits = bits;
+    fasted::BitsLayout layout;
+    HIP_CHECK(fasted::launch_join(jl, stream, &layout));
     if (events) HIP_CHECK(hipEventRecord(t.ev[2], stream));
+    if (bits) HIP_CHECK(fasted::launch_expand_bits(bits, layout, (int)q.n, (int)c.n, counters, dPairs, cap, stream));
     // c[0] = pairs found; every slot below the capacity received exactly one pair, the rest were
     // counted only (source/pair.cuh:123-133), so stored = min(found, capacity)
     unsigned long long cnt[4] = {0, 0, 0, 0};
@@ -318,7 +350,7 @@ void join_on_device(PointSet q, PointSet c, bool selfJoin, int d, double epsilon
         // reports, because it failed, falls through to the stream's own wait, which returns the error.)
         volatile unsigned long long* const w = g_ws.hostCount;
         bool reported = false;
-        if (stamped) {
+        if (stamped && !bits) {
             const auto t0 = std::chrono::steady_clock::now();
             for (unsigned spins = 1; !(reported = w[3] != 0); ++spins)
                 if ((spins & 1023u) == 0 && std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(2)) break;
@@ -340,7 +372,10 @@ void join_on_device(PointSet q, PointSet c, bool selfJoin, int d, double epsilon
         cnt[2] = side * (side + 1) / 2;
     }
     float sortMs = 0.f;
-    if ((flags & FASTED_SORT_PAIRS) && cnt[1] > 1) {
+    if (bits) {
+        const volatile unsigned long long* const w = g_ws.hostCount;  // [3] its kernel started, [4] and was through
+        if (w[3] != 0 && w[4] > w[3]) sortMs = (float)((double)(w[4] - w[3]) / g_ws.clockKHz());
+    } else if ((flags & FASTED_SORT_PAIRS) && cnt[1] > 1) {
         const auto w0 = std::chrono::steady_clock::now();
         const hipError_t e = fasted::sort_pairs_row_major(dPairs, cnt[1], stream, &g_sortWs, 0, q.n, c.n);
         if (e != hipSuccess) {

@@ -3,6 +3,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include "join_kernels.h"
 #include "tile_order.hpp"
 
 namespace fasted {
@@ -26,7 +27,9 @@ constexpr int kQueueBase = 16, kQueueStride = 16;
 // kernel through).  It sits here and not among the kernel's arguments because the tile loop has no scalar
 // registers to spare.
 constexpr int kCounterHostWords = kQueueBase + kQueues * kQueueStride;
-constexpr int kCounterWords = kCounterHostWords + 16;
+// Of a join that leaves hit bits: 32-bit words, hits of every band of 32 query rows (kMaxBands).
+constexpr int kCounterBands = kCounterHostWords + 16;
+constexpr int kCounterWords = kCounterBands + kMaxBands / 2;
 
 struct JoinParams {
     const u32x4* ptsQ;  // query rows
@@ -44,7 +47,26 @@ struct JoinParams {
     int2* pairs;
     unsigned long long cap;
     TileOrder raster;
+    unsigned* bits;  // hit bits instead of pairs: see the join kernel's kBits
 };
+
+// v plus what a DPP move brings (0 where it brings nothing): inclusive sums over the lanes of a wave in the vector unit.
+template <int kControl, int kRows = 0xf>
+__device__ __forceinline__ unsigned add_moved(unsigned v) {
+    return v + (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, kControl, kRows, 0xf, false);
+}
+__device__ __forceinline__ unsigned wave_inclusive_scan(unsigned v) {
+    v = add_moved<0x111>(v);       // row_shr:1, then 2, 4, 8: sums inside the rows of 16 lanes
+    v = add_moved<0x112>(v);
+    v = add_moved<0x114>(v);
+    v = add_moved<0x118>(v);
+    v = add_moved<0x142, 0xa>(v);  // row_bcast:15 into rows 1 and 3
+    return add_moved<0x143, 0xc>(v);  // row_bcast:31 into rows 2 and 3
+}
+// Sum over the wave's 64 lanes, uniform.
+__device__ __forceinline__ unsigned wave_sum(unsigned v) {
+    return (unsigned)__builtin_amdgcn_readlane((int)wave_inclusive_scan(v), 63);
+}
 
 // Lane number 0..63, re-derived from the execution mask where it is needed.  Volatile on purpose: the
 // optimiser then cannot hoist it (and what is derived from it) out of the tile loop, where it would

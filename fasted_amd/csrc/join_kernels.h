@@ -18,6 +18,20 @@ enum class Triangle {
     kAuto    // whichever is the faster one at this size (launch_join)
 };
 
+// Hit bits: what a join of few points leaves instead of pairs, one bit per element of the distance matrix, for
+// launch_expand_bits to make the row-major pair list from.  Tile (row, col) of tileRows x 256 elements fills the
+// words [(row * tileCols + col) * 8 * tileWords, ...): per wave (2 x 4 of them, sub-tiles of tileRows / 2 x 64) tileWords
+// of 64 lanes, word p of lane l at p * 64 + l, as the matrix instruction leaves its elements: bit 31 - e of it is
+// row p * 32 + (e >> 4) * 16 + (l >> 4) * 4 + e % 4, column (e >> 2) % 4 * 16 + l % 16 of the sub-tile.
+struct BitsLayout {
+    int tileRows = 0;     // 256, or 128
+    unsigned rowsOfTiles = 0, tileCols = 0;
+    bool upper = false;   // tiles on and above the diagonal only
+};
+constexpr int kMaxBitRows = 63 * kTile;            // points of either set of a join that leaves hit bits
+constexpr int kBandRows = 32, kMaxBands = 512;     // query rows are counted, and expanded, in bands
+static_assert(kMaxBitRows / kBandRows <= kMaxBands, "a counter per band");
+
 struct JoinLaunch {
     const void* queries;         // FP16 rows
     const void* candidates;      // FP16 rows; the same buffer for a self-join
@@ -43,7 +57,17 @@ struct JoinLaunch {
     void* pairs;                 // FastedPair[cap]
     unsigned long long cap;
     bool epilogue;               // false: contraction only (measurement)
+    unsigned* bits = nullptr;    // hit bits are left here (bits_bytes(nQ, nC); neither set above kMaxBitRows points) and
+                                 // the bands counted in the counter block; no pairs, no count, no report
 };
+
+// Device bytes of the hit bits of a join, in either tile height.
+size_t bits_bytes(int nQ, int nC);
+// The row-major list out of the hit bits that a launch_join has left: pairs[0, min(found, cap)).  Reports through the
+// counter block's host words: [0] pairs found, [1] clock when the first norm kernel started, [3] (never 0) when this kernel
+// did, [4] when its last band was through.
+hipError_t launch_expand_bits(const unsigned* bits, const BitsLayout& layout, int nQ, int nC, unsigned long long* counters,
+                              void* pairs, unsigned long long cap, hipStream_t stream);
 
 // Host mirror of the device tile order.
 // upperOnly: the order of a symmetric self-join (super-squares on and above the diagonal only).
@@ -80,7 +104,8 @@ hipError_t launch_offset_pairs(void* pairs, unsigned long long first, unsigned l
 // the counter in mark[1].  No host round trip: the range is read on the device.
 hipError_t launch_offset_appended_pairs(void* pairs, unsigned long long* mark, const unsigned long long* counters,
                                         unsigned long long cap, int qOffset, int cOffset, hipStream_t stream);
-hipError_t launch_join(const JoinLaunch& p, hipStream_t stream);
+// `layout` (may be null): how the hit bits lie.
+hipError_t launch_join(const JoinLaunch& p, hipStream_t stream, BitsLayout* layout = nullptr);
 // "" for the library proper; a measurement build of the join kernel (parts compiled out) names itself here.
 const char* build_tag();
 

@@ -134,9 +134,9 @@ inline void raster_decode(const Raster& r, bool tall, unsigned q, unsigned long 
 // counter and the queue heads for the join kernel that follows in the stream: no launch of its own for that.
 __device__ __forceinline__ void reset_for_join(unsigned long long* __restrict__ counters) {
     if (blockIdx.x != 0) return;
-    const int t = threadIdx.x;
-    if (t == 0) counters[kCounterStampNorms] = wall_clock64();  // the timed region of a small join starts here
-    if (t < kCounterWords && t != kCounterNonFinite && t != kCounterStampNorms && t != kCounterHostWords) counters[t] = 0ull;
+    if (threadIdx.x == 0) counters[kCounterStampNorms] = wall_clock64();  // the timed region of a small join starts here
+    for (int t = threadIdx.x; t < kCounterWords; t += blockDim.x)
+        if (t != kCounterNonFinite && t != kCounterStampNorms && t != kCounterHostWords) counters[t] = 0ull;
 }
 
 __global__ void __launch_bounds__(256) sum_squared_kernel(const u32x4* __restrict__ pts, long long ld16, int n,
@@ -238,9 +238,8 @@ __global__ void __launch_bounds__(256) pad_rows_kernel(const unsigned short* __r
 // of the join that raised it.  (A join that computes its norms first needs no launch of this: the norm kernel's
 // first workgroup does the clearing.)
 __global__ void reset_counters_kernel(unsigned long long* c, int keepFound) {
-    if (threadIdx.x < kCounterWords && threadIdx.x != kCounterNonFinite && threadIdx.x != kCounterHostWords &&
-        !(keepFound && threadIdx.x == kCounterFound))
-        c[threadIdx.x] = 0ull;
+    for (int t = threadIdx.x; t < kCounterWords; t += blockDim.x)
+        if (t != kCounterNonFinite && t != kCounterHostWords && !(keepFound && t == kCounterFound)) c[t] = 0ull;
 }
 
 // Adds the first row of the query block and of the candidate block to the pairs [first, last) that a
@@ -275,6 +274,12 @@ __global__ void __launch_bounds__(256) offset_appended_pairs_kernel(int2* pairs,
     }
 }
 
+// base[at + kOffset], in bytes, = v: one store instruction, whatever the compiler knows about outstanding operations.
+template <int kOffset>
+__device__ __forceinline__ void store_word(unsigned* base, unsigned at, unsigned v) {
+    asm volatile("global_store_dword %0, %1, %2 offset:%3" ::"v"(at), "v"(v), "s"(base), "n"(kOffset) : "memory");
+}
+
 // ------------------------------------------------------------------------------------------
 // The barrier of the tile loop: every global->LDS transfer this wave has issued has landed (they are vector
 // memory operations: vmcnt), every LDS operation of the wave is complete, then the workgroup meets.  The wait
@@ -285,6 +290,15 @@ __global__ void __launch_bounds__(256) offset_appended_pairs_kernel(int2* pairs,
 // MFMA).
 __device__ __forceinline__ void transfers_landed_barrier() {
     __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0) lgkmcnt(0), export counter left alone
+    __syncthreads();
+}
+
+// The same where exactly kYounger vector memory operations were issued since the last transfer: they need not be complete
+// (the counter goes down in the order of issue).
+template <int kYounger>
+__device__ __forceinline__ void transfers_landed_barrier_behind() {
+    static_assert(kYounger < 16, "the low field of the counter");
+    __builtin_amdgcn_s_waitcnt(0x0070 | kYounger);
     __syncthreads();
 }
 
@@ -316,11 +330,15 @@ __device__ __forceinline__ void static_for(F&& f) {
 // kHalfTail: no more than 32 dimensions reach into a tile's last slab, so its second k-step would multiply padding.  Join
 // kernel, with that k-step -> without: 100000 x 24 795 -> 696 us, 60000 x 80 428 -> 396, 60000 x 150 572 -> 542, 10007 x 250000
 // x 200 988 -> 938, 50000 x 544 1015 -> 986.
+// kBits: a join of few points whose pairs are wanted in order.  The hit bits themselves leave (BitsLayout), the hits of
+// every band of 32 query rows are counted, and launch_expand_bits makes the list: no staging, no reservations, no records
+// that have to be sorted, and no count that the host waits for in between.
 template <bool kEpilogue, bool kTall, int kTileRows, bool kOneSlab, bool kBitsInLastSlab = false, bool kMirror = false,
-          bool kHalfTail = false>
+          bool kHalfTail = false, bool kBits = false>
 __global__ void __launch_bounds__(kThreads, 1) join_kernel(JoinParams p) {
     static_assert(!kMirror || (kEpilogue && kTileRows == 256), "pairs are mirrored across the diagonal of square tiles");
     const bool upperOnly = kEpilogue ? kMirror : p.symmetric != 0;
+    static_assert(!kBits || kEpilogue, "hit bits come from the epilogue");
     static_assert(!kHalfTail || kBitsInLastSlab, "only the last slab that gathers the hit bits leaves its second k-step out");
     static_assert(!kBitsInLastSlab || kEpilogue, "hit bits are gathered only when there is an epilogue");
     static_assert(kTileRows == 256 || kTileRows == 128, "tile rows");
@@ -374,6 +392,7 @@ __global__ void __launch_bounds__(kThreads, 1) join_kernel(JoinParams p) {
     // pair counter are over by then as well -- their old values have come back and been used -- so the last to
     // sign off reads the final count.
     auto sign_off = [&]() {
+        if (kBits) return;  // (launch_expand_bits reports)
         unsigned long long* const hostWords = host_words();
         if (!hostWords) return;
         __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
@@ -410,6 +429,22 @@ __global__ void __launch_bounds__(kThreads, 1) join_kernel(JoinParams p) {
         int hops = 0;
         *row = kNoTile;
         *col = 0u;
+        if constexpr (kBits) {
+            // strips without padding tiles, 32 tiles to a queue in turn (of 39 x 39 tiles the super-squares hold 1536 places
+            // for the 780 above the diagonal, and a place that is skipped costs the latency of a reservation)
+            const unsigned total = upperOnly ? ras.tileRows * (ras.tileRows + 1) / 2 : ras.tileRows * ras.tileCols;
+            for (;;) {
+                const unsigned long long number = pos / kSubTiles * (kQueues * kSubTiles) + q * kSubTiles + pos % kSubTiles;
+                if (number < total) {
+                    tile_strip_decode((unsigned)number, ras.tileRows, ras.tileCols, upperOnly, row, col);
+                    home = q;
+                    return;
+                }
+                if (++hops == kQueues) return;
+                q = (q + 1) & (kQueues - 1);
+                pos = atomicAdd(&p.counters[kQueueBase + q * kQueueStride], 1ull);
+            }
+        }
         for (;;) {
             if (pos < ras.perQueue) {
                 unsigned tr, tc;
@@ -588,12 +623,20 @@ __global__ void __launch_bounds__(kThreads, 1) join_kernel(JoinParams p) {
     unsigned long long popped = 0;  // thread 0: the home queue position reserved for the tile after the next one to be decoded
     if (wave == 0 && lane_now() == 0 && !p.direct) popped = atomicAdd(&p.counters[kQueueBase + home * kQueueStride], 1ull);
 
+    // With kBits, what was reserved during the tile before, taken over where every operation is known to be complete: the
+    // barrier at the top of a tile lets the bits of the tile before it be on their way, and the compiler would wait for them.
+    constexpr bool kTakeOver = kBits && !kOneSlab;
+    unsigned long long reserved = popped;
+
     int stage = 0;  // LDS stage that holds slab 0 of the current tile
     int sumsBuf = 0;
 
-    for (;;) {
+    for (bool again = false;; again = true) {
         // slab 0 of this tile (issued during the previous tile's last slab) has landed
-        transfers_landed_barrier();
+        if (kBits && again)
+            transfers_landed_barrier_behind<kFragRows / 2 + 1>();  // (not the bits and counts that left since)
+        else
+            transfers_landed_barrier();
         if (wave == 0 && lane_now() == 0) {
             // the reservation made a whole tile ago has long arrived: no wait here
             unsigned r, c;
@@ -601,7 +644,7 @@ __global__ void __launch_bounds__(kThreads, 1) join_kernel(JoinParams p) {
                 r = kNoTile;
                 c = 0u;
             } else {
-                find_tile(popped, &r, &c);
+                find_tile(kTakeOver ? reserved : popped, &r, &c);
                 popped = atomicAdd(&p.counters[kQueueBase + home * kQueueStride], 1ull);
             }
             const int slot = kOneSlab ? 2 * sumsBuf : 0;  // (sumsBuf is the tile count's parity)
@@ -837,6 +880,7 @@ __global__ void __launch_bounds__(kThreads, 1) join_kernel(JoinParams p) {
             slab_step(kFirstSlab, stage, true, gA + kRowBytes, gB + kRowBytes, offA, offB);
             stage ^= 1;
             transfers_landed_barrier();
+            if (kTakeOver) reserved = popped;
         }
         for (int s = 1; s + 1 < p.nSlabs; ++s) {
             slab_step(kLaterSlab, stage, true, gA + (s + 1) * kRowBytes, gB + (s + 1) * kRowBytes, offA, offB);
@@ -960,7 +1004,43 @@ __global__ void __launch_bounds__(kThreads, 1) join_kernel(JoinParams p) {
                     hits[fp] = m;
                 }
             }
-            if (kNoExtract) {
+            if constexpr (kBits) {
+                constexpr int kWords = kFragRows / 2;
+                if (!kFusedBits && !any) {
+#pragma unroll
+                    for (int fp = 0; fp < kWords; ++fp) hits[fp] = 0u;
+                }
+                const unsigned tile = tr * p.raster.tileCols + tc;
+                const unsigned at = ((tile * (kThreads / 64) + (unsigned)wave) * kWords * 64 + (unsigned)ln) * 4u;
+                // Two counts to a word: hits of the sub-tile's bands of 32 rows and, where the tile also stands for its mirror
+                // image, of its two bands of 32 columns.
+                constexpr int kSums = kWords / 2 + (kMirror ? 1 : 0);
+                unsigned sum[3] = {0u, 0u, 0u};
+#pragma unroll
+                for (int fp = 0; fp < kWords; ++fp) {
+                    sum[fp >> 1] += (unsigned)__builtin_popcount(hits[fp]) << (16 * (fp & 1));
+                    if (kMirror)
+                        sum[kWords / 2] += (unsigned)__builtin_popcount(hits[fp] & 0xff00ff00u) |
+                                           (unsigned)__builtin_popcount(hits[fp] & 0x00ff00ffu) << 16;
+                }
+                unsigned mine = 0u;
+#pragma unroll
+                for (int i = 0; i < kSums; ++i) {
+                    const unsigned all = wave_sum(sum[i]);
+                    if ((ln >> 1) == i) mine = all >> (16 * (ln & 1)) & 0xffffu;
+                }
+                const bool columns = kMirror && ln >= kWords;
+                if (columns && !mirror) mine = 0u;
+                const unsigned band = columns ? tc * (kTile / kBandRows) + (unsigned)wc * 2 + (unsigned)(ln & 1)
+                                              : tr * (kTileRows / kBandRows) + (unsigned)wr * kWords + (unsigned)ln;
+                unsigned* const bands = reinterpret_cast<unsigned*>(p.counters + kCounterBands);
+                // Written as instructions, kWords + 1 of them: the barrier at the top of the next tile counts them.
+                static_for<0, kWords>([&](auto fpc) {
+                    constexpr int fp = decltype(fpc)::value;
+                    store_word<fp * 256>(p.bits, at, hits[fp]);
+                });
+                if (ln < 2 * kSums) asm volatile("global_atomic_add %0, %1, %2" ::"v"(band * 4u), "v"(mine), "s"(bands) : "memory");
+            } else if (kNoExtract) {
                 if (any && !kNoHits) {
 #pragma unroll
                     for (int fp = 0; fp < kFragRows / 2; ++fp) asm volatile("" ::"v"(hits[fp]));
@@ -1030,7 +1110,7 @@ __global__ void __launch_bounds__(kThreads, 1) join_kernel(JoinParams p) {
         tc = ntc;
         sumsBuf ^= 1;
     }
-    if (kEpilogue) {
+    if constexpr (kEpilogue && !kBits) {
         // What is left in the eight regions goes out with one reservation for the workgroup: every workgroup
         // ends at about the same time, and one atomic per wave, all on one address, would serialise for
         // longer than a small join takes.  No transfer is in flight any more, so ordinary LDS accesses do.
@@ -1176,6 +1256,26 @@ hipError_t launch_join_grid(JoinParams p, bool rows128, bool tall, bool epilogue
     if (grid == 0) grid = 1;
     const dim3 g(grid), b(kThreads);
     const bool oneSlab = p.nSlabs == 1;
+    if (p.bits) {
+        const int k = oneSlab ? 2 : p.nSlabs <= 16 ? 1 : 0;  // the hit bits behind the k-loop, in the last of several slabs, in the only one
+        const int bitsVariant = rows128 ? k : (p.symmetric ? 16 : 8) + (halfTail && k != 0 ? 4 : 0) + k;
+        switch (bitsVariant) {
+            case 0: join_kernel<true, false, 128, false, false, false, false, true><<<g, b, 0, stream>>>(p); break;
+            case 1: join_kernel<true, false, 128, false, true, false, false, true><<<g, b, 0, stream>>>(p); break;
+            case 2: join_kernel<true, false, 128, true, true, false, false, true><<<g, b, 0, stream>>>(p); break;
+            case 8: join_kernel<true, false, 256, false, false, false, false, true><<<g, b, 0, stream>>>(p); break;
+            case 9: join_kernel<true, false, 256, false, true, false, false, true><<<g, b, 0, stream>>>(p); break;
+            case 10: join_kernel<true, false, 256, true, true, false, false, true><<<g, b, 0, stream>>>(p); break;
+            case 13: join_kernel<true, false, 256, false, true, false, true, true><<<g, b, 0, stream>>>(p); break;
+            case 14: join_kernel<true, false, 256, true, true, false, true, true><<<g, b, 0, stream>>>(p); break;
+            case 16: join_kernel<true, false, 256, false, false, true, false, true><<<g, b, 0, stream>>>(p); break;
+            case 17: join_kernel<true, false, 256, false, true, true, false, true><<<g, b, 0, stream>>>(p); break;
+            case 18: join_kernel<true, false, 256, true, true, true, false, true><<<g, b, 0, stream>>>(p); break;
+            case 21: join_kernel<true, false, 256, false, true, true, true, true><<<g, b, 0, stream>>>(p); break;
+            default: join_kernel<true, false, 256, true, true, true, true, true><<<g, b, 0, stream>>>(p); break;
+        }
+        return hipGetLastError();
+    }
     // Tiles of up to 16 slabs gather their hit bits in their last slab; longer ones screen behind the k-loop.
     const bool bitsInLastSlab = epilogue && p.nSlabs <= 16;
     const int variant = (oneSlab ? 8 : 0) | (tall ? 2 : 0) | (rows128 ? 1 : 0);
@@ -1237,7 +1337,12 @@ hipError_t launch_join_grid(JoinParams p, bool rows128, bool tall, bool epilogue
 
 }  // namespace
 
-hipError_t launch_join(const JoinLaunch& launch, hipStream_t stream) {
+size_t bits_bytes(int nQ, int nC) {
+    // (in tiles of 128 rows as many bytes, or half a tile row less)
+    return (size_t)((nQ + kTile - 1) / kTile) * (size_t)((nC + kTile - 1) / kTile) * (kTile * kTile / 8);
+}
+
+hipError_t launch_join(const JoinLaunch& launch, hipStream_t stream, BitsLayout* layout) {
     // (the compute units of the current device, looked up at every launch: the device may change between calls)
     int dev = 0, numCUs = 0;
     hipError_t e = hipGetDevice(&dev);
@@ -1282,6 +1387,8 @@ hipError_t launch_join(const JoinLaunch& launch, hipStream_t stream) {
     p.symmetric = (mayMirror && !rows128) ? 1 : 0;
     const int tileRows = rows128 ? 128 : kTile;
     p.raster = make_raster(l.nQ, l.nC, p.symmetric != 0, tileRows);
+    p.bits = l.bits;
+    if (layout) *layout = BitsLayout{tileRows, p.raster.tileRows, p.raster.tileCols, p.symmetric != 0};
     return launch_join_grid(p, rows128, tall_order(l.nQ, tileRows), l.epilogue, l.dPad - l.d >= kSlabK / 2, numCUs, stream);
 }
 

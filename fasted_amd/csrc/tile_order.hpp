@@ -98,6 +98,35 @@ FASTED_HD inline void tile_order_upper_decode(unsigned b, unsigned* tr, unsigned
     *tr = b - c * (c + 1) / 2;
 }
 
+// Tile `number` of a matrix of rows x cols tiles taken in strips of four columns, row by row in a strip: 32 consecutive
+// numbers are 8 x 4 tiles.  upper: of its upper triangle (rows == cols), diagonal included.  Every number below
+// rows * cols, or rows * (rows + 1) / 2, is a tile: no padding, whatever the shape.
+FASTED_HD inline void tile_strip_decode(unsigned number, unsigned rows, unsigned cols, bool upper, unsigned* tr, unsigned* tc) {
+    if (upper) {
+        // strips 0 .. j - 1 hold 8 j^2 + 2 j tiles; the root is an estimate, then corrected
+        unsigned j = (unsigned)((__builtin_sqrtf(8.0f * (float)number + 1.0f) - 1.0f) * 0.125f);
+        while (j > 0 && 8 * j * j + 2 * j > number) --j;
+        while (8 * (j + 1) * (j + 1) + 2 * (j + 1) <= number) ++j;
+        const unsigned first = 4 * j, width = cols - first < 4 ? cols - first : 4;
+        unsigned s = number - (8 * j * j + 2 * j);
+        if (s < first * width) {
+            *tr = s / width;
+            *tc = first + s % width;
+        } else {
+            s -= first * width;
+            unsigned i = 0;  // rows first + i of the strip start at the diagonal
+            for (; s >= width - i; ++i) s -= width - i;
+            *tr = first + i;
+            *tc = first + i + s;
+        }
+    } else {
+        const unsigned strip = number / (4 * rows), s = number % (4 * rows);
+        const unsigned width = cols - 4 * strip < 4 ? cols - 4 * strip : 4;
+        *tr = s / width;
+        *tc = 4 * strip + s % width;
+    }
+}
+
 // LDS placement of operand rows.  gfx950 serves a ds_read_b128 in four phases of 16 lanes --
 // {0-3,12-15,20-23,24-27}, {4-7,8-11,16-19,28-31} and the same two groups +32 -- and the fragment read
 // of v_mfma_f32_16x16x32_f16 has lane l on row l%16, 16-byte chunk l/16 of a 32-wide k-step.  A phase is

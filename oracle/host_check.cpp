@@ -165,6 +165,20 @@ static void check_tile_order() {
                 CHECK(tr == r && tc == c);
             }
     }
+    // strips of four columns: every tile of a matrix, or of its upper triangle, exactly once
+    for (unsigned rows = 1; rows <= 70; ++rows)
+        for (unsigned cols = 1; cols <= 70; ++cols)
+            for (int upper = 0; upper <= (rows == cols ? 1 : 0); ++upper) {
+                std::set<std::pair<unsigned, unsigned>> seen;
+                const unsigned total = upper ? rows * (rows + 1) / 2 : rows * cols;
+                for (unsigned i = 0; i < total; ++i) {
+                    unsigned r = 0, c = 0;
+                    fasted::tile_strip_decode(i, rows, cols, upper != 0, &r, &c);
+                    CHECK(r < rows && c < cols && (!upper || r <= c));
+                    seen.insert({r, c});
+                }
+                CHECK(seen.size() == total);
+            }
     // LDS swizzles: the 16 lanes of every ds_read_b128 phase touch all 64 banks once
     const int groups[2][16] = {{0, 1, 2, 3, 12, 13, 14, 15, 20, 21, 22, 23, 24, 25, 26, 27},
                                {4, 5, 6, 7, 8, 9, 10, 11, 16, 17, 18, 19, 28, 29, 30, 31}};
