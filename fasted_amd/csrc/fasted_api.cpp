@@ -112,7 +112,7 @@ struct Workspace {
         if (!counters) {
             // all zero (the non-finite flag is compared with join numbers, which start at 1), except for the word
             // that tells the join kernel where to report the pair count and its clock readings
-            const size_t bytes = fasted::counter_words() * sizeof(unsigned long long);
+            const size_t bytes = (fasted::counter_words() + fasted::band_words()) * sizeof(unsigned long long);
             HIP_CHECK(hipMalloc(&counters, bytes));
             HIP_CHECK(hipMemset(counters, 0, bytes));
             HIP_CHECK(hipMemcpy(counters + fasted::host_words_slot(), &hostCountDev, sizeof hostCountDev, hipMemcpyHostToDevice));
@@ -297,13 +297,14 @@ void join_on_device(PointSet q, PointSet c, bool selfJoin, int d, double epsilon
     // (source/findPairs.cuh:625-639,695-697,728-736).
     const bool stamped = !fixed && !(flags & FASTED_EVENT_TIMING) && (bits || fasted::tile_count(q.n, c.n) <= 512);
     const bool events = !stamped && stats != nullptr;
+    const fasted::Reset reset = bits ? fasted::Reset::kCountersAndBands : fasted::Reset::kCounters;
     if (events) HIP_CHECK(hipEventRecord(t.ev[0], stream));
     if (!(flags & FASTED_SKIP_SUMS)) {
-        HIP_CHECK(fasted::launch_sum_squared(q.ptr, q.ld, (int)q.n, dPad, sumsQ, halfQ, eps2, counters, stream, epoch, true));
+        HIP_CHECK(fasted::launch_sum_squared(q.ptr, q.ld, (int)q.n, dPad, sumsQ, halfQ, eps2, counters, stream, epoch, reset));
         if (!selfJoin)
             HIP_CHECK(fasted::launch_sum_squared(c.ptr, c.ld, (int)c.n, dPad, sumsC, halfC, eps2, counters, stream, epoch));
     } else {
-        HIP_CHECK(fasted::launch_halves(sumsQ, (int)q.n, eps2, halfQ, counters, stream, epoch, true));
+        HIP_CHECK(fasted::launch_halves(sumsQ, (int)q.n, eps2, halfQ, counters, stream, epoch, reset));
         if (!selfJoin) HIP_CHECK(fasted::launch_halves(sumsC, (int)c.n, eps2, halfC, counters, stream, epoch));
     }
     if (events) HIP_CHECK(hipEventRecord(t.ev[1], stream));

@@ -74,22 +74,24 @@ hipError_t launch_expand_bits(const unsigned* bits, const BitsLayout& layout, in
 unsigned long long raster_count(long long nQ, long long nC, bool upperOnly = false);
 int raster_coord(unsigned long long idx, long long nQ, long long nC, bool upperOnly, int* row, int* col);
 int counter_words();
+int band_words();  // behind them, for joins that leave hit bits
 int host_words_slot();
 unsigned long long tile_count(long long nQ, long long nC);  // 256x256 tiles the kernel processes
 // Slot (0..7) of 16-byte chunk `chunk` of slab row `row` in LDS (host mirror of the device swizzle).
 int lds_chunk_slot(int row, int chunk);
 
+enum class Reset { kNothing = 0, kCounters = 1, kCountersAndBands = 2 };
 // Squared norms of n points into `sums` (may be null) and, when `halves` is given, the per-point start value of
 // the join's accumulators  h = eps2/4 - s/2  (eps2 = (float)(eps*eps), source/findPairs.cuh:678): the join kernel
 // tests  h_q + h_c + q.c >= 0.  A non-finite norm raises the flag in `counters` (the join then tests element
 // by element): the flag word receives `epoch`.  With `reset` the kernel also clears the pair counter and the
-// queue heads for the join that follows (no launch_reset_counters needed).
+// queue heads, and the counts of the bands, for the join that follows (no launch_reset_counters needed).
 hipError_t launch_sum_squared(const void* points, long long ld, int n, int dPad, float* sums, float* halves, float eps2,
                               unsigned long long* counters, hipStream_t stream, unsigned long long epoch = 1,
-                              bool reset = false);
+                              Reset reset = Reset::kNothing);
 // The same halves from norms that are already there.
 hipError_t launch_halves(const float* sums, int n, float eps2, float* halves, unsigned long long* counters,
-                         hipStream_t stream, unsigned long long epoch = 1, bool reset = false);
+                         hipStream_t stream, unsigned long long epoch = 1, Reset reset = Reset::kNothing);
 // rows x d halves, packed -> rows x dPad halves, the columns d .. dPad-1 zero.  dst is 16-byte aligned, src 2-byte.
 hipError_t launch_pad_rows(const void* src, int d, void* dst, int dPad, long long rows, hipStream_t stream);
 // *badRows += number of rows whose columns d .. dPad-1 are not all zeros.

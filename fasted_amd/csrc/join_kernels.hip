@@ -132,8 +132,12 @@ inline void raster_decode(const Raster& r, bool tall, unsigned q, unsigned long 
 // word receives `epoch`, the number of the join this launch belongs to, so that it never has to be cleared
 // (clearing it in this kernel would race with raising it).  With `reset`, the first workgroup clears the pair
 // counter and the queue heads for the join kernel that follows in the stream: no launch of its own for that.
-__device__ __forceinline__ void reset_for_join(unsigned long long* __restrict__ counters) {
+__device__ __forceinline__ void reset_for_join(unsigned long long* __restrict__ counters, int reset) {
     if (blockIdx.x != 0) return;
+    if (reset > 1) {
+        u32x4* const bands = reinterpret_cast<u32x4*>(counters + kCounterBands);
+        for (int t = threadIdx.x; t < kMaxBands * kBandStride / 4; t += blockDim.x) bands[t] = u32x4{0u, 0u, 0u, 0u};
+    }
     if (threadIdx.x == 0) counters[kCounterStampNorms] = wall_clock64();  // the timed region of a small join starts here
     for (int t = threadIdx.x; t < kCounterWords; t += blockDim.x)
         if (t != kCounterNonFinite && t != kCounterStampNorms && t != kCounterHostWords) counters[t] = 0ull;
@@ -144,7 +148,7 @@ __global__ void __launch_bounds__(256) sum_squared_kernel(const u32x4* __restric
                                                           float* __restrict__ sums, float* __restrict__ halves,
                                                           float quarterEps2, unsigned long long* __restrict__ counters,
                                                           unsigned long long epoch, int reset) {
-    if (reset) reset_for_join(counters);
+    if (reset) reset_for_join(counters, reset);
     const int lane = threadIdx.x & 63;
     const long long wave = ((long long)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
     const int rowsPerWave = 64 / lanesPerRow;
@@ -193,7 +197,7 @@ __global__ void __launch_bounds__(256) sum_squared_kernel(const u32x4* __restric
 __global__ void __launch_bounds__(256) halves_kernel(const float* __restrict__ sums, int n, float quarterEps2,
                                                      float* __restrict__ halves, unsigned long long* __restrict__ counters,
                                                      unsigned long long epoch, int reset) {
-    if (reset) reset_for_join(counters);
+    if (reset) reset_for_join(counters, reset);
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const float s = sums[i];
@@ -1039,7 +1043,7 @@ __global__ void __launch_bounds__(kThreads, 1) join_kernel(JoinParams p) {
                     constexpr int fp = decltype(fpc)::value;
                     store_word<fp * 256>(p.bits, at, hits[fp]);
                 });
-                if (ln < 2 * kSums) asm volatile("global_atomic_add %0, %1, %2" ::"v"(band * 4u), "v"(mine), "s"(bands) : "memory");
+                if (ln < 2 * kSums) asm volatile("global_atomic_add %0, %1, %2" ::"v"(band * (kBandStride * 4u)), "v"(mine), "s"(bands) : "memory");
             } else if (kNoExtract) {
                 if (any && !kNoHits) {
 #pragma unroll
@@ -1157,6 +1161,7 @@ int raster_coord(unsigned long long idx, long long nQ, long long nC, bool upperO
 }
 
 int counter_words() { return kCounterWords; }
+int band_words() { return kMaxBands * kBandStride / 2; }
 int host_words_slot() { return kCounterHostWords; }
 
 // "" for the library proper; a measurement build names what it leaves out (its results are wrong by construction)
@@ -1182,7 +1187,7 @@ int lds_chunk_slot(int row, int chunk) { return (chunk ^ swz(row)) & 7; }
 float quarter_eps2(float eps2) { return (eps2 != eps2 ? -3.0e38f : (eps2 > 3.0e38f ? 3.0e38f : eps2)) * 0.25f; }
 
 hipError_t launch_sum_squared(const void* points, long long ld, int n, int dPad, float* sums, float* halves, float eps2,
-                              unsigned long long* counters, hipStream_t stream, unsigned long long epoch, bool reset) {
+                              unsigned long long* counters, hipStream_t stream, unsigned long long epoch, Reset reset) {
     const int chunksPerRow = dPad / 8;
     int lanesPerRow = 64;
     while (lanesPerRow > chunksPerRow) lanesPerRow >>= 1;
@@ -1191,14 +1196,14 @@ hipError_t launch_sum_squared(const void* points, long long ld, int n, int dPad,
     const long long blocks = (waves + 3) / 4;
     sum_squared_kernel<<<dim3((unsigned)blocks), dim3(256), 0, stream>>>(static_cast<const u32x4*>(points), ld / 8, n,
                                                                         chunksPerRow, lanesPerRow, sums, halves,
-                                                                        quarter_eps2(eps2), counters, epoch, reset ? 1 : 0);
+                                                                        quarter_eps2(eps2), counters, epoch, (int)reset);
     return hipGetLastError();
 }
 
 hipError_t launch_halves(const float* sums, int n, float eps2, float* halves, unsigned long long* counters,
-                         hipStream_t stream, unsigned long long epoch, bool reset) {
+                         hipStream_t stream, unsigned long long epoch, Reset reset) {
     halves_kernel<<<dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream>>>(sums, n, quarter_eps2(eps2), halves, counters,
-                                                                               epoch, reset ? 1 : 0);
+                                                                               epoch, (int)reset);
     return hipGetLastError();
 }
 

@@ -27,7 +27,7 @@ __global__ void __launch_bounds__(kThreads) expand_bits_kernel(const unsigned* _
     const unsigned band = blockIdx.x;
     const unsigned long long started = wall_clock64();
     // where the band's records begin: behind those of the bands before it
-    const unsigned hits = threadIdx.x < gridDim.x ? reinterpret_cast<const unsigned*>(counters + kCounterBands)[threadIdx.x] : 0u;
+    const unsigned hits = threadIdx.x < gridDim.x ? reinterpret_cast<const unsigned*>(counters + kCounterBands)[threadIdx.x * kBandStride] : 0u;
     const unsigned before = wave_sum(threadIdx.x < band || band == 0 ? hits : 0u);  // (the first band adds up all)
     const unsigned pitch = (unsigned)(nC + 31) / 32 | 1u;
     for (unsigned i = threadIdx.x; i < kBandRows * pitch; i += kThreads) rows[i] = 0u;
