@@ -70,7 +70,7 @@ struct Workspace {
     unsigned long long* hostCount = nullptr;
     unsigned long long* hostCountDev = nullptr;  // the same words as the device addresses them
     double clockRate = 0.0;
-    // hit bits of joins of few points whose pairs are wanted in order (at most 31.5 MiB)
+    // hit bits of joins of few points whose pairs are wanted in order (at most 64 MiB)
     unsigned* bits = nullptr;
     size_t bitsBytes = 0;
 

@@ -28,8 +28,8 @@ struct BitsLayout {
     unsigned rowsOfTiles = 0, tileCols = 0;
     bool upper = false;   // tiles on and above the diagonal only
 };
-constexpr int kMaxBitRows = 63 * kTile;            // points of either set of a join that leaves hit bits
-constexpr int kBandRows = 32, kMaxBands = 512;     // query rows are counted, and expanded, in bands
+constexpr int kMaxBitRows = 79 * kTile;            // points of either set of a join that leaves hit bits
+constexpr int kBandRows = 32, kMaxBands = 640;     // query rows are counted, and expanded, in bands
 static_assert(kMaxBitRows / kBandRows <= kMaxBands, "a counter per band");
 
 struct JoinLaunch {

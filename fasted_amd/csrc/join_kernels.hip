@@ -90,15 +90,13 @@ constexpr int kFragCols = kWaveCols / 16;  // a wave's sub-tile: 8 (or 4) x 4 MF
 // SQ_LDS_BANK_CONFLICT counter on the device).
 __host__ __device__ __forceinline__ int swz(int row) { return lds_swizzle128(row); }
 
-// Work queues of the 256x256 kernel (tile_order.hpp).  From 64 x 64 tiles on, an XCD's sub-rectangle is
-// 8 x 4 tiles: the 32 workgroups resident on one XCD work on 8 query panels and 4 candidate panels at a time,
-// and a super-square is 32 x 8 tiles, so a round of the 256 workgroups brings 8 new candidate panels from HBM
-// while the 32 query panels stay in the Infinity Cache.  Measured against 4 x 8 sub-rectangles (16 x 16
-// super-squares, 16 new candidate panels per round): memory-controller activity 2 % instead of 4 %, 1.5 %
-// faster at 1M x 4096, 2 % at 500k x 960 and 100k x 4096, 2.5 % at 2M x 384; still taller super-squares
-// (64 x 4) gain nothing more at D = 384, flatter ones lose (2 x 16: -8 %, 1 x 32: -15 %).
-// Small matrices keep 4 x 8 sub-rectangles (16 x 16 super-squares): fewer padding tiles, and no XCD whose
-// own queue holds nothing but padding.  The join kernel is compiled for both shapes.
+// Work queues (tile_order.hpp).  A matrix of many points is taken in super-squares of 32 x 8 tiles: the 32 workgroups
+// resident on one XCD work on a sub-rectangle of 8 x 4 of them, 8 query panels and 4 candidate panels at a time, and a
+// round of the 256 workgroups brings 8 new candidate panels from HBM while the 32 query panels stay in the Infinity
+// Cache.  Measured against 4 x 8 sub-rectangles (16 x 16 super-squares, 16 new candidate panels per round):
+// memory-controller activity 2 % instead of 4 %, 1.5 % faster at 1M x 4096, 2 % at 500k x 960 and 100k x 4096, 2.5 % at
+// 2M x 384; still taller super-squares (64 x 4) gain nothing more at D = 384, flatter ones lose (2 x 16: -8 %, 1 x 32:
+// -15 %).  Fewer points are taken in strips, without places for tiles that are not there (launch_join).
 // An XCD whose queue is exhausted takes from the next XCD's queue, so the tail stays balanced.
 typedef TileOrder Raster;
 constexpr int kSubTiles = 32;  // per sub-rectangle: the workgroups resident on one XCD
@@ -108,6 +106,7 @@ struct SubShape {
     static constexpr int rows = kTall ? 8 : 4, cols = kTall ? 4 : 8;
 };
 
+// (the host's mirror keeps 4 x 8 sub-rectangles, 16 x 16 super-squares, for matrices of fewer than 64 rows of tiles)
 inline bool tall_order(long long nQueries, int tileRows = kTile) {
     return (nQueries + tileRows - 1) / tileRows >= 64;
 }
@@ -118,7 +117,6 @@ inline Raster make_raster(long long nQueries, long long nCandidates, bool upperO
                 : make_tile_order(nQueries, nCandidates, tileRows, kTile, SubShape<false>::rows, SubShape<false>::cols, upperOnly);
 }
 
-// host mirror of the kernels' decoding
 inline void raster_decode(const Raster& r, bool tall, unsigned q, unsigned long long t, unsigned* tr, unsigned* tc) {
     if (tall)
         tile_order_decode(r, SubShape<true>::rows, SubShape<true>::cols, q, t, tr, tc);
@@ -316,6 +314,7 @@ __device__ __forceinline__ void static_for(F&& f) {
     }
 }
 
+// kSquares: tiles in the order of the super-squares, otherwise in strips.
 // kTileRows = 256, or 128 for matrices of few tiles: the tile grid is then twice as fine along the queries (a wave's
 // sub-tile is 64 x 64, 4 x 4 blocks), so that twice as many workgroups find work.  The transfers stay as they
 // are -- 256 query rows from the tile's first row on are staged, the lower half unused -- which costs nothing
@@ -337,9 +336,10 @@ __device__ __forceinline__ void static_for(F&& f) {
 // kBits: a join of few points whose pairs are wanted in order.  The hit bits themselves leave (BitsLayout), the hits of
 // every band of 32 query rows are counted, and launch_expand_bits makes the list: no staging, no reservations, no records
 // that have to be sorted, and no count that the host waits for in between.
-template <bool kEpilogue, bool kTall, int kTileRows, bool kOneSlab, bool kBitsInLastSlab = false, bool kMirror = false,
+template <bool kEpilogue, bool kSquares, int kTileRows, bool kOneSlab, bool kBitsInLastSlab = false, bool kMirror = false,
           bool kHalfTail = false, bool kBits = false>
 __global__ void __launch_bounds__(kThreads, 1) join_kernel(JoinParams p) {
+    static_assert(kEpilogue || kSquares, "without the epilogue, squares");
     static_assert(!kMirror || (kEpilogue && kTileRows == 256), "pairs are mirrored across the diagonal of square tiles");
     const bool upperOnly = kEpilogue ? kMirror : p.symmetric != 0;
     static_assert(!kBits || kEpilogue, "hit bits come from the epilogue");
@@ -423,20 +423,23 @@ __global__ void __launch_bounds__(kThreads, 1) join_kernel(JoinParams p) {
 
     // Thread 0 only.  `pos` was popped from the home queue; walks on (and on to the other queues
     // once a queue is exhausted) until a tile that has to be computed turns up.  Skipped on the way:
-    // padding tiles of the last super-squares and, in symmetric mode, tiles below the diagonal.
+    // padding tiles of the last super-squares.
     auto find_tile = [&](unsigned long long pos, unsigned* row, unsigned* col) {
         // the divisors pass through an empty volatile statement so that the reciprocals the division
         // needs are formed here, once per tile, instead of living in registers across the k loop
         Raster ras = p.raster;
-        asm volatile("" : "+s"(ras.squareCols));
+        if constexpr (kSquares)
+            asm volatile("" : "+s"(ras.squareCols));
+        else
+            asm volatile("" : "+s"(ras.tileRows));
         unsigned q = home;
         int hops = 0;
         *row = kNoTile;
         *col = 0u;
-        if constexpr (kBits) {
-            // strips without padding tiles, 32 tiles to a queue in turn (of 39 x 39 tiles the super-squares hold 1536 places
-            // for the 780 above the diagonal, and a place that is skipped costs the latency of a reservation)
+        if constexpr (!kSquares) {
+            // strips, 32 tiles to a queue in turn
             const unsigned total = upperOnly ? ras.tileRows * (ras.tileRows + 1) / 2 : ras.tileRows * ras.tileCols;
+#pragma clang loop unroll(disable)
             for (;;) {
                 const unsigned long long number = pos / kSubTiles * (kQueues * kSubTiles) + q * kSubTiles + pos % kSubTiles;
                 if (number < total) {
@@ -452,7 +455,7 @@ __global__ void __launch_bounds__(kThreads, 1) join_kernel(JoinParams p) {
         for (;;) {
             if (pos < ras.perQueue) {
                 unsigned tr, tc;
-                tile_order_decode(ras, SubShape<kTall>::rows, SubShape<kTall>::cols, q, pos, &tr, &tc);
+                tile_order_decode(ras, SubShape<true>::rows, SubShape<true>::cols, q, pos, &tr, &tc);
                 if (tr < ras.tileRows && tc < ras.tileCols && !(upperOnly && tc < tr)) {
                     *row = tr;
                     *col = tc;
@@ -1251,7 +1254,7 @@ namespace {
 
 // One launch of the join kernel over the tile grid described by p.raster, in the queue or the direct mode, with
 // tiles of 256 or 128 query rows.
-hipError_t launch_join_grid(JoinParams p, bool rows128, bool tall, bool epilogue, bool halfTail, int numCUs, hipStream_t stream) {
+hipError_t launch_join_grid(JoinParams p, bool rows128, bool squares, bool epilogue, bool halfTail, int numCUs, hipStream_t stream) {
     const unsigned long long realTiles = p.symmetric ? (unsigned long long)p.raster.tileRows * (p.raster.tileRows + 1) / 2
                                                      : (unsigned long long)p.raster.tileRows * p.raster.tileCols;
     // Up to two tiles per CU, workgroup b computes tile b and ends, one workgroup per tile (the hardware places
@@ -1261,10 +1264,13 @@ hipError_t launch_join_grid(JoinParams p, bool rows128, bool tall, bool epilogue
     if (grid == 0) grid = 1;
     const dim3 g(grid), b(kThreads);
     const bool oneSlab = p.nSlabs == 1;
+    // Tiles of up to 16 slabs gather their hit bits in their last slab; longer ones screen behind the k-loop.
+    const int k = oneSlab ? 2 : epilogue && p.nSlabs <= 16 ? 1 : 0;
+    // (128-row tiles run in one round of the workgroups, whose time is latency: 1000 x 30 is the same without the k-step)
+    const bool half = halfTail && k != 0 && !rows128;
+    const int variant = (half ? 4 : 0) + k;
     if (p.bits) {
-        const int k = oneSlab ? 2 : p.nSlabs <= 16 ? 1 : 0;  // the hit bits behind the k-loop, in the last of several slabs, in the only one
-        const int bitsVariant = rows128 ? k : (p.symmetric ? 16 : 8) + (halfTail && k != 0 ? 4 : 0) + k;
-        switch (bitsVariant) {
+        switch (rows128 ? k : (p.symmetric ? 16 : 8) + variant) {
             case 0: join_kernel<true, false, 128, false, false, false, false, true><<<g, b, 0, stream>>>(p); break;
             case 1: join_kernel<true, false, 128, false, true, false, false, true><<<g, b, 0, stream>>>(p); break;
             case 2: join_kernel<true, false, 128, true, true, false, false, true><<<g, b, 0, stream>>>(p); break;
@@ -1279,62 +1285,47 @@ hipError_t launch_join_grid(JoinParams p, bool rows128, bool tall, bool epilogue
             case 21: join_kernel<true, false, 256, false, true, true, true, true><<<g, b, 0, stream>>>(p); break;
             default: join_kernel<true, false, 256, true, true, true, true, true><<<g, b, 0, stream>>>(p); break;
         }
-        return hipGetLastError();
-    }
-    // Tiles of up to 16 slabs gather their hit bits in their last slab; longer ones screen behind the k-loop.
-    const bool bitsInLastSlab = epilogue && p.nSlabs <= 16;
-    const int variant = (oneSlab ? 8 : 0) | (tall ? 2 : 0) | (rows128 ? 1 : 0);
-    // (128-row tiles run in one round of the workgroups, whose time is latency: 1000 x 30 is the same without the k-step)
-    if (bitsInLastSlab && halfTail && !rows128) {
-        const int halfVariant = (p.symmetric ? 4 : 0) | (oneSlab ? 2 : 0) | (tall ? 1 : 0);
-        switch (halfVariant) {
-            case 7: join_kernel<true, true, 256, true, true, true, true><<<g, b, 0, stream>>>(p); break;
+    } else if (!epilogue) {
+        switch ((oneSlab ? 2 : 0) + (rows128 ? 1 : 0)) {
+            case 0: join_kernel<false, true, 256, false><<<g, b, 0, stream>>>(p); break;
+            case 1: join_kernel<false, true, 128, false><<<g, b, 0, stream>>>(p); break;
+            case 2: join_kernel<false, true, 256, true><<<g, b, 0, stream>>>(p); break;
+            default: join_kernel<false, true, 128, true><<<g, b, 0, stream>>>(p); break;
+        }
+    } else if (p.symmetric) {
+        switch ((squares ? 8 : 0) + variant) {
+            case 0: join_kernel<true, false, 256, false, false, true><<<g, b, 0, stream>>>(p); break;
+            case 1: join_kernel<true, false, 256, false, true, true><<<g, b, 0, stream>>>(p); break;
+            case 2: join_kernel<true, false, 256, true, true, true><<<g, b, 0, stream>>>(p); break;
+            case 5: join_kernel<true, false, 256, false, true, true, true><<<g, b, 0, stream>>>(p); break;
             case 6: join_kernel<true, false, 256, true, true, true, true><<<g, b, 0, stream>>>(p); break;
-            case 5: join_kernel<true, true, 256, false, true, true, true><<<g, b, 0, stream>>>(p); break;
-            case 4: join_kernel<true, false, 256, false, true, true, true><<<g, b, 0, stream>>>(p); break;
-            case 3: join_kernel<true, true, 256, true, true, false, true><<<g, b, 0, stream>>>(p); break;
-            case 2: join_kernel<true, false, 256, true, true, false, true><<<g, b, 0, stream>>>(p); break;
-            case 1: join_kernel<true, true, 256, false, true, false, true><<<g, b, 0, stream>>>(p); break;
-            default: join_kernel<true, false, 256, false, true, false, true><<<g, b, 0, stream>>>(p); break;
+            case 8: join_kernel<true, true, 256, false, false, true><<<g, b, 0, stream>>>(p); break;
+            case 9: join_kernel<true, true, 256, false, true, true><<<g, b, 0, stream>>>(p); break;
+            case 10: join_kernel<true, true, 256, true, true, true><<<g, b, 0, stream>>>(p); break;
+            case 13: join_kernel<true, true, 256, false, true, true, true><<<g, b, 0, stream>>>(p); break;
+            default: join_kernel<true, true, 256, true, true, true, true><<<g, b, 0, stream>>>(p); break;
         }
-    } else if (epilogue && p.symmetric) {
-        const int mirrorVariant = (oneSlab ? 4 : bitsInLastSlab ? 2 : 0) | (tall ? 1 : 0);
-        switch (mirrorVariant) {
-            case 5: join_kernel<true, true, 256, true, true, true><<<g, b, 0, stream>>>(p); break;
-            case 4: join_kernel<true, false, 256, true, true, true><<<g, b, 0, stream>>>(p); break;
-            case 3: join_kernel<true, true, 256, false, true, true><<<g, b, 0, stream>>>(p); break;
-            case 2: join_kernel<true, false, 256, false, true, true><<<g, b, 0, stream>>>(p); break;
-            case 1: join_kernel<true, true, 256, false, false, true><<<g, b, 0, stream>>>(p); break;
-            default: join_kernel<true, false, 256, false, false, true><<<g, b, 0, stream>>>(p); break;
-        }
-    } else if (bitsInLastSlab) {
-        switch (variant) {
-            case 11: join_kernel<true, true, 128, true, true><<<g, b, 0, stream>>>(p); break;
-            case 10: join_kernel<true, true, 256, true, true><<<g, b, 0, stream>>>(p); break;
-            case 9: join_kernel<true, false, 128, true, true><<<g, b, 0, stream>>>(p); break;
-            case 8: join_kernel<true, false, 256, true, true><<<g, b, 0, stream>>>(p); break;
-            case 3: join_kernel<true, true, 128, false, true><<<g, b, 0, stream>>>(p); break;
-            case 2: join_kernel<true, true, 256, false, true><<<g, b, 0, stream>>>(p); break;
+    } else if (rows128) {
+        switch ((squares ? 4 : 0) + k) {
+            case 0: join_kernel<true, false, 128, false><<<g, b, 0, stream>>>(p); break;
             case 1: join_kernel<true, false, 128, false, true><<<g, b, 0, stream>>>(p); break;
-            default: join_kernel<true, false, 256, false, true><<<g, b, 0, stream>>>(p); break;
-        }
-    } else if (epilogue) {  // more than 16 slabs
-        switch (variant) {
-            case 3: join_kernel<true, true, 128, false><<<g, b, 0, stream>>>(p); break;
-            case 2: join_kernel<true, true, 256, false><<<g, b, 0, stream>>>(p); break;
-            case 1: join_kernel<true, false, 128, false><<<g, b, 0, stream>>>(p); break;
-            default: join_kernel<true, false, 256, false><<<g, b, 0, stream>>>(p); break;
+            case 2: join_kernel<true, false, 128, true, true><<<g, b, 0, stream>>>(p); break;
+            case 4: join_kernel<true, true, 128, false><<<g, b, 0, stream>>>(p); break;
+            case 5: join_kernel<true, true, 128, false, true><<<g, b, 0, stream>>>(p); break;
+            default: join_kernel<true, true, 128, true, true><<<g, b, 0, stream>>>(p); break;
         }
     } else {
-        switch (variant) {
-            case 11: join_kernel<false, true, 128, true><<<g, b, 0, stream>>>(p); break;
-            case 10: join_kernel<false, true, 256, true><<<g, b, 0, stream>>>(p); break;
-            case 9: join_kernel<false, false, 128, true><<<g, b, 0, stream>>>(p); break;
-            case 8: join_kernel<false, false, 256, true><<<g, b, 0, stream>>>(p); break;
-            case 3: join_kernel<false, true, 128, false><<<g, b, 0, stream>>>(p); break;
-            case 2: join_kernel<false, true, 256, false><<<g, b, 0, stream>>>(p); break;
-            case 1: join_kernel<false, false, 128, false><<<g, b, 0, stream>>>(p); break;
-            default: join_kernel<false, false, 256, false><<<g, b, 0, stream>>>(p); break;
+        switch ((squares ? 8 : 0) + variant) {
+            case 0: join_kernel<true, false, 256, false><<<g, b, 0, stream>>>(p); break;
+            case 1: join_kernel<true, false, 256, false, true><<<g, b, 0, stream>>>(p); break;
+            case 2: join_kernel<true, false, 256, true, true><<<g, b, 0, stream>>>(p); break;
+            case 5: join_kernel<true, false, 256, false, true, false, true><<<g, b, 0, stream>>>(p); break;
+            case 6: join_kernel<true, false, 256, true, true, false, true><<<g, b, 0, stream>>>(p); break;
+            case 8: join_kernel<true, true, 256, false><<<g, b, 0, stream>>>(p); break;
+            case 9: join_kernel<true, true, 256, false, true><<<g, b, 0, stream>>>(p); break;
+            case 10: join_kernel<true, true, 256, true, true><<<g, b, 0, stream>>>(p); break;
+            case 13: join_kernel<true, true, 256, false, true, false, true><<<g, b, 0, stream>>>(p); break;
+            default: join_kernel<true, true, 256, true, true, false, true><<<g, b, 0, stream>>>(p); break;
         }
     }
     return hipGetLastError();
@@ -1391,10 +1382,23 @@ hipError_t launch_join(const JoinLaunch& launch, hipStream_t stream, BitsLayout*
     if (mayMirror && l.triangle == Triangle::kUpper) rows128 = false;
     p.symmetric = (mayMirror && !rows128) ? 1 : 0;
     const int tileRows = rows128 ? 128 : kTile;
-    p.raster = make_raster(l.nQ, l.nC, p.symmetric != 0, tileRows);
+    // The order of the tiles.  Strips leave nothing out and nothing over: of the places that super-squares have for the upper
+    // triangle, or for 40 rows of tiles, a tenth to a half are skipped, at the latency of a reservation each.  But a round of
+    // the workgroups comes to 64 query panels in a strip and to 32 in a super-square, which are to stay in the Infinity Cache
+    // while the candidate panels pass: up to 64 rows of tiles, or 64 MB of queries (and a number of tiles that fits 32 bits)
+    // unless the squares have next to no padding.  Join kernel, squares -> strips: 9733 x 257 47.7 -> 43.4 us, 16000 x 1024
+    // 218 -> 201, 46416 x 64 213 -> 202, 100000 x 128 1149 -> 1118, 10007 x 250000 x 200 (40 rows) 912 -> 868, 20000 x 60000 x
+    // 200 (79) 465 -> 446; but 16384 x 200000 x 384 (64 rows, two squares) 1.85 -> 1.87 ms, 200000 x 384, 154 MB, 12.73 -> 12.80,
+    // 100000 x 4096, 819 MB, 29.8 -> 30.6.
+    const unsigned long long rowsOfTiles = ((unsigned long long)l.nQ + tileRows - 1) / tileRows;
+    const unsigned long long tileCount = rowsOfTiles * (((unsigned long long)l.nC + kTile - 1) / kTile);
+    const bool fewSkipped = !p.symmetric && (32 - rowsOfTiles % 32) % 32 * 16 <= rowsOfTiles;
+    const bool squares = !l.epilogue || (!l.bits && rowsOfTiles >= 64 &&
+                                         (fewSkipped || (unsigned long long)l.nQ * l.dPad * 2 > 64ull << 20 || tileCount >> 32));
+    p.raster = make_tile_order(l.nQ, l.nC, tileRows, kTile, SubShape<true>::rows, SubShape<true>::cols, p.symmetric != 0);
     p.bits = l.bits;
     if (layout) *layout = BitsLayout{tileRows, p.raster.tileRows, p.raster.tileCols, p.symmetric != 0};
-    return launch_join_grid(p, rows128, tall_order(l.nQ, tileRows), l.epilogue, l.dPad - l.d >= kSlabK / 2, numCUs, stream);
+    return launch_join_grid(p, rows128, squares, l.epilogue, l.dPad - l.d >= kSlabK / 2, numCUs, stream);
 }
 
 }  // namespace fasted

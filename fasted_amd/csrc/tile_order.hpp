@@ -13,6 +13,8 @@
 #else
 #define FASTED_HD
 #endif
+// (a call that is left in a kernel would take the kernel's variables out of its registers)
+#define FASTED_INLINE FASTED_HD inline __attribute__((always_inline))
 
 namespace fasted {
 
@@ -100,8 +102,8 @@ FASTED_HD inline void tile_order_upper_decode(unsigned b, unsigned* tr, unsigned
 
 // Tile `number` of a matrix of rows x cols tiles taken in strips of four columns, row by row in a strip: 32 consecutive
 // numbers are 8 x 4 tiles.  upper: of its upper triangle (rows == cols), diagonal included.  Every number below
-// rows * cols, or rows * (rows + 1) / 2, is a tile: no padding, whatever the shape.
-FASTED_HD inline void tile_strip_decode(unsigned number, unsigned rows, unsigned cols, bool upper, unsigned* tr, unsigned* tc) {
+// rows * cols, or rows * (rows + 1) / 2, is a tile: no padding, whatever the shape.  (Both products fit 32 bits.)
+FASTED_INLINE void tile_strip_decode(unsigned number, unsigned rows, unsigned cols, bool upper, unsigned* tr, unsigned* tc) {
     if (upper) {
         // strips 0 .. j - 1 hold 8 j^2 + 2 j tiles; the root is an estimate, then corrected
         unsigned j = (unsigned)((__builtin_sqrtf(8.0f * (float)number + 1.0f) - 1.0f) * 0.125f);

@@ -73,7 +73,7 @@ void releaseResources(void);
 
 /* The two kernel times are HIP-event times on the stream, as the reference measures them
  * (source/findPairs.cuh:625-639,695-697); for joins of at most 512 tiles of 256 x 256, and sorted ones of at most
- * 16 128 points a side, where three event records would cost a third of the call, they are differences of the device's constant-rate clock, read by the kernels
+ * 20 224 points a side, where three event records would cost a third of the call, they are differences of the device's constant-rate clock, read by the kernels
  * themselves (hipDeviceAttributeWallClockRate ticks): by the first norm kernel and the join kernel as they start,
  * and by the join kernel's last workgroup when it has nothing left to do (sorted: by the kernel that makes the list, as
  * it starts). */
@@ -81,7 +81,7 @@ typedef struct FastedJoinStats {
     float sumSquaredMs; /* squared-norm pre-pass (which also clears the counters): its start to the join kernel's start */
     float joinMs;       /* the join kernel: its start to the event behind it (small joins: to its last workgroup's report) */
     float sortMs;       /* host wall time of the row-major sort, stream synchronisation included (0 when not sorted); up to
-                           16 128 points a side, where the list is made in order, the device's time of the kernel that does it */
+                           20 224 points a side, where the list is made in order, the device's time of the kernel that does it */
     int paddedN;        /* rows covered by the tile grid */
     int paddedD;        /* K extent the kernel looped over */
     unsigned long long tiles;      /* size of the distance matrix in 256x256 tiles (with FASTED_SYMMETRIC: those on and
@@ -148,9 +148,9 @@ int fasted_self_join_blocked(const uint16_t* points, long long n, int d, double 
  * count to the host (a few microseconds before the stream itself reports idle, a fifth of such a call).  Every
  * pair record and squared norm is in device memory by then, for any stream, copy or kernel that reads them next;
  * the stream may still answer hipStreamQuery with hipErrorNotReady for a moment.  With FASTED_SORT_PAIRS the stream is
- * drained, and where more pairs are found than fit, up to 16 128 points a side the first `cap` of the row-major list are
+ * drained, and where more pairs are found than fit, up to 20 224 points a side the first `cap` of the row-major list are
  * stored (otherwise some `cap` of them, in order).  The device buffers of that are allocated by the library and kept: up to
- * 16 128 points a side a bit per element of the distance matrix (1 to 32 MB); beyond that none up to 8192 pairs, 4 bytes a pair up to
+ * 20 224 points a side a bit per element of the distance matrix (1 to 64 MB); beyond that none up to 8192 pairs, 4 bytes a pair up to
  * 2^20 and 8 beyond, and tables of up to about 35 MB; lists that leave the distribution for the radix sort take 8 bytes
  * a pair and its storage, about as much again.  The counters and, without d_sums, the squared norms are kept as well.
  * releaseResources() frees all of it.  Replaces the
@@ -209,8 +209,9 @@ int fasted_check_padding_device(const void* d_points, long long n, int d, long l
  * SumSqd::ComputeSquaredSums (source/sumSquared.cuh:84-118). */
 int fasted_sum_squared_device(const void* d_points, long long n, int d, long long ld, float* d_sums, void* stream);
 
-/* Tile order of the work queues: writes the (row, col) origin, in points, of the 256x256 tile
- * that queue index `idx` stands for in an n-point problem.  idx enumerates the eight per-XCD
+/* Tile order of the work queues in super-squares, which is how the join kernel takes a matrix of 64 rows of tiles and more
+ * and more than 64 MB of points (smaller ones it takes in strips without padding): writes the (row, col) origin, in points, of the
+ * 256x256 tile that queue index `idx` stands for in an n-point problem.  idx enumerates the eight per-XCD
  * queues round-robin (queue idx % 8, position idx / 8).  Returns 0 past the end, 1 for a real
  * tile, 2 for a padding tile of the last raster squares (the kernel skips those).  Host-side
  * mirror of the device rasterizer, the counterpart of Raster::OnDemandRasterizer::nextChunk

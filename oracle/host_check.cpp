@@ -166,8 +166,9 @@ static void check_tile_order() {
             }
     }
     // strips of four columns: every tile of a matrix, or of its upper triangle, exactly once
-    for (unsigned rows = 1; rows <= 70; ++rows)
-        for (unsigned cols = 1; cols <= 70; ++cols)
+    const unsigned sides[] = {1, 2, 3, 4, 5, 7, 8, 31, 32, 33, 63, 64, 65, 79, 97, 391, 978};
+    for (unsigned rows : sides)
+        for (unsigned cols : sides)
             for (int upper = 0; upper <= (rows == cols ? 1 : 0); ++upper) {
                 std::set<std::pair<unsigned, unsigned>> seen;
                 const unsigned total = upper ? rows * (rows + 1) / 2 : rows * cols;
@@ -179,6 +180,14 @@ static void check_tile_order() {
                 }
                 CHECK(seen.size() == total);
             }
+    // the ends of the largest matrices that are taken in strips (64 MB of rows of 128 bytes, and of two sets)
+    for (unsigned back : {1u, 2u, 3u}) {
+        unsigned r = 0, c = 0;
+        fasted::tile_strip_decode(2048u * 2049u / 2 - back, 2048, 2048, true, &r, &c);
+        CHECK(r <= c && c >= 2046 && c <= 2047 && r >= 2046);
+        fasted::tile_strip_decode(500u * 8388000u - back, 500, 8388000, false, &r, &c);
+        CHECK(r == 499 && c == 8388000 - back);
+    }
     // LDS swizzles: the 16 lanes of every ds_read_b128 phase touch all 64 banks once
     const int groups[2][16] = {{0, 1, 2, 3, 12, 13, 14, 15, 20, 21, 22, 23, 24, 25, 26, 27},
                                {4, 5, 6, 7, 8, 9, 10, 11, 16, 17, 18, 19, 28, 29, 30, 31}};

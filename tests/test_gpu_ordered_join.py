@@ -57,8 +57,8 @@ def test_lists_of_every_density(n, d, share):
 
 
 @pytest.mark.parametrize("rows", [None, "256", "128"])
-@pytest.mark.parametrize("nq,nc,d", [(1, 16128, 64), (16128, 1, 40), (33, 9000, 100), (9000, 33, 1100), (3000, 5000, 64), (16128, 700, 65),
-                                     (16129, 700, 65), (700, 16129, 65)])
+@pytest.mark.parametrize("nq,nc,d", [(1, 20224, 64), (20224, 1, 40), (33, 9000, 100), (9000, 33, 1100), (3000, 5000, 64), (20224, 700, 65),
+                                     (20225, 700, 65), (700, 20225, 65)])
 def test_two_sets(nq, nc, d, rows, monkeypatch):
     """Both sides up to the last size that leaves hit bits, and one past it on either side; both tile heights."""
     import torch
@@ -80,7 +80,7 @@ def test_two_sets(nq, nc, d, rows, monkeypatch):
         assert torch.equal(pairs[: len(want)], want)
 
 
-@pytest.mark.parametrize("n", [16128, 16129])
+@pytest.mark.parametrize("n", [20224, 20225])
 @pytest.mark.parametrize("rows", [None, "128"])
 def test_the_last_size_in_bits_and_the_next(n, rows, monkeypatch):
     import torch
