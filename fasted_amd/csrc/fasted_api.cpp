@@ -289,20 +289,22 @@ void join_on_device(PointSet q, PointSet c, bool selfJoin, int d, double epsilon
                                    q.n <= fasted::kMaxBitRows && c.n <= fasted::kMaxBitRows
                                ? g_ws.ensure_bits(fasted::bits_bytes((int)q.n, (int)c.n))
                                : nullptr;
-    // Timing.  Three event records cost a call about 10 us, a third of a join of a few thousand points, so a
-    // join of at most two tiles per compute unit is timed by the kernels themselves instead: the first norm
+    // Timing.  Three event records cost a call about 10 us, a third of a join of a few thousand points, so joins of up to
+    // 2^17 tiles (a millisecond or two) are timed by the kernels themselves instead: the first norm
     // kernel and the join kernel note the device's constant-rate clock when they start, and the join kernel's
     // last workgroup when it hands the pair count to the host.  Larger joins, and the entry
     // that owns no pinned memory, are timed with events on the stream as the reference is
-    // (source/findPairs.cuh:625-639,695-697,728-736).
-    const bool stamped = !fixed && !(flags & FASTED_EVENT_TIMING) && (bits || fasted::tile_count(q.n, c.n) <= 512);
+    // (source/findPairs.cuh:625-639,695-697,728-736).  The host takes the report for the end of the join, up to two tiles
+    // per compute unit and where the sort follows, which drains the stream; otherwise it waits for the stream.
+    const unsigned long long tiles = fasted::tile_count(q.n, c.n);
+    const bool stamped = !fixed && !(flags & FASTED_EVENT_TIMING) && (bits || tiles <= 1ull << 17);
+    const bool polled = stamped && !bits && (tiles <= 512 || (flags & FASTED_SORT_PAIRS));
     const bool events = !stamped && stats != nullptr;
     const fasted::Reset reset = bits ? fasted::Reset::kCountersAndBands : fasted::Reset::kCounters;
     if (events) HIP_CHECK(hipEventRecord(t.ev[0], stream));
     if (!(flags & FASTED_SKIP_SUMS)) {
-        HIP_CHECK(fasted::launch_sum_squared(q.ptr, q.ld, (int)q.n, dPad, sumsQ, halfQ, eps2, counters, stream, epoch, reset));
-        if (!selfJoin)
-            HIP_CHECK(fasted::launch_sum_squared(c.ptr, c.ld, (int)c.n, dPad, sumsC, halfC, eps2, counters, stream, epoch));
+        const fasted::NormPoints nq{q.ptr, q.ld, (int)q.n, sumsQ, halfQ}, nc{c.ptr, c.ld, (int)c.n, sumsC, halfC};
+        HIP_CHECK(fasted::launch_sum_squared(nq, selfJoin ? nullptr : &nc, dPad, eps2, counters, stream, epoch, reset));
     } else {
         HIP_CHECK(fasted::launch_halves(sumsQ, (int)q.n, eps2, halfQ, counters, stream, epoch, reset));
         if (!selfJoin) HIP_CHECK(fasted::launch_halves(sumsC, (int)c.n, eps2, halfC, counters, stream, epoch));
@@ -351,7 +353,7 @@ void join_on_device(PointSet q, PointSet c, bool selfJoin, int d, double epsilon
         // reports, because it failed, falls through to the stream's own wait, which returns the error.)
         volatile unsigned long long* const w = g_ws.hostCount;
         bool reported = false;
-        if (stamped && !bits) {
+        if (polled) {
             const auto t0 = std::chrono::steady_clock::now();
             for (unsigned spins = 1; !(reported = w[3] != 0); ++spins)
                 if ((spins & 1023u) == 0 && std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(2)) break;
@@ -367,7 +369,8 @@ void join_on_device(PointSet q, PointSet c, bool selfJoin, int d, double epsilon
         }
     }
     cnt[1] = (jl.epilogue && cnt[0] > cap) ? cap : cnt[0];
-    cnt[2] = fasted::tile_count(q.n, c.n);
+    if (polled && tiles > 512 && cnt[1] < 2) HIP_CHECK(hipStreamSynchronize(stream));  // (no sort that would)
+    cnt[2] = tiles;
     if (jl.triangle == fasted::Triangle::kUpper) {
         const unsigned long long side = ((unsigned long long)q.n + fasted::kTile - 1) / fasted::kTile;
         cnt[2] = side * (side + 1) / 2;
@@ -603,8 +606,8 @@ void self_join_blocked(const uint16_t* points, long long n, int d, double epsilo
     auto make_ready = [&](BlockBuffer& b) {
         HIP_CHECK(hipStreamWaitEvent(dev.compute, b.uploaded, 0));
         if (!haveHalves[(size_t)b.block]) {
-            HIP_CHECK(fasted::launch_sum_squared(b.rows, dPad, (int)block_rows(b.block), dPad, nullptr,
-                                                 halves + (size_t)b.block * rows, eps2, g_ws.counters, dev.compute, epoch));
+            const fasted::NormPoints np{b.rows, dPad, (int)block_rows(b.block), nullptr, halves + (size_t)b.block * rows};
+            HIP_CHECK(fasted::launch_sum_squared(np, nullptr, dPad, eps2, g_ws.counters, dev.compute, epoch));
             haveHalves[(size_t)b.block] = 1;
         }
     };
@@ -1260,8 +1263,8 @@ int fasted_sum_squared_device(const void* d_points, long long n, int d, long lon
     return guarded([&] {
         if (!d_points || !d_sums) throw std::invalid_argument("null pointer");
         validate_shape(n, d, ld);
-        HIP_CHECK(fasted::launch_sum_squared(d_points, ld, (int)n, round_up(d, fasted::kSlabK), d_sums, nullptr, 0.0f,
-                                             nullptr, static_cast<hipStream_t>(stream)));
+        const fasted::NormPoints np{d_points, ld, (int)n, d_sums, nullptr};
+        HIP_CHECK(fasted::launch_sum_squared(np, nullptr, round_up(d, fasted::kSlabK), 0.0f, nullptr, static_cast<hipStream_t>(stream)));
         HIP_CHECK(hipStreamSynchronize(static_cast<hipStream_t>(stream)));
     });
 }

@@ -86,9 +86,15 @@ enum class Reset { kNothing = 0, kCounters = 1, kCountersAndBands = 2 };
 // tests  h_q + h_c + q.c >= 0.  A non-finite norm raises the flag in `counters` (the join then tests element
 // by element): the flag word receives `epoch`.  With `reset` the kernel also clears the pair counter and the
 // queue heads, and the counts of the bands, for the join that follows (no launch_reset_counters needed).
-hipError_t launch_sum_squared(const void* points, long long ld, int n, int dPad, float* sums, float* halves, float eps2,
-                              unsigned long long* counters, hipStream_t stream, unsigned long long epoch = 1,
-                              Reset reset = Reset::kNothing);
+// One launch serves one set of points or two.
+struct NormPoints {
+    const void* points;
+    long long ld;
+    int n;
+    float *sums, *halves;
+};
+hipError_t launch_sum_squared(const NormPoints& first, const NormPoints* second, int dPad, float eps2, unsigned long long* counters,
+                              hipStream_t stream, unsigned long long epoch = 1, Reset reset = Reset::kNothing);
 // The same halves from norms that are already there.
 hipError_t launch_halves(const float* sums, int n, float eps2, float* halves, unsigned long long* counters,
                          hipStream_t stream, unsigned long long epoch = 1, Reset reset = Reset::kNothing);

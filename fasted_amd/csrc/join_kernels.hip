@@ -141,14 +141,26 @@ __device__ __forceinline__ void reset_for_join(unsigned long long* __restrict__ 
         if (t != kCounterNonFinite && t != kCounterStampNorms && t != kCounterHostWords) counters[t] = 0ull;
 }
 
-__global__ void __launch_bounds__(256) sum_squared_kernel(const u32x4* __restrict__ pts, long long ld16, int n,
-                                                          int chunksPerRow, int lanesPerRow,
-                                                          float* __restrict__ sums, float* __restrict__ halves,
+// (two sets of points in one launch: the second begins at workgroup `firstGroups`; 1668 and 38602 x 32 in two launches took a
+// call 80 us, in one, and without events behind it, 66)
+struct NormSet {
+    const u32x4* pts;
+    long long ld16;
+    int n;
+    float *sums, *halves;
+};
+__global__ void __launch_bounds__(256) sum_squared_kernel(NormSet a, NormSet b, unsigned firstGroups, int chunksPerRow, int lanesPerRow,
                                                           float quarterEps2, unsigned long long* __restrict__ counters,
                                                           unsigned long long epoch, int reset) {
     if (reset) reset_for_join(counters, reset);
+    const bool second = blockIdx.x >= firstGroups;
+    const u32x4* __restrict__ const pts = second ? b.pts : a.pts;
+    const long long ld16 = second ? b.ld16 : a.ld16;
+    const int n = second ? b.n : a.n;
+    float* __restrict__ const sums = second ? b.sums : a.sums;
+    float* __restrict__ const halves = second ? b.halves : a.halves;
     const int lane = threadIdx.x & 63;
-    const long long wave = ((long long)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
+    const long long wave = ((long long)(blockIdx.x - (second ? firstGroups : 0u)) * blockDim.x + threadIdx.x) >> 6;
     const int rowsPerWave = 64 / lanesPerRow;
     const long long row = wave * rowsPerWave + lane / lanesPerRow;
     const int sub = lane % lanesPerRow;
@@ -1189,17 +1201,17 @@ int lds_chunk_slot(int row, int chunk) { return (chunk ^ swz(row)) & 7; }
 // distance compares <= NaN in the reference (source/warpMma.cuh:257), and only the forced self pairs remain.
 float quarter_eps2(float eps2) { return (eps2 != eps2 ? -3.0e38f : (eps2 > 3.0e38f ? 3.0e38f : eps2)) * 0.25f; }
 
-hipError_t launch_sum_squared(const void* points, long long ld, int n, int dPad, float* sums, float* halves, float eps2,
-                              unsigned long long* counters, hipStream_t stream, unsigned long long epoch, Reset reset) {
+hipError_t launch_sum_squared(const NormPoints& first, const NormPoints* second, int dPad, float eps2, unsigned long long* counters,
+                              hipStream_t stream, unsigned long long epoch, Reset reset) {
     const int chunksPerRow = dPad / 8;
     int lanesPerRow = 64;
     while (lanesPerRow > chunksPerRow) lanesPerRow >>= 1;
-    const int rowsPerWave = 64 / lanesPerRow;
-    const long long waves = ((long long)n + rowsPerWave - 1) / rowsPerWave;
-    const long long blocks = (waves + 3) / 4;
-    sum_squared_kernel<<<dim3((unsigned)blocks), dim3(256), 0, stream>>>(static_cast<const u32x4*>(points), ld / 8, n,
-                                                                        chunksPerRow, lanesPerRow, sums, halves,
-                                                                        quarter_eps2(eps2), counters, epoch, (int)reset);
+    const int rowsPerGroup = 4 * (64 / lanesPerRow);
+    auto set = [](const NormPoints& p) { return NormSet{static_cast<const u32x4*>(p.points), p.ld / 8, p.n, p.sums, p.halves}; };
+    auto groups = [&](const NormPoints& p) { return (unsigned)(((long long)p.n + rowsPerGroup - 1) / rowsPerGroup); };
+    const unsigned firstGroups = groups(first);
+    sum_squared_kernel<<<dim3(firstGroups + (second ? groups(*second) : 0u)), dim3(256), 0, stream>>>(
+        set(first), second ? set(*second) : NormSet{}, firstGroups, chunksPerRow, lanesPerRow, quarter_eps2(eps2), counters, epoch, (int)reset);
     return hipGetLastError();
 }
 
@@ -1385,16 +1397,17 @@ hipError_t launch_join(const JoinLaunch& launch, hipStream_t stream, BitsLayout*
     // The order of the tiles.  Strips leave nothing out and nothing over: of the places that super-squares have for the upper
     // triangle, or for 40 rows of tiles, a tenth to a half are skipped, at the latency of a reservation each.  But a round of
     // the workgroups comes to 64 query panels in a strip and to 32 in a super-square, which are to stay in the Infinity Cache
-    // while the candidate panels pass: up to 64 rows of tiles, or 64 MB of queries (and a number of tiles that fits 32 bits)
+    // while the candidate panels pass: up to 64 rows of tiles, or 32 MB of queries (and a number of tiles that fits 32 bits)
     // unless the squares have next to no padding.  Join kernel, squares -> strips: 9733 x 257 47.7 -> 43.4 us, 16000 x 1024
     // 218 -> 201, 46416 x 64 213 -> 202, 100000 x 128 1149 -> 1118, 10007 x 250000 x 200 (40 rows) 912 -> 868, 20000 x 60000 x
-    // 200 (79) 465 -> 446; but 16384 x 200000 x 384 (64 rows, two squares) 1.85 -> 1.87 ms, 200000 x 384, 154 MB, 12.73 -> 12.80,
+    // 200 (79) 465 -> 446; but 16384 x 200000 x 384 (64 rows, two squares) 1.85 -> 1.87 ms, 46416 x 512,
+    // 47 MB, 846 -> 838 us on one box and, by whole calls, 2 % slower on another, 200000 x 384, 154 MB, 12.73 -> 12.80,
     // 100000 x 4096, 819 MB, 29.8 -> 30.6.
     const unsigned long long rowsOfTiles = ((unsigned long long)l.nQ + tileRows - 1) / tileRows;
     const unsigned long long tileCount = rowsOfTiles * (((unsigned long long)l.nC + kTile - 1) / kTile);
     const bool fewSkipped = !p.symmetric && (32 - rowsOfTiles % 32) % 32 * 16 <= rowsOfTiles;
     const bool squares = !l.epilogue || (!l.bits && rowsOfTiles >= 64 &&
-                                         (fewSkipped || (unsigned long long)l.nQ * l.dPad * 2 > 64ull << 20 || tileCount >> 32));
+                                         (fewSkipped || (unsigned long long)l.nQ * l.dPad * 2 > 32ull << 20 || tileCount >> 32));
     p.raster = make_tile_order(l.nQ, l.nC, tileRows, kTile, SubShape<true>::rows, SubShape<true>::cols, p.symmetric != 0);
     p.bits = l.bits;
     if (layout) *layout = BitsLayout{tileRows, p.raster.tileRows, p.raster.tileCols, p.symmetric != 0};

@@ -72,14 +72,14 @@ void releaseResources(void);
  * Return 0 on success, non-zero on failure; fasted_last_error() then describes it.     */
 
 /* The two kernel times are HIP-event times on the stream, as the reference measures them
- * (source/findPairs.cuh:625-639,695-697); for joins of at most 512 tiles of 256 x 256, and sorted ones of at most
- * 20 224 points a side, where three event records would cost a third of the call, they are differences of the device's constant-rate clock, read by the kernels
+ * (source/findPairs.cuh:625-639,695-697); for joins of at most 131 072 tiles of 256 x 256, where three event
+ * records would cost up to a third of the call, they are differences of the device's constant-rate clock, read by the kernels
  * themselves (hipDeviceAttributeWallClockRate ticks): by the first norm kernel and the join kernel as they start,
  * and by the join kernel's last workgroup when it has nothing left to do (sorted: by the kernel that makes the list, as
  * it starts). */
 typedef struct FastedJoinStats {
     float sumSquaredMs; /* squared-norm pre-pass (which also clears the counters): its start to the join kernel's start */
-    float joinMs;       /* the join kernel: its start to the event behind it (small joins: to its last workgroup's report) */
+    float joinMs;       /* the join kernel: its start to the event behind it (without events: to its last workgroup's report) */
     float sortMs;       /* host wall time of the row-major sort, stream synchronisation included (0 when not sorted); up to
                            20 224 points a side, where the list is made in order, the device's time of the kernel that does it */
     int paddedN;        /* rows covered by the tile grid */
@@ -103,7 +103,7 @@ enum {
                                smaller tiles.  Same pair set in every case. */
     FASTED_EVENT_TIMING = 16, /* time the kernels with HIP events and wait for the stream whatever the size of the
                                join, as the reference does (source/findPairs.cuh:625-639,695-697): for joins of at
-                               most 512 tiles this costs the call about 15 us and is what a profiler's kernel
+                               most 131 072 tiles this costs the call 10 to 15 us and is what a profiler's kernel
                                durations compare with. */
     FASTED_FULL_MATRIX = 32 /* self-join only: compute every tile of the matrix, all 2*N*N*D operations, as the
                                reference always does (source/findPairs.cuh:650-653).  For measurements that divide
@@ -210,7 +210,7 @@ int fasted_check_padding_device(const void* d_points, long long n, int d, long l
 int fasted_sum_squared_device(const void* d_points, long long n, int d, long long ld, float* d_sums, void* stream);
 
 /* Tile order of the work queues in super-squares, which is how the join kernel takes a matrix of 64 rows of tiles and more
- * and more than 64 MB of points (smaller ones it takes in strips without padding): writes the (row, col) origin, in points, of the
+ * and more than 32 MB of points (smaller ones it takes in strips without padding): writes the (row, col) origin, in points, of the
  * 256x256 tile that queue index `idx` stands for in an n-point problem.  idx enumerates the eight per-XCD
  * queues round-robin (queue idx % 8, position idx / 8).  Returns 0 past the end, 1 for a real
  * tile, 2 for a padding tile of the last raster squares (the kernel skips those).  Host-side
