@@ -117,7 +117,7 @@ enum {
  * SimSearch::FindPairs (source/findPairs.cuh:615-764) for a caller that owns its data.
  * Device memory: the padded points and `cap` records (at least 32 MB of them where D % 64 != 0), and what the sort
  * needs.  A buffer of up to 256 MB for points and records stays allocated for the next call, one for the whole
- * process; releaseResources() frees it.  `cap` of more than 2^45 is refused. */
+ * process, and 4 MB of pinned host memory where lists of 4 MB and more came down; releaseResources() frees them.  `cap` of more than 2^45 is refused. */
 int fasted_self_join(const uint16_t* points, long long n, int d, double epsilon, FastedPair* out,
                      unsigned long long cap, unsigned long long* found, unsigned long long* stored);
 

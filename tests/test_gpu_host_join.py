@@ -71,3 +71,33 @@ def test_host_join_after_one_that_was_refused():
         assert rc != 0
         rc, got, found = _self_join(bits, eps, len(want))
         assert rc == 0 and found == len(want) and np.array_equal(got, want)
+
+
+# lists that come down in one copy and in pinned pieces of 2 MB: a record short of 4 MB and as much, whole pieces, a piece and a
+# record, many; in one go and in blocks of rows
+@pytest.mark.parametrize("n,cap", [(725, 524287), (725, 524288), (725, 525625), (900, 786432), (900, 786433), (2900, 2900 * 2900)])
+@pytest.mark.parametrize("block", [0, 512])
+def test_long_lists_come_down_whole(n, cap, block):
+    import fasted_amd as fasted
+
+    bits = datasets.small_integers(n, 5, high=3, seed=n)
+    lib = fasted.load_findpairs()
+    found, stored = ctypes.c_ulonglong(), ctypes.c_ulonglong()
+    want = np.stack(np.divmod(np.arange(cap, dtype=np.int32), np.int32(n)), 1)
+    for _ in range(2):
+        out = np.full((cap + 1, 2), -1, dtype=np.int32)
+        args = (out.ctypes.data, cap, ctypes.byref(found), ctypes.byref(stored))
+        if block:
+            rc = lib.fasted_self_join_blocked(bits.ctypes.data, n, 5, float("inf"), block, *args)
+        else:
+            rc = lib.fasted_self_join(bits.ctypes.data, n, 5, float("inf"), *args)
+        assert rc == 0
+        if not block:
+            assert found.value == n * n and stored.value == cap
+            assert np.array_equal(out[:cap], want) and (out[cap] == -1).all()
+        else:
+            # (a block of rows keeps 256 pairs per point: as many of its pairs as that, in order)
+            got = out[: stored.value]
+            assert found.value == n * n and stored.value == min(cap, 256 * 512 * -(-n // 512))
+            keys = got[:, 0].astype(np.int64) * n + got[:, 1]
+            assert (np.diff(keys) > 0).all() and got.min() >= 0 and got.max() < n and (out[stored.value :] == -1).all()
