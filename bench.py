@@ -351,7 +351,7 @@ def main():
     sums_ms = sum(s.sumSquaredMs for s in stats) / len(stats)
     timing = "hip events on the launch stream"
     device_clock = None
-    if st.tiles <= 512 and not args.no_epilogue:
+    if st.tiles <= 1 << 17 and not args.no_epilogue:
         # A join this small returns on the join kernel's own report and times its kernels with the device's clock
         # (first instruction of the first workgroup to the last workgroup's sign-off): shorter than the dispatch
         # that events and a profiler's kernel trace see.  The roofline's duration is the events' one, from as
