@@ -1401,7 +1401,7 @@ hipError_t launch_join(const JoinLaunch& launch, hipStream_t stream, BitsLayout*
     // unless the squares have next to no padding.  Join kernel, squares -> strips: 9733 x 257 47.7 -> 43.4 us, 16000 x 1024
     // 218 -> 201, 46416 x 64 213 -> 202, 100000 x 128 1149 -> 1118, 10007 x 250000 x 200 (40 rows) 912 -> 868, 20000 x 60000 x
     // 200 (79) 465 -> 446; but 16384 x 200000 x 384 (64 rows, two squares) 1.85 -> 1.87 ms, 46416 x 512,
-    // 47 MB, 846 -> 838 us on one box and, by whole calls, 2 % slower on another, 200000 x 384, 154 MB, 12.73 -> 12.80,
+    // 47 MB, 846 -> 838 us on one card and, by whole calls, 2 % slower on another, 200000 x 384, 154 MB, 12.73 -> 12.80,
     // 100000 x 4096, 819 MB, 29.8 -> 30.6.
     const unsigned long long rowsOfTiles = ((unsigned long long)l.nQ + tileRows - 1) / tileRows;
     const unsigned long long tileCount = rowsOfTiles * (((unsigned long long)l.nC + kTile - 1) / kTile);
