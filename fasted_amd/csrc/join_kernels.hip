@@ -1397,17 +1397,19 @@ hipError_t launch_join(const JoinLaunch& launch, hipStream_t stream, BitsLayout*
     // The order of the tiles.  Strips leave nothing out and nothing over: of the places that super-squares have for the upper
     // triangle, or for 40 rows of tiles, a tenth to a half are skipped, at the latency of a reservation each.  But a round of
     // the workgroups comes to 64 query panels in a strip and to 32 in a super-square, which are to stay in the Infinity Cache
-    // while the candidate panels pass: up to 64 rows of tiles, or 32 MB of queries (and a number of tiles that fits 32 bits)
-    // unless the squares have next to no padding.  Join kernel, squares -> strips: 9733 x 257 47.7 -> 43.4 us, 16000 x 1024
-    // 218 -> 201, 46416 x 64 213 -> 202, 100000 x 128 1149 -> 1118, 10007 x 250000 x 200 (40 rows) 912 -> 868, 20000 x 60000 x
-    // 200 (79) 465 -> 446; but 16384 x 200000 x 384 (64 rows, two squares) 1.85 -> 1.87 ms, 46416 x 512,
-    // 47 MB, 846 -> 838 us on one card and, by whole calls, 2 % slower on another, 200000 x 384, 154 MB, 12.73 -> 12.80,
-    // 100000 x 4096, 819 MB, 29.8 -> 30.6.
+    // while the candidate panels pass, and a queue's next tiles find none of their query panels in the L2: up to 64 rows of
+    // tiles, or 32 MB of queries (and a number of tiles that fits 32 bits) unless the squares have next to no padding, and
+    // triangles of up to 128 rows.  Join kernel, squares -> strips: 9733 x 257 47.7 -> 43.4 us, 16000 x 1024 218 -> 201, 22000 x
+    // 300 150 -> 143, 30000 x 200 203 -> 188, 10007 x 250000 x 200 (40 rows) 912 -> 868, 20000 x 60000 x 200 (79) 465 -> 446; but
+    // 16384 x 200000 x 384 (64 rows, two squares) 1.85 -> 1.87 ms, 100000 x 128 (391 rows) 1124 -> 1110 us on one card and 2 %
+    // slower on another, 200000 x 384, 154 MB, 12.73 -> 12.80 ms, 100000 x 4096, 819 MB, 29.8 -> 30.6.  (Strips of eight rows
+    // instead of four columns, whose queries stay in the L2: the same within 2 %, 16000 x 128 50.6 against 53.9 us.)
     const unsigned long long rowsOfTiles = ((unsigned long long)l.nQ + tileRows - 1) / tileRows;
     const unsigned long long tileCount = rowsOfTiles * (((unsigned long long)l.nC + kTile - 1) / kTile);
     const bool fewSkipped = !p.symmetric && (32 - rowsOfTiles % 32) % 32 * 16 <= rowsOfTiles;
     const bool squares = !l.epilogue || (!l.bits && rowsOfTiles >= 64 &&
-                                         (fewSkipped || (unsigned long long)l.nQ * l.dPad * 2 > 32ull << 20 || tileCount >> 32));
+                                         (fewSkipped || (p.symmetric && rowsOfTiles > 128) ||
+                                          (unsigned long long)l.nQ * l.dPad * 2 > 32ull << 20 || tileCount >> 32));
     p.raster = make_tile_order(l.nQ, l.nC, tileRows, kTile, SubShape<true>::rows, SubShape<true>::cols, p.symmetric != 0);
     p.bits = l.bits;
     if (layout) *layout = BitsLayout{tileRows, p.raster.tileRows, p.raster.tileCols, p.symmetric != 0};

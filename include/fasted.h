@@ -209,8 +209,8 @@ int fasted_check_padding_device(const void* d_points, long long n, int d, long l
  * SumSqd::ComputeSquaredSums (source/sumSquared.cuh:84-118). */
 int fasted_sum_squared_device(const void* d_points, long long n, int d, long long ld, float* d_sums, void* stream);
 
-/* Tile order of the work queues in super-squares, which is how the join kernel takes a matrix of 64 rows of tiles and more
- * and more than 32 MB of points (smaller ones it takes in strips without padding): writes the (row, col) origin, in points, of the
+/* Tile order of the work queues in super-squares, which is how the join kernel takes a matrix of more than 128 rows of tiles
+ * or 32 MB of points, 64 rows at least (smaller ones it takes in strips without padding): writes the (row, col) origin, in points, of the
  * 256x256 tile that queue index `idx` stands for in an n-point problem.  idx enumerates the eight per-XCD
  * queues round-robin (queue idx % 8, position idx / 8).  Returns 0 past the end, 1 for a real
  * tile, 2 for a padding tile of the last raster squares (the kernel skips those).  Host-side
