@@ -86,13 +86,27 @@ enum class Reset { kNothing = 0, kCounters = 1, kCountersAndBands = 2 };
 // tests  h_q + h_c + q.c >= 0.  A non-finite norm raises the flag in `counters` (the join then tests element
 // by element): the flag word receives `epoch`.  With `reset` the kernel also clears the pair counter and the
 // queue heads, and the counts of the bands, for the join that follows (no launch_reset_counters needed).
-// One launch serves one set of points or two.
+// One launch serves one set of points, or two where a launch can hold the workgroups of both (2^32 - 1 threads).
 struct NormPoints {
     const void* points;
     long long ld;
     int n;
     float *sums, *halves;
 };
+constexpr int kNormThreads = 256;
+// Lanes that share a row of dPad halves, and the workgroups of n such rows.
+constexpr int norm_lanes(int dPad) {
+    int lanes = 64;
+    while (lanes > dPad / 8) lanes >>= 1;
+    return lanes;
+}
+constexpr unsigned norm_groups(int n, int dPad) {
+    const int rows = kNormThreads / norm_lanes(dPad);
+    return (unsigned)(((long long)n + rows - 1) / rows);
+}
+constexpr bool norms_fit_one_launch(int first, int second, int dPad) {
+    return ((unsigned long long)norm_groups(first, dPad) + norm_groups(second, dPad)) * kNormThreads < 1ull << 32;
+}
 hipError_t launch_sum_squared(const NormPoints& first, const NormPoints* second, int dPad, float eps2, unsigned long long* counters,
                               hipStream_t stream, unsigned long long epoch = 1, Reset reset = Reset::kNothing);
 // The same halves from norms that are already there.

@@ -149,7 +149,7 @@ struct NormSet {
     int n;
     float *sums, *halves;
 };
-__global__ void __launch_bounds__(256) sum_squared_kernel(NormSet a, NormSet b, unsigned firstGroups, int chunksPerRow, int lanesPerRow,
+__global__ void __launch_bounds__(kNormThreads) sum_squared_kernel(NormSet a, NormSet b, unsigned firstGroups, int chunksPerRow, int lanesPerRow,
                                                           float quarterEps2, unsigned long long* __restrict__ counters,
                                                           unsigned long long epoch, int reset) {
     if (reset) reset_for_join(counters, reset);
@@ -1203,15 +1203,14 @@ float quarter_eps2(float eps2) { return (eps2 != eps2 ? -3.0e38f : (eps2 > 3.0e3
 
 hipError_t launch_sum_squared(const NormPoints& first, const NormPoints* second, int dPad, float eps2, unsigned long long* counters,
                               hipStream_t stream, unsigned long long epoch, Reset reset) {
-    const int chunksPerRow = dPad / 8;
-    int lanesPerRow = 64;
-    while (lanesPerRow > chunksPerRow) lanesPerRow >>= 1;
-    const int rowsPerGroup = 4 * (64 / lanesPerRow);
+    if (second && !norms_fit_one_launch(first.n, second->n, dPad)) {
+        const hipError_t e = launch_sum_squared(first, nullptr, dPad, eps2, counters, stream, epoch, reset);
+        return e != hipSuccess ? e : launch_sum_squared(*second, nullptr, dPad, eps2, counters, stream, epoch);
+    }
     auto set = [](const NormPoints& p) { return NormSet{static_cast<const u32x4*>(p.points), p.ld / 8, p.n, p.sums, p.halves}; };
-    auto groups = [&](const NormPoints& p) { return (unsigned)(((long long)p.n + rowsPerGroup - 1) / rowsPerGroup); };
-    const unsigned firstGroups = groups(first);
-    sum_squared_kernel<<<dim3(firstGroups + (second ? groups(*second) : 0u)), dim3(256), 0, stream>>>(
-        set(first), second ? set(*second) : NormSet{}, firstGroups, chunksPerRow, lanesPerRow, quarter_eps2(eps2), counters, epoch, (int)reset);
+    const unsigned firstGroups = norm_groups(first.n, dPad), groups = firstGroups + (second ? norm_groups(second->n, dPad) : 0u);
+    sum_squared_kernel<<<dim3(groups), dim3(kNormThreads), 0, stream>>>(set(first), second ? set(*second) : NormSet{}, firstGroups, dPad / 8,
+                                                                       norm_lanes(dPad), quarter_eps2(eps2), counters, epoch, (int)reset);
     return hipGetLastError();
 }
 

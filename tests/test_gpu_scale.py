@@ -116,3 +116,25 @@ def test_config5_output_heavy_2m_x_384(env):
 
 def test_config3_headline_1m_x_4096(env):
     run_config(env, "c3", sample_rows=1024, oracle_rows=4)
+
+
+def test_two_sets_whose_norms_do_not_fit_one_launch(env):
+    """One query and 67 108 860 candidates of 512 dimensions: as many workgroups of the norm kernel as a launch can hold for
+    the candidates alone, and one more for the query."""
+    torch, _, fasted = env
+    n, d = 67_108_860, 512
+    if torch.cuda.mem_get_info()[0] < 80 << 30:
+        pytest.skip("needs 70 GB of device memory")
+    points = torch.zeros((n, d), dtype=torch.float16, device="cuda")
+    query = torch.ones((1, d), dtype=torch.float16, device="cuda")
+    near = torch.tensor([0, 255, 256, n // 2, n - 1], device="cuda")
+    points[near] = 1.0
+    sq, sc = torch.empty(1, device="cuda"), torch.full((n,), -1.0, device="cuda")
+    pairs = torch.full((16, 2), -1, dtype=torch.int32, device="cuda")
+    st = fasted.join_device(query.data_ptr(), 1, d, points.data_ptr(), n, d, d, 0.5, pairs.data_ptr(), 16, flags=fp.FASTED_SORT_PAIRS,
+                            sums_queries_ptr=sq.data_ptr(), sums_candidates_ptr=sc.data_ptr())
+    assert st.pairsFound == st.pairsStored == len(near)
+    assert torch.equal(pairs[: len(near), 1].long(), near) and bool((pairs[: len(near), 0] == 0).all())
+    assert float(sq[0]) == d and bool((sc[near] == d).all()) and float(sc.double().sum()) == d * len(near)
+    del points, sc
+    torch.cuda.empty_cache()
