@@ -369,7 +369,7 @@ void join_on_device(PointSet q, PointSet c, bool selfJoin, int d, double epsilon
         }
     }
     cnt[1] = (jl.epilogue && cnt[0] > cap) ? cap : cnt[0];
-    if (polled && tiles > 512 && cnt[1] < 2) HIP_CHECK(hipStreamSynchronize(stream));  // (no sort that would)
+    if (polled && (flags & FASTED_SORT_PAIRS) && cnt[1] < 2) HIP_CHECK(hipStreamSynchronize(stream));  // (no sort that would)
     cnt[2] = tiles;
     if (jl.triangle == fasted::Triangle::kUpper) {
         const unsigned long long side = ((unsigned long long)q.n + fasted::kTile - 1) / fasted::kTile;

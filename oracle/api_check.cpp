@@ -6,6 +6,7 @@
 // `make -C oracle asan`; run with the name of a check.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdint>
 #include <cstdio>
@@ -14,6 +15,7 @@
 #include <functional>
 #include <map>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "../fasted_amd/csrc/join_kernels.h"
@@ -209,7 +211,27 @@ void check_norms_of_two_large_sets() {
     CHECK(!norms_fit_one_launch(34000000, 34000000, 512) && norms_fit_one_launch(34000000, 33000000, 512));
 }
 
+// A sorted call returns with its stream drained, however few pairs there are to sort and whoever reported them.
+void check_sorted_joins_drain_the_stream() {
+    const hipStream_t stream = reinterpret_cast<hipStream_t>(&world);
+    // up to 512 tiles, more, more than report themselves; hit bits
+    for (auto [nQ, nC] : {std::pair<long long, long long>{256, 30000}, {30000, 256}, {30000, 2560}, {30000, 400000}, {300, 300}})
+        for (unsigned long long found : {0ull, 1ull, 2ull, 4ull})
+            for (unsigned more : {0u, (unsigned)FASTED_EVENT_TIMING})
+                for (bool wantStats : {true, false}) {
+                    world.found = found;
+                    alignas(16) static char points[64];
+                    FastedPair pairs[4];
+                    FastedJoinStats st{};
+                    CHECK(fasted_join_device(points, nQ, 64, points, nC, 64, 64, 1.0, nullptr, nullptr, pairs, 4, FASTED_SORT_PAIRS | more, stream,
+                                             wantStats ? &st : nullptr) == 0);
+                    CHECK(world.underWay.count(stream) == 0);
+                    CHECK(!wantStats || st.pairsStored == found);
+                }
+}
+
 const std::map<std::string, std::function<void()>> kChecks = {
+    {"sorted_joins_drain_the_stream", check_sorted_joins_drain_the_stream},
     {"norms_of_two_large_sets", check_norms_of_two_large_sets},
 };
 
