@@ -337,8 +337,9 @@ void join_on_device(PointSet q, PointSet c, bool selfJoin, int d, double epsilon
     jl.bits = bits;
     fasted::BitsLayout layout;
     HIP_CHECK(fasted::launch_join(jl, stream, &layout));
-    if (events) HIP_CHECK(hipEventRecord(t.ev[2], stream));
+    // (the list is part of the join, as appending the pairs is in the reference's kernel)
     if (bits) HIP_CHECK(fasted::launch_expand_bits(bits, layout, (int)q.n, (int)c.n, counters, dPairs, cap, stream));
+    if (events) HIP_CHECK(hipEventRecord(t.ev[2], stream));
     // c[0] = pairs found; every slot below the capacity received exactly one pair, the rest were
     // counted only (source/pair.cuh:123-133), so stored = min(found, capacity)
     unsigned long long cnt[4] = {0, 0, 0, 0};
@@ -376,10 +377,7 @@ void join_on_device(PointSet q, PointSet c, bool selfJoin, int d, double epsilon
         cnt[2] = side * (side + 1) / 2;
     }
     float sortMs = 0.f;
-    if (bits) {
-        const volatile unsigned long long* const w = g_ws.hostCount;  // [3] its kernel started, [4] and was through
-        if (w[3] != 0 && w[4] > w[3]) sortMs = (float)((double)(w[4] - w[3]) / g_ws.clockKHz());
-    } else if ((flags & FASTED_SORT_PAIRS) && cnt[1] > 1) {
+    if (!bits && (flags & FASTED_SORT_PAIRS) && cnt[1] > 1) {
         const auto w0 = std::chrono::steady_clock::now();
         const hipError_t e = fasted::sort_pairs_row_major(dPairs, cnt[1], stream, &g_sortWs, 0, q.n, c.n);
         if (e != hipSuccess) {
@@ -391,10 +389,11 @@ void join_on_device(PointSet q, PointSet c, bool selfJoin, int d, double epsilon
     }
     if (stats) {
         if (stamped) {
-            const volatile unsigned long long* const w = g_ws.hostCount;  // [1] norms start, [2] join start, [3] join over
+            const volatile unsigned long long* const w = g_ws.hostCount;  // [1] norms start, [2] join start, [3] join over, [4] list over
             const bool reportedTimes = w[3] != 0;  // (no report, no clock readings: the times stay 0)
+            const unsigned long long over = w[bits ? 4 : 3];
             stats->sumSquaredMs = reportedTimes ? (float)((double)(w[2] - w[1]) / g_ws.clockKHz()) : 0.f;
-            stats->joinMs = reportedTimes ? (float)((double)(w[3] - w[2]) / g_ws.clockKHz()) : 0.f;
+            stats->joinMs = reportedTimes ? (float)((double)(over - w[2]) / g_ws.clockKHz()) : 0.f;
         } else {
             stats->sumSquaredMs = t.ms(0, 1);
             stats->joinMs = t.ms(1, 2);

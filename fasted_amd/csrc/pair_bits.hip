@@ -174,6 +174,8 @@ __global__ void __launch_bounds__(kThreads, 8) expand_bits_kernel(const unsigned
             }
         }
     }
+    // The last workgroup to start stands for the last to end.  (With a reading by every workgroup, or by the one with the most
+    // records as well, a call of 1000 x 64 took 26.4 us instead of 25.9, of 9733 x 257 69.5 instead of 68.6.)
     if (band + 1 == gridDim.x) {
         __syncthreads();
         if (threadIdx.x == 0) {

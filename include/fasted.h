@@ -75,13 +75,15 @@ void releaseResources(void);
  * (source/findPairs.cuh:625-639,695-697); for joins of at most 131 072 tiles of 256 x 256, where three event
  * records would cost up to a third of the call, they are differences of the device's constant-rate clock, read by the kernels
  * themselves (hipDeviceAttributeWallClockRate ticks): by the first norm kernel and the join kernel as they start,
- * and by the join kernel's last workgroup when it has nothing left to do (sorted: by the kernel that makes the list, as
- * it starts). */
+ * and by the join kernel's last workgroup when it has nothing left to do. */
 typedef struct FastedJoinStats {
     float sumSquaredMs; /* squared-norm pre-pass (which also clears the counters): its start to the join kernel's start */
-    float joinMs;       /* the join kernel: its start to the event behind it (without events: to its last workgroup's report) */
-    float sortMs;       /* host wall time of the row-major sort, stream synchronisation included (0 when not sorted); up to
-                           20 224 points a side, where the list is made in order, the device's time of the kernel that does it */
+    float joinMs;       /* the join kernel: its start to the event behind it (without events: to its last workgroup's report).
+                           A sorted join of up to 20 224 points a side writes its pairs, in order, in a kernel of its own
+                           behind that: up to the event behind this kernel then (without events: to the end of its last
+                           workgroup, which writes the last rows) */
+    float sortMs;       /* host wall time of the row-major sort, stream synchronisation included (0 when there is none: not
+                           sorted, fewer than two pairs, or written in order) */
     int paddedN;        /* rows covered by the tile grid */
     int paddedD;        /* K extent the kernel looped over */
     unsigned long long tiles;      /* size of the distance matrix in 256x256 tiles (with FASTED_SYMMETRIC: those on and

@@ -230,7 +230,30 @@ void check_sorted_joins_drain_the_stream() {
                 }
 }
 
+// The join's time spans the writing of its pairs, whoever writes them and whatever it is timed with; a sort is not part of it.
+void check_join_time_spans_the_writing_of_the_pairs() {
+    alignas(16) static char points[64];
+    FastedPair pairs[4];
+    auto near = [](double a, double b) { return std::fabs(a - b) < 1e-3; };
+    for (unsigned long long found : {0ull, 3ull})
+        for (unsigned more : {0u, (unsigned)FASTED_EVENT_TIMING, (unsigned)FASTED_FULL_MATRIX})
+            for (long long n : {100, 5000, 20224, 20225, 90000, 200000}) {
+                world.found = found;
+                world.sorts = 0;
+                const int listsBefore = world.lists;
+                FastedJoinStats st{};
+                CHECK(fasted_self_join_device(points, n, 64, 64, 1.0, nullptr, pairs, 4, FASTED_SORT_PAIRS | more, nullptr, &st) == 0);
+                const bool list = n <= 20224;
+                CHECK(world.lists - listsBefore == (list ? 1 : 0) && world.sorts == (!list && found > 1 ? 1 : 0));
+                CHECK(near(st.sumSquaredMs, kNormsMs) && near(st.joinMs, kJoinMs + (list ? kListMs : 0.0)));
+                CHECK(!list || st.sortMs == 0.0f);
+                CHECK(fasted_self_join_device(points, n, 64, 64, 1.0, nullptr, pairs, 4, more, nullptr, &st) == 0);
+                CHECK(near(st.sumSquaredMs, kNormsMs) && near(st.joinMs, kJoinMs) && st.sortMs == 0.0f);
+            }
+}
+
 const std::map<std::string, std::function<void()>> kChecks = {
+    {"join_time_spans_the_writing_of_the_pairs", check_join_time_spans_the_writing_of_the_pairs},
     {"sorted_joins_drain_the_stream", check_sorted_joins_drain_the_stream},
     {"norms_of_two_large_sets", check_norms_of_two_large_sets},
 };

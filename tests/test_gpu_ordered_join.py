@@ -47,7 +47,8 @@ def test_lists_of_every_density(n, d, share):
         st = fasted.self_join_device(pts.data_ptr(), n, d, ld, eps2**0.5, pairs.data_ptr(), cap, flags=flags | fp.FASTED_SORT_PAIRS)
         assert st.pairsFound == st.pairsStored == len(want), flags
         assert torch.equal(pairs[: len(want)], want) and bool((pairs[len(want) :] == -1).all()), flags
-        assert st.joinMs > 0 and st.sumSquaredMs > 0 and st.sortMs >= 0
+        # the list is part of the join, and 8 bytes a pair take their time at 8 TB/s
+        assert st.joinMs > len(want) * 8 / 8e9 and st.sumSquaredMs > 0 and st.sortMs == 0
     # a buffer that is too small holds the beginning of the list; what lies behind it is left alone
     small = max(1, len(want) // 3)
     pairs = torch.full((cap, 2), -1, dtype=torch.int32, device="cuda")

@@ -28,7 +28,8 @@ def test_host_code_is_clean_under_address_and_ub_sanitizers():
 # what api_check checks: each fault here needs memory that is refused, a wait that fails or a set no test could hold, or is a
 # launch or a wait that a caller on the GPU cannot see
 @pytest.mark.skipif(not os.path.exists(CLANG) or shutil.which("make") is None, reason="clang with sanitizer runtimes not installed")
-@pytest.mark.parametrize("check", ["norms_of_two_large_sets", "sorted_joins_drain_the_stream"])
+@pytest.mark.parametrize("check", ["norms_of_two_large_sets", "sorted_joins_drain_the_stream",
+                                   "join_time_spans_the_writing_of_the_pairs"])
 def test_host_orchestration(check):
     build = subprocess.run(["make", "-C", os.path.join(ROOT, "oracle"), "_asan/api_check"], capture_output=True, text=True, timeout=600)
     assert build.returncode == 0, build.stdout[-2000:] + build.stderr[-2000:]
