@@ -974,8 +974,10 @@ Results find_pairs_resident(double epsilon, bool savePairs, bool skipUpload, con
     const PointSet all{g_res.dPoints, tb.n, tb.dPad, nullptr};
     // a sort that fails (no memory for its buffers) is reported and the pairs leave unsorted, as the
     // reference carries on after "Failed to sort pairs" (source/findPairs.cuh:701-718).  The whole matrix is
-    // computed: Results.TFLOPS divides 2*N*N*D by the kernel time and means operations that were executed.
-    join_on_device(all, all, true, tb.dPad, epsilon, dPairs, maxPairs, FASTED_SORT_PAIRS | FASTED_FULL_MATRIX, nullptr, &st,
+    // computed: Results.TFLOPS divides 2*N*N*D by the kernel time and means operations that were executed.  The time is
+    // that between events, as there, for all but the smallest joins, whose calls three event records would lengthen by a third.
+    const unsigned timing = fasted::tile_count(tb.n, tb.n) > 512 ? FASTED_EVENT_TIMING : 0u;
+    join_on_device(all, all, true, tb.dPad, epsilon, dPairs, maxPairs, FASTED_SORT_PAIRS | FASTED_FULL_MATRIX | timing, nullptr, &st,
                    nullptr, /*sortMayFail=*/true);
     if (!quiet()) {
         std::printf("Number of pairs found %llu\n", st.pairsFound);

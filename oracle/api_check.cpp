@@ -33,7 +33,8 @@ static int failures = 0;
 // ---- the stand-in ------------------------------------------------------------------------
 namespace {
 
-constexpr double kNormsMs = 1.0, kJoinMs = 10.0, kListMs = 5.0, kSortMs = 3.0;  // what a launch takes
+constexpr double kNormsMs = 1.0, kJoinMs = 10.0, kListMs = 5.0, kSortMs = 3.0;  // what a kernel takes
+constexpr double kDispatchMs = 0.25;                                            // and what its launch does, before it
 constexpr int kClockKHz = 100000;
 
 struct World {
@@ -132,6 +133,7 @@ void SortBuffers::release() {}
 
 hipError_t launch_sum_squared(const NormPoints&, const NormPoints*, int, float, unsigned long long* counters, hipStream_t s,
                               unsigned long long, Reset reset) {
+    world.now += kDispatchMs;
     if (counters && reset != Reset::kNothing) counters[2] = ticks();
     world.now += kNormsMs;
     ++world.underWay[s];
@@ -155,6 +157,7 @@ hipError_t launch_pair_distances(const void*, long long, int, const void*, long 
 }
 hipError_t launch_join(const JoinLaunch& l, hipStream_t s, BitsLayout*) {
     world.joins.push_back(l);
+    world.now += kDispatchMs;
     unsigned long long* const w = host_words(l.counters);
     if (w) {
         w[1] = l.counters[2];
@@ -174,6 +177,7 @@ hipError_t launch_join(const JoinLaunch& l, hipStream_t s, BitsLayout*) {
 hipError_t launch_expand_bits(const unsigned*, const BitsLayout&, int, int, unsigned long long* counters, void* pairs, unsigned long long cap,
                               hipStream_t s) {
     ++world.lists;
+    world.now += kDispatchMs;
     unsigned long long* const w = host_words(counters);
     write_pairs(pairs, cap);
     w[0] = counters[0] = world.found;
@@ -243,16 +247,32 @@ void check_join_time_spans_the_writing_of_the_pairs() {
                 const int listsBefore = world.lists;
                 FastedJoinStats st{};
                 CHECK(fasted_self_join_device(points, n, 64, 64, 1.0, nullptr, pairs, 4, FASTED_SORT_PAIRS | more, nullptr, &st) == 0);
-                const bool list = n <= 20224;
+                const bool list = n <= 20224, events = more & FASTED_EVENT_TIMING || n > 92672;
+                const double before = events ? kDispatchMs : 0.0, between = events ? 0.0 : kDispatchMs;
                 CHECK(world.lists - listsBefore == (list ? 1 : 0) && world.sorts == (!list && found > 1 ? 1 : 0));
-                CHECK(near(st.sumSquaredMs, kNormsMs) && near(st.joinMs, kJoinMs + (list ? kListMs : 0.0)));
+                CHECK(near(st.sumSquaredMs, before + kNormsMs + between) &&
+                      near(st.joinMs, before + kJoinMs + (list ? kDispatchMs + kListMs : 0.0)));
                 CHECK(!list || st.sortMs == 0.0f);
                 CHECK(fasted_self_join_device(points, n, 64, 64, 1.0, nullptr, pairs, 4, more, nullptr, &st) == 0);
-                CHECK(near(st.sumSquaredMs, kNormsMs) && near(st.joinMs, kJoinMs) && st.sortMs == 0.0f);
+                CHECK(near(st.sumSquaredMs, before + kNormsMs + between) && near(st.joinMs, before + kJoinMs) && st.sortMs == 0.0f);
             }
 }
 
+// Results.TFLOPS: 2 N^2 D over the time between events, as the reference has it, for all but the smallest joins, whose calls
+// three event records would lengthen by a third.
+void check_results_are_timed_with_events() {
+    world.found = 3;
+    for (int n : {300, 5632, 5633, 20225}) {
+        const Results r = runFromExponentialDataset(n, 2, 40.0, 1.0, 0.1, false);
+        const double list = n <= 20224 ? kDispatchMs + kListMs : 0.0;
+        const double ms = kDispatchMs + kNormsMs + kJoinMs + list + (n <= 5632 ? 0.0 : kDispatchMs);
+        CHECK(std::fabs(r.TFLOPS * ms / (2.0 * n * n * 2 / 1e9) - 1.0) < 1e-4);
+        CHECK(r.pairsFound == 3 && r.pairsStored == 3);
+    }
+}
+
 const std::map<std::string, std::function<void()>> kChecks = {
+    {"results_are_timed_with_events", check_results_are_timed_with_events},
     {"join_time_spans_the_writing_of_the_pairs", check_join_time_spans_the_writing_of_the_pairs},
     {"sorted_joins_drain_the_stream", check_sorted_joins_drain_the_stream},
     {"norms_of_two_large_sets", check_norms_of_two_large_sets},
