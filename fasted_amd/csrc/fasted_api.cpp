@@ -977,7 +977,7 @@ Results find_pairs_resident(double epsilon, bool savePairs, bool skipUpload, con
     // computed: Results.TFLOPS divides 2*N*N*D by the kernel time and means operations that were executed.  The time is
     // that between events, as there, for all but the smallest joins, whose calls three event records would lengthen by a third.
     const unsigned timing = fasted::tile_count(tb.n, tb.n) > 512 ? FASTED_EVENT_TIMING : 0u;
-    join_on_device(all, all, true, tb.dPad, epsilon, dPairs, maxPairs, FASTED_SORT_PAIRS | FASTED_FULL_MATRIX | timing, nullptr, &st,
+    join_on_device(all, all, true, tb.d, epsilon, dPairs, maxPairs, FASTED_SORT_PAIRS | FASTED_FULL_MATRIX | timing, nullptr, &st,
                    nullptr, /*sortMayFail=*/true);
     if (!quiet()) {
         std::printf("Number of pairs found %llu\n", st.pairsFound);
@@ -1114,7 +1114,7 @@ FastedJoinStats count_resident(double epsilon) {
     const fasted::PointTable& tb = g_res.table;
     FastedJoinStats st{};
     const PointSet all{g_res.dPoints, tb.n, tb.dPad, nullptr};
-    join_on_device(all, all, true, tb.dPad, epsilon, nullptr, 0, FASTED_SYMMETRIC, nullptr, &st);
+    join_on_device(all, all, true, tb.d, epsilon, nullptr, 0, FASTED_SYMMETRIC, nullptr, &st);
     return st;
 }
 
@@ -1141,7 +1141,7 @@ FastedJoinStats count_resident_sampled(double epsilon, int sampleRows) {
     FastedJoinStats st{};
     const PointSet sample{g_res.dSample, sampleRows, tb.dPad, nullptr};
     const PointSet all{g_res.dPoints, tb.n, tb.dPad, nullptr};
-    join_on_device(sample, all, false, tb.dPad, epsilon, nullptr, 0, 0, nullptr, &st, nullptr, false,
+    join_on_device(sample, all, false, tb.d, epsilon, nullptr, 0, 0, nullptr, &st, nullptr, false,
                    /*forcedStride=*/tb.n / sampleRows);
     return st;
 }

@@ -43,6 +43,7 @@ struct World {
     std::vector<fasted::JoinLaunch> joins;
     int lists = 0, sorts = 0;
     unsigned long long found = 0;              // pairs of the next joins: the first of a row-major list of 0/1 columns
+    unsigned foundPerQuery = 0;                // where set, `found` follows the number of query points
     size_t refuseFrom = ~(size_t)0;            // device allocations of so many bytes are refused
     int eventWaitsToFail = 0;                  // after how many waits for an event one fails (0: none)
     int pinnedAllocations = 0;
@@ -157,6 +158,7 @@ hipError_t launch_pair_distances(const void*, long long, int, const void*, long 
 }
 hipError_t launch_join(const JoinLaunch& l, hipStream_t s, BitsLayout*) {
     world.joins.push_back(l);
+    if (world.foundPerQuery) world.found = (unsigned long long)world.foundPerQuery * l.nQ;
     world.now += kDispatchMs;
     unsigned long long* const w = host_words(l.counters);
     if (w) {
@@ -271,7 +273,46 @@ void check_results_are_timed_with_events() {
     }
 }
 
+// Every entry tells the join how many dimensions there are, so that none multiplies padding where a kernel can leave it out.
+void check_every_join_is_told_the_dimensionality() {
+    constexpr int n = 700, d = 65, dPad = 128;
+    std::vector<uint16_t> points((size_t)n * dPad, 0);
+    FastedPair pairs[4];
+    unsigned long long found = 0, stored = 0;
+    double epsilon = 0.0, selectivity = 0.0;
+    int probes = 0, rows = 0;
+    const std::function<void()> entries[] = {
+        [&] { (void)runFromExponentialDataset(n, d, 40.0, 1.0, 0.1, false); },
+        [&] { (void)reRun(0.2, false); },
+        [&] { CHECK(fasted_count_pairs(0.1, &found, nullptr) == 0); },
+        [&] { CHECK(fasted_count_pairs_sampled(0.1, 100, &found, &rows, nullptr) == 0); },
+        [&] { CHECK(fasted_find_epsilon(1.0, 0.1, &epsilon, &selectivity, &probes) == 0); },
+        [&] { CHECK(fasted_find_epsilon_sampled(1.0, 0.1, 100, &epsilon, &selectivity, &probes) == 0); },
+        [&] { CHECK(fasted_find_epsilon_volumetric(1.0, 0.1, &epsilon, &selectivity, &probes) == 0); },
+        [&] { CHECK(fasted_self_join(points.data(), n, d, 0.1, pairs, 4, &found, &stored) == 0); },
+        [&] { CHECK(fasted_self_join_blocked(points.data(), n, d, 0.1, 256, pairs, 4, &found, &stored) == 0); },
+        [&] { CHECK(fasted_self_join_device(points.data(), n, d, dPad, 0.1, nullptr, pairs, 4, 0, nullptr, nullptr) == 0); },
+        [&] { CHECK(fasted_self_join_device_noalloc(points.data(), n, d, dPad, 0.1, pairs, 4, 0, nullptr, nullptr) == 0); },
+        [&] { CHECK(fasted_join_device(points.data(), n, dPad, points.data(), n, dPad, d, 0.1, nullptr, nullptr, pairs, 4, 0, nullptr, nullptr) == 0); },
+    };
+    int entry = 0;
+    for (const auto& call : entries) {
+        world.joins.clear();
+        world.foundPerQuery = 2;  // (the selectivity the searches look for)
+        call();
+        CHECK(!world.joins.empty());
+        for (const fasted::JoinLaunch& l : world.joins)
+            if (l.d != d || l.dPad != dPad) {
+                std::fprintf(stderr, "entry %d: %d dimensions of %d\n", entry, l.d, l.dPad);
+                ++failures;
+                break;
+            }
+        ++entry;
+    }
+}
+
 const std::map<std::string, std::function<void()>> kChecks = {
+    {"every_join_is_told_the_dimensionality", check_every_join_is_told_the_dimensionality},
     {"results_are_timed_with_events", check_results_are_timed_with_events},
     {"join_time_spans_the_writing_of_the_pairs", check_join_time_spans_the_writing_of_the_pairs},
     {"sorted_joins_drain_the_stream", check_sorted_joins_drain_the_stream},
