@@ -515,11 +515,11 @@ private:
 std::atomic<HostJoinBuffer::Block*> HostJoinBuffer::kept_{nullptr};
 
 // Two pieces of pinned host memory through which results leave the device: one piece travels while the other is copied to
-// the caller's buffer.  Kept like the buffer above: at most one pair, taken out by a call that works with it.  (Straight into
-// pageable memory, 9 MB took 540 us to come down, 173 into pinned memory and 131 from there.  Whole host joins, without ->
-// with: 30000 x 200 with 9 MB of pairs 1369 -> 1224 us, 50000 x 100 with 47 MB 3761 -> 2696 in pieces of 2 MB, 2826 of 4, 3363
-// of 0.5; with 1.0 MB 137 -> 144, hence the limit below.  The way up is left to the runtime: 12 MB in 350 us, 390 through
-// pinned memory.)
+// the caller's buffer.  Kept like the buffer above: at most one pair, taken out by a call that works with it, and freed
+// instead where that call fails.  (Straight into pageable memory, 9 MB took 540 us to come down, 173 into pinned memory and
+// 131 from there.  Whole host joins, without -> with: 30000 x 200 with 9 MB of pairs 1369 -> 1224 us, 50000 x 100 with 47 MB
+// 3761 -> 2696 in pieces of 2 MB, 2826 of 4, 3363 of 0.5; with 1.0 MB 137 -> 144, hence the limit below.  The way up is left
+// to the runtime: 12 MB in 350 us, 390 through pinned memory.)
 class PinnedPieces {
 public:
     PinnedPieces() {
@@ -537,10 +537,13 @@ public:
     }
     PinnedPieces(const PinnedPieces&) = delete;
     PinnedPieces& operator=(const PinnedPieces&) = delete;
-    ~PinnedPieces() { delete kept_.exchange(pieces_.release()); }
+    ~PinnedPieces() {
+        if (through_) delete kept_.exchange(pieces_.release());
+    }
     static void release() { delete kept_.exchange(nullptr); }
 
     void download(void* to, const void* from, size_t bytes, hipStream_t stream) {
+        through_ = false;
         auto send = [&](size_t at) {
             const int slot = (int)(at / kPiece % 2);
             HIP_CHECK(hipMemcpyAsync(piece(slot), static_cast<const char*>(from) + at, std::min(kPiece, bytes - at), hipMemcpyDeviceToHost, stream));
@@ -553,6 +556,7 @@ public:
             HIP_CHECK(hipEventSynchronize(pieces_->landed[slot]));
             std::memcpy(static_cast<char*>(to) + at, piece(slot), std::min(kPiece, bytes - at));
         }
+        through_ = true;
     }
 
 private:
@@ -573,6 +577,7 @@ private:
     void* piece(int slot) const { return static_cast<char*>(pieces_->memory) + (size_t)slot * kPiece; }
     static inline std::atomic<Pieces*> kept_{nullptr};
     std::unique_ptr<Pieces> pieces_;
+    bool through_ = true;  // no transfer is under way: the pieces may be kept
 };
 
 // Device -> pageable host memory, behind what the stream holds.

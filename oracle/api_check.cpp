@@ -311,7 +311,41 @@ void check_every_join_is_told_the_dimensionality() {
     }
 }
 
+// Pinned pieces with a transfer that nobody has waited for are not used again: not by the next call, and not by one that
+// follows on another stream.
+void check_a_failed_download_gives_up_its_pieces() {
+    constexpr int n = 4000;
+    constexpr unsigned long long cap = 1000000;  // 8 MB, four pieces
+    std::vector<uint16_t> points((size_t)n * 64, 0);
+    std::vector<FastedPair> pairs(cap);
+    unsigned long long found = 0, stored = 0;
+    world.found = cap;
+    auto join = [&](bool blocked) {
+        std::fill(pairs.begin(), pairs.end(), FastedPair{-1, -1});
+        return blocked ? fasted_self_join_blocked(points.data(), n, 64, 1.0, 8192, pairs.data(), cap, &found, &stored)
+                       : fasted_self_join(points.data(), n, 64, 1.0, pairs.data(), cap, &found, &stored);
+    };
+    auto whole = [&] {
+        for (unsigned long long i = 0; i < cap; ++i)
+            if (pairs[i].QueryPoint != (int)(i / 2) || pairs[i].CandidatePoint != (int)(i % 2)) return false;
+        return true;
+    };
+    for (bool blocked : {false, true}) {
+        CHECK(join(blocked) == 0 && stored == cap && whole());
+        const int allocations = world.pinnedAllocations;
+        const size_t held = world.pinned.size();
+        CHECK(join(blocked) == 0 && whole() && world.pinnedAllocations == allocations);  // kept
+        for (int wait : {1, 2, 4}) {
+            const int before = world.pinnedAllocations;
+            world.eventWaitsToFail = wait;
+            CHECK(join(blocked) != 0 && world.pinned.size() == held - 1);
+            CHECK(join(blocked) == 0 && whole() && world.pinnedAllocations == before + 1 && world.pinned.size() == held);
+        }
+    }
+}
+
 const std::map<std::string, std::function<void()>> kChecks = {
+    {"a_failed_download_gives_up_its_pieces", check_a_failed_download_gives_up_its_pieces},
     {"every_join_is_told_the_dimensionality", check_every_join_is_told_the_dimensionality},
     {"results_are_timed_with_events", check_results_are_timed_with_events},
     {"join_time_spans_the_writing_of_the_pairs", check_join_time_spans_the_writing_of_the_pairs},
