@@ -530,7 +530,11 @@ public:
         if (!p) {
             p = std::make_unique<Pieces>();
             p->device = device;
-            HIP_CHECK(hipHostMalloc(&p->memory, 2 * kPiece, hipHostMallocDefault));
+            if (hipHostMalloc(&p->memory, 2 * kPiece, hipHostMallocDefault) != hipSuccess) {
+                (void)hipGetLastError();
+                p->memory = nullptr;
+                return;
+            }
             for (auto& e : p->landed) HIP_CHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
         }
         pieces_ = std::move(p);
@@ -538,8 +542,9 @@ public:
     PinnedPieces(const PinnedPieces&) = delete;
     PinnedPieces& operator=(const PinnedPieces&) = delete;
     ~PinnedPieces() {
-        if (through_) delete kept_.exchange(pieces_.release());
+        if (pieces_ && through_) delete kept_.exchange(pieces_.release());
     }
+    bool there() const { return pieces_ != nullptr; }  // (there may be no memory for them)
     static void release() { delete kept_.exchange(nullptr); }
 
     void download(void* to, const void* from, size_t bytes, hipStream_t stream) {
@@ -582,12 +587,12 @@ private:
 
 // Device -> pageable host memory, behind what the stream holds.
 void download(void* to, const void* from, size_t bytes, hipStream_t stream) {
-    if (bytes < (size_t)4 << 20) {
-        HIP_CHECK(hipMemcpyAsync(to, from, bytes, hipMemcpyDeviceToHost, stream));
-        HIP_CHECK(hipStreamSynchronize(stream));
-        return;
+    if (bytes >= (size_t)4 << 20) {
+        PinnedPieces pieces;
+        if (pieces.there()) return pieces.download(to, from, bytes, stream);
     }
-    PinnedPieces().download(to, from, bytes, stream);
+    HIP_CHECK(hipMemcpyAsync(to, from, bytes, hipMemcpyDeviceToHost, stream));
+    HIP_CHECK(hipStreamSynchronize(stream));
 }
 
 // Self-join of a host-resident dataset that is streamed through the device in blocks of `blockRows`

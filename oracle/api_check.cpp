@@ -47,6 +47,7 @@ struct World {
     size_t refuseFrom = ~(size_t)0;            // device allocations of so many bytes are refused
     int eventWaitsToFail = 0;                  // after how many waits for an event one fails (0: none)
     int pinnedAllocations = 0;
+    size_t refusePinnedFrom = ~(size_t)0;      // pinned allocations of so many bytes are refused
     std::map<void*, size_t> pinned;
 } world;
 
@@ -101,6 +102,7 @@ hipError_t hipMalloc(void** p, size_t bytes) {
 }
 hipError_t hipFree(void* p) { world.underWay.clear(); std::free(p); return hipSuccess; }
 hipError_t hipHostMalloc(void** p, size_t bytes, unsigned) {
+    if (bytes >= world.refusePinnedFrom) return hipErrorOutOfMemory;
     *p = std::calloc(1, bytes);
     world.pinned[*p] = bytes;
     ++world.pinnedAllocations;
@@ -344,7 +346,21 @@ void check_a_failed_download_gives_up_its_pieces() {
     }
 }
 
+// Long lists come down without pinned memory where there is none to be had.
+void check_lists_come_down_without_pinned_memory() {
+    constexpr int n = 1000;
+    constexpr unsigned long long cap = 700000;  // 5.6 MB
+    std::vector<uint16_t> points((size_t)n * 64, 0);
+    std::vector<FastedPair> pairs(cap, FastedPair{-1, -1});
+    unsigned long long found = 0, stored = 0;
+    world.found = cap;
+    world.refusePinnedFrom = (size_t)1 << 20;
+    CHECK(fasted_self_join(points.data(), n, 64, 1.0, pairs.data(), cap, &found, &stored) == 0 && stored == cap);
+    for (unsigned long long i = 0; i < cap && failures == 0; ++i) CHECK(pairs[i].QueryPoint == (int)(i / 2) && pairs[i].CandidatePoint == (int)(i % 2));
+}
+
 const std::map<std::string, std::function<void()>> kChecks = {
+    {"lists_come_down_without_pinned_memory", check_lists_come_down_without_pinned_memory},
     {"a_failed_download_gives_up_its_pieces", check_a_failed_download_gives_up_its_pieces},
     {"every_join_is_told_the_dimensionality", check_every_join_is_told_the_dimensionality},
     {"results_are_timed_with_events", check_results_are_timed_with_events},
