@@ -99,29 +99,18 @@ __host__ __device__ __forceinline__ int swz(int row) { return lds_swizzle128(row
 // -15 %).  Fewer points are taken in strips, without places for tiles that are not there (launch_join).
 // An XCD whose queue is exhausted takes from the next XCD's queue, so the tail stays balanced.
 typedef TileOrder Raster;
-constexpr int kSubTiles = 32;  // per sub-rectangle: the workgroups resident on one XCD
+constexpr unsigned kSquaresFrom = 64;  // rows of tiles; launch_join
 static_assert(kSubTiles * kQueues == kSquareTiles, "8 sub-rectangles tile a super-square");
-template <bool kTall>
-struct SubShape {
-    static constexpr int rows = kTall ? 8 : 4, cols = kTall ? 4 : 8;
-};
+constexpr int kSubRows = 8, kSubCols = 4;
+static_assert(kSubRows * kSubCols == kSubTiles, "a sub-rectangle is one XCD's share");
 
-// (the host's mirror keeps 4 x 8 sub-rectangles, 16 x 16 super-squares, for matrices of fewer than 64 rows of tiles)
-inline bool tall_order(long long nQueries, int tileRows = kTile) {
-    return (nQueries + tileRows - 1) / tileRows >= 64;
+inline Raster make_raster(long long nQueries, long long nCandidates, bool upperOnly, int tileRows = kTile) {
+    return make_tile_order(nQueries, nCandidates, tileRows, kTile, kSubRows, kSubCols, upperOnly);
 }
 
-inline Raster make_raster(long long nQueries, long long nCandidates, bool upperOnly = false, int tileRows = kTile) {
-    const bool tall = tall_order(nQueries, tileRows);
-    return tall ? make_tile_order(nQueries, nCandidates, tileRows, kTile, SubShape<true>::rows, SubShape<true>::cols, upperOnly)
-                : make_tile_order(nQueries, nCandidates, tileRows, kTile, SubShape<false>::rows, SubShape<false>::cols, upperOnly);
-}
-
-inline void raster_decode(const Raster& r, bool tall, unsigned q, unsigned long long t, unsigned* tr, unsigned* tc) {
-    if (tall)
-        tile_order_decode(r, SubShape<true>::rows, SubShape<true>::cols, q, t, tr, tc);
-    else
-        tile_order_decode(r, SubShape<false>::rows, SubShape<false>::cols, q, t, tr, tc);
+// Tiles of a matrix, or of its upper triangle.
+inline unsigned long long tiles_of(const Raster& r, bool upperOnly) {
+    return upperOnly ? (unsigned long long)r.tileRows * (r.tileRows + 1) / 2 : (unsigned long long)r.tileRows * r.tileCols;
 }
 
 // ------------------------------------------------------------------------------------------
@@ -453,7 +442,7 @@ __global__ void __launch_bounds__(kThreads, 1) join_kernel(JoinParams p) {
             const unsigned total = upperOnly ? ras.tileRows * (ras.tileRows + 1) / 2 : ras.tileRows * ras.tileCols;
 #pragma clang loop unroll(disable)
             for (;;) {
-                const unsigned long long number = pos / kSubTiles * (kQueues * kSubTiles) + q * kSubTiles + pos % kSubTiles;
+                const unsigned long long number = tile_strip_number(q, pos);
                 if (number < total) {
                     tile_strip_decode((unsigned)number, ras.tileRows, ras.tileCols, upperOnly, row, col);
                     home = q;
@@ -467,7 +456,7 @@ __global__ void __launch_bounds__(kThreads, 1) join_kernel(JoinParams p) {
         for (;;) {
             if (pos < ras.perQueue) {
                 unsigned tr, tc;
-                tile_order_decode(ras, SubShape<true>::rows, SubShape<true>::cols, q, pos, &tr, &tc);
+                tile_order_decode(ras, kSubRows, kSubCols, q, pos, &tr, &tc);
                 if (tr < ras.tileRows && tc < ras.tileCols && !(upperOnly && tc < tr)) {
                     *row = tr;
                     *col = tc;
@@ -1157,19 +1146,30 @@ __global__ void __launch_bounds__(kThreads, 1) join_kernel(JoinParams p) {
 
 }  // namespace
 
+// Fewer than 64 rows of tiles: strips; otherwise super-squares, the order of points that fill more than 32 MB (launch_join).
+static bool mirrors_strips(const Raster& r) { return r.tileRows < kSquaresFrom; }
+
 unsigned long long raster_count(long long nQ, long long nC, bool upperOnly) {
-    return make_raster(nQ, nC, upperOnly).perQueue * kQueues;
+    const Raster r = make_raster(nQ, nC, upperOnly);
+    if (!mirrors_strips(r)) return r.perQueue * kQueues;
+    constexpr unsigned long long round = kQueues * kSubTiles;
+    return (tiles_of(r, upperOnly) + round - 1) / round * round;
 }
 
 // Index idx enumerates the queues round-robin: queue idx % 8, position idx / 8 -- the order in
-// which eight equally fast XCDs would take the tiles.  Returns 0 past the end, 2 for a padding
+// which eight equally fast XCDs would take the tiles.  Returns 0 past the end, 2 for a position without a
 // tile that the kernel skips, 1 for a real tile.
 // With upperOnly (symmetric self-join) the tiles below the diagonal count as skipped as well.
 int raster_coord(unsigned long long idx, long long nQ, long long nC, bool upperOnly, int* row, int* col) {
     const Raster r = make_raster(nQ, nC, upperOnly);
-    if (idx >= r.perQueue * kQueues) return 0;
-    unsigned tr, tc;
-    raster_decode(r, tall_order(nQ), (unsigned)(idx % kQueues), idx / kQueues, &tr, &tc);
+    if (idx >= raster_count(nQ, nC, upperOnly)) return 0;
+    unsigned tr = r.tileRows, tc = r.tileCols;  // (the queues' last positions in strips are nowhere)
+    if (!mirrors_strips(r)) {
+        tile_order_decode(r, kSubRows, kSubCols, (unsigned)(idx % kQueues), idx / kQueues, &tr, &tc);
+    } else {
+        const unsigned long long number = tile_strip_number((unsigned)(idx % kQueues), idx / kQueues);
+        if (number < tiles_of(r, upperOnly)) tile_strip_decode((unsigned)number, r.tileRows, r.tileCols, upperOnly, &tr, &tc);
+    }
     *row = (int)tr * kTile;
     *col = (int)tc * kTile;
     return (tr < r.tileRows && tc < r.tileCols && !(upperOnly && tc < tr)) ? 1 : 2;
@@ -1189,8 +1189,7 @@ const char* build_tag() {
 }
 
 unsigned long long tile_count(long long nQ, long long nC) {
-    const Raster r = make_raster(nQ, nC);
-    return (unsigned long long)r.tileRows * r.tileCols;
+    return tiles_of(make_raster(nQ, nC, false), false);
 }
 
 int lds_chunk_slot(int row, int chunk) { return (chunk ^ swz(row)) & 7; }
@@ -1266,8 +1265,7 @@ namespace {
 // One launch of the join kernel over the tile grid described by p.raster, in the queue or the direct mode, with
 // tiles of 256 or 128 query rows.
 hipError_t launch_join_grid(JoinParams p, bool rows128, bool squares, bool epilogue, bool halfTail, int numCUs, hipStream_t stream) {
-    const unsigned long long realTiles = p.symmetric ? (unsigned long long)p.raster.tileRows * (p.raster.tileRows + 1) / 2
-                                                     : (unsigned long long)p.raster.tileRows * p.raster.tileCols;
+    const unsigned long long realTiles = tiles_of(p.raster, p.symmetric != 0);
     // Up to two tiles per CU, workgroup b computes tile b and ends, one workgroup per tile (the hardware places
     // the second round as CUs fall free); from there on, one persistent workgroup per CU draws from the queues.
     p.direct = realTiles <= 2ull * (unsigned long long)numCUs ? 1 : 0;
@@ -1406,10 +1404,10 @@ hipError_t launch_join(const JoinLaunch& launch, hipStream_t stream, BitsLayout*
     const unsigned long long rowsOfTiles = ((unsigned long long)l.nQ + tileRows - 1) / tileRows;
     const unsigned long long tileCount = rowsOfTiles * (((unsigned long long)l.nC + kTile - 1) / kTile);
     const bool fewSkipped = !p.symmetric && (32 - rowsOfTiles % 32) % 32 * 16 <= rowsOfTiles;
-    const bool squares = !l.epilogue || (!l.bits && rowsOfTiles >= 64 &&
+    const bool squares = !l.epilogue || (!l.bits && rowsOfTiles >= kSquaresFrom &&
                                          (fewSkipped || (p.symmetric && rowsOfTiles > 128) ||
                                           (unsigned long long)l.nQ * l.dPad * 2 > 32ull << 20 || tileCount >> 32));
-    p.raster = make_tile_order(l.nQ, l.nC, tileRows, kTile, SubShape<true>::rows, SubShape<true>::cols, p.symmetric != 0);
+    p.raster = make_raster(l.nQ, l.nC, p.symmetric != 0, tileRows);
     p.bits = l.bits;
     if (layout) *layout = BitsLayout{tileRows, p.raster.tileRows, p.raster.tileCols, p.symmetric != 0};
     return launch_join_grid(p, rows128, squares, l.epilogue, l.dPad - l.d >= kSlabK / 2, numCUs, stream);

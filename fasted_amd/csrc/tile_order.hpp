@@ -18,7 +18,8 @@
 
 namespace fasted {
 
-constexpr int kQueues = 8;  // one work queue per XCD
+constexpr int kQueues = 8;     // one work queue per XCD
+constexpr int kSubTiles = 32;  // tiles that a queue takes in a row: one to each of the workgroups resident on one XCD
 
 // Work queues.  The matrix of tiles is cut into super-squares of 4 * subRows x 2 * subCols tiles; a
 // super-square is cut into 8 sub-rectangles of subRows x subCols
@@ -127,6 +128,11 @@ FASTED_INLINE void tile_strip_decode(unsigned number, unsigned rows, unsigned co
         *tr = s / width;
         *tc = 4 * strip + s % width;
     }
+}
+
+// Number, in that order, of the tile at position `pos` of queue q: 32 tiles to a queue in turn.
+FASTED_INLINE unsigned long long tile_strip_number(unsigned q, unsigned long long pos) {
+    return pos / kSubTiles * (kQueues * kSubTiles) + q * kSubTiles + pos % kSubTiles;
 }
 
 // LDS placement of operand rows.  gfx950 serves a ds_read_b128 in four phases of 16 lanes --

@@ -211,18 +211,20 @@ int fasted_check_padding_device(const void* d_points, long long n, int d, long l
  * SumSqd::ComputeSquaredSums (source/sumSquared.cuh:84-118). */
 int fasted_sum_squared_device(const void* d_points, long long n, int d, long long ld, float* d_sums, void* stream);
 
-/* Tile order of the work queues in super-squares, which is how the join kernel takes a matrix of more than 128 rows of tiles
- * or 32 MB of points, 64 rows at least (smaller ones it takes in strips without padding): writes the (row, col) origin, in points, of the
- * 256x256 tile that queue index `idx` stands for in an n-point problem.  idx enumerates the eight per-XCD
- * queues round-robin (queue idx % 8, position idx / 8).  Returns 0 past the end, 1 for a real
- * tile, 2 for a padding tile of the last raster squares (the kernel skips those).  Host-side
+/* Tile order of the work queues: writes the (row, col) origin, in points, of the 256x256 tile that queue index `idx`
+ * stands for in a self-join of n points that computes the full matrix.  idx enumerates the eight per-XCD queues
+ * round-robin (queue idx % 8, position idx / 8).  Under 64 rows of tiles the order is strips of four columns, row by
+ * row, 32 tiles to a queue in turn; from there on super-squares of 32 x 8 tiles, as the join kernel takes points of more
+ * than 32 MB.  (Points of up to 32 MB it takes in strips as well, unless their rows of tiles fill the super-squares but
+ * for a sixteenth; sorted joins of up to 20 224 points always.)  Returns 0 past the end, 1 for a real tile, 2 for a
+ * position without one (the kernel skips those).  Host-side
  * mirror of the device rasterizer, the counterpart of Raster::OnDemandRasterizer::nextChunk
  * (source/rasterizer/onDemandRasterizer.cuh:78-108). */
 int fasted_raster_coord(unsigned long long idx, long long n, int* row, int* col);
 unsigned long long fasted_raster_count(long long n);
-/* The same for a FASTED_SYMMETRIC join: only the super-squares (32 x 8 tiles) that reach the diagonal or
- * lie above it are enumerated (row by row), and tiles below the diagonal inside those squares
- * return 2 like padding tiles.  No counterpart in the reference, which always walks the full grid
+/* The same for a FASTED_SYMMETRIC join: strips hold the tiles on and above the diagonal only; of the super-squares those
+ * that reach the diagonal or lie above it are enumerated (row by row), and tiles below the diagonal inside them
+ * return 2 like padding tiles.  (Points of up to 32 MB the kernel takes in strips up to 128 rows of tiles.)  No counterpart in the reference, which always walks the full grid
  * (source/rasterizer/onDemandRasterizer.cuh:50-71). */
 int fasted_raster_coord_symmetric(unsigned long long idx, long long n, int* row, int* col);
 unsigned long long fasted_raster_count_symmetric(long long n);

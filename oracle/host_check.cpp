@@ -180,7 +180,7 @@ static void check_tile_order() {
                 }
                 CHECK(seen.size() == total);
             }
-    // the ends of the largest matrices that are taken in strips (32 MB of rows of 128 bytes, and of two sets)
+    // the ends of large matrices: a triangle (eight times the rows that are taken in strips), and two sets with nearly 2^32 tiles
     for (unsigned back : {1u, 2u, 3u}) {
         unsigned r = 0, c = 0;
         fasted::tile_strip_decode(1024u * 1025u / 2 - back, 1024, 1024, true, &r, &c);

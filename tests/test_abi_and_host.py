@@ -221,38 +221,50 @@ def test_symmetric_tile_queues_cover_the_upper_triangle_exactly_once(lib, n):
         square_rows, square_cols = -(-tiles // 32), -(-tiles // 8)
         expected = 256 * sum(square_cols - 4 * i for i in range(square_rows))
     else:
-        # small matrices: 16 x 16 super-squares, the upper triangle of them
-        squares = -(-tiles // 16)
-        expected = 256 * squares * (squares + 1) // 2
+        # fewer points: strips, which have no places but the tiles' own, 32 to a queue in turn
+        expected = 256 * -(-(tiles * (tiles + 1) // 2) // 256)
     assert total == expected <= lib.fasted_raster_count(n)
 
 
 def test_tile_queue_locality(lib):
-    """32 consecutive positions of one queue are one block of tiles (one XCD's share of a super-square), the 8
-    queues together tile that super-square, and consecutive super-squares follow each other along the
-    candidates (the query panels stay).  Matrices of 64 x 64 tiles and more: blocks of 8 x 4, super-squares of
-    32 x 8; smaller ones: 4 x 8 and 16 x 16."""
+    """Matrices of 64 x 64 tiles and more: 32 consecutive positions of one queue are one block of 8 x 4 tiles (one XCD's
+    share of a super-square), the 8 queues together tile that super-square of 32 x 8, and consecutive super-squares follow
+    each other along the candidates (the query panels stay)."""
     row, col = ctypes.c_int(), ctypes.c_int()
-    for n_tiles, (br, bc), expected in ((96, (8, 4), [(0, 0), (0, 8), (0, 32), (32, 0), (32, 8)]),
-                                       (48, (4, 8), [(0, 0), (0, 16), (16, 16), (32, 0), (32, 16)])):
-        n = 256 * n_tiles
-        origins = []
-        squares = (0, 1, 4, 12, 13) if n_tiles == 96 else (0, 1, 4, 6, 7)
-        for square in squares:
-            cover = set()
-            for q in range(8):
-                block = []
-                for t in range(32):
-                    idx = (square * 32 + t) * 8 + q
-                    assert lib.fasted_raster_coord(idx, n, ctypes.byref(row), ctypes.byref(col)) == 1
-                    block.append((row.value // 256, col.value // 256))
-                r0, c0 = block[0]
-                assert block == [(r0 + t // bc, c0 + t % bc) for t in range(32)]
-                cover |= set(block)
-            rs, cs = min(r for r, _ in cover), min(c for _, c in cover)
-            assert cover == {(rs + i, cs + j) for i in range(4 * br) for j in range(2 * bc)}
-            origins.append((rs, cs))
-        assert origins == expected
+    n, br, bc = 256 * 96, 8, 4
+    origins = []
+    for square in (0, 1, 4, 12, 13):
+        cover = set()
+        for q in range(8):
+            block = []
+            for t in range(32):
+                idx = (square * 32 + t) * 8 + q
+                assert lib.fasted_raster_coord(idx, n, ctypes.byref(row), ctypes.byref(col)) == 1
+                block.append((row.value // 256, col.value // 256))
+            r0, c0 = block[0]
+            assert block == [(r0 + t // bc, c0 + t % bc) for t in range(32)]
+            cover |= set(block)
+        rs, cs = min(r for r, _ in cover), min(c for _, c in cover)
+        assert cover == {(rs + i, cs + j) for i in range(4 * br) for j in range(2 * bc)}
+        origins.append((rs, cs))
+    assert origins == [(0, 0), (0, 8), (0, 32), (32, 0), (32, 8)]
+
+
+@pytest.mark.parametrize("n_tiles,symmetric", [(5, False), (48, False), (63, False), (5, True), (48, True), (63, True)])
+def test_tile_queue_order_of_strips(lib, n_tiles, symmetric):
+    """Fewer than 64 rows of tiles: strips of four columns, row by row, of which the queues take 32 tiles in turn."""
+    coord = lib.fasted_raster_coord_symmetric if symmetric else lib.fasted_raster_coord
+    count = lib.fasted_raster_count_symmetric if symmetric else lib.fasted_raster_count
+    order = [(r, c) for first in range(0, n_tiles, 4) for r in range(n_tiles) for c in range(first, min(first + 4, n_tiles))
+             if r <= c or not symmetric]
+    row, col = ctypes.c_int(), ctypes.c_int()
+    for idx in range(count(256 * n_tiles)):
+        q, t = idx % 8, idx // 8
+        number = t // 32 * 256 + q * 32 + t % 32
+        kind = coord(idx, 256 * n_tiles, ctypes.byref(row), ctypes.byref(col))
+        assert kind == (1 if number < len(order) else 2)
+        if kind == 1:
+            assert (row.value // 256, col.value // 256) == order[number]
 
 
 # ---------------------------------------------------------------- LDS swizzle (host mirror)
