@@ -340,7 +340,6 @@ __device__ __forceinline__ void static_for(F&& f) {
 template <bool kEpilogue, bool kSquares, int kTileRows, bool kOneSlab, bool kBitsInLastSlab = false, bool kMirror = false,
           bool kHalfTail = false, bool kBits = false>
 __global__ void __launch_bounds__(kThreads, 1) join_kernel(JoinParams p) {
-    static_assert(kEpilogue || kSquares, "without the epilogue, squares");
     static_assert(!kMirror || (kEpilogue && kTileRows == 256), "pairs are mirrored across the diagonal of square tiles");
     const bool upperOnly = kEpilogue ? kMirror : p.symmetric != 0;
     static_assert(!kBits || kEpilogue, "hit bits come from the epilogue");
@@ -1295,10 +1294,14 @@ hipError_t launch_join_grid(JoinParams p, bool rows128, bool squares, bool epilo
             default: join_kernel<true, false, 256, true, true, true, true, true><<<g, b, 0, stream>>>(p); break;
         }
     } else if (!epilogue) {
-        switch ((oneSlab ? 2 : 0) + (rows128 ? 1 : 0)) {
-            case 0: join_kernel<false, true, 256, false><<<g, b, 0, stream>>>(p); break;
-            case 1: join_kernel<false, true, 128, false><<<g, b, 0, stream>>>(p); break;
-            case 2: join_kernel<false, true, 256, true><<<g, b, 0, stream>>>(p); break;
+        switch ((rows128 ? 4 : 0) + (squares ? 2 : 0) + (oneSlab ? 1 : 0)) {
+            case 0: join_kernel<false, false, 256, false><<<g, b, 0, stream>>>(p); break;
+            case 1: join_kernel<false, false, 256, true><<<g, b, 0, stream>>>(p); break;
+            case 2: join_kernel<false, true, 256, false><<<g, b, 0, stream>>>(p); break;
+            case 3: join_kernel<false, true, 256, true><<<g, b, 0, stream>>>(p); break;
+            case 4: join_kernel<false, false, 128, false><<<g, b, 0, stream>>>(p); break;
+            case 5: join_kernel<false, false, 128, true><<<g, b, 0, stream>>>(p); break;
+            case 6: join_kernel<false, true, 128, false><<<g, b, 0, stream>>>(p); break;
             default: join_kernel<false, true, 128, true><<<g, b, 0, stream>>>(p); break;
         }
     } else if (p.symmetric) {
@@ -1404,9 +1407,8 @@ hipError_t launch_join(const JoinLaunch& launch, hipStream_t stream, BitsLayout*
     const unsigned long long rowsOfTiles = ((unsigned long long)l.nQ + tileRows - 1) / tileRows;
     const unsigned long long tileCount = rowsOfTiles * (((unsigned long long)l.nC + kTile - 1) / kTile);
     const bool fewSkipped = !p.symmetric && (32 - rowsOfTiles % 32) % 32 * 16 <= rowsOfTiles;
-    const bool squares = !l.epilogue || (!l.bits && rowsOfTiles >= kSquaresFrom &&
-                                         (fewSkipped || (p.symmetric && rowsOfTiles > 128) ||
-                                          (unsigned long long)l.nQ * l.dPad * 2 > 32ull << 20 || tileCount >> 32));
+    const bool squares = !l.bits && rowsOfTiles >= kSquaresFrom &&
+                         (fewSkipped || (p.symmetric && rowsOfTiles > 128) || (unsigned long long)l.nQ * l.dPad * 2 > 32ull << 20 || tileCount >> 32);
     p.raster = make_raster(l.nQ, l.nC, p.symmetric != 0, tileRows);
     p.bits = l.bits;
     if (layout) *layout = BitsLayout{tileRows, p.raster.tileRows, p.raster.tileCols, p.symmetric != 0};

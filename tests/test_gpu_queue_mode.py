@@ -176,3 +176,20 @@ def test_last_slab_with_one_and_two_steps(fasted, n, d):
                             flags=fp.FASTED_SORT_PAIRS)
     two = want[(want[:, 0] < m) & (want[:, 1] >= m)] - torch.tensor([0, m], dtype=torch.int32, device="cuda")
     assert st.pairsFound == len(two) and torch.equal(pairs[: len(two)], two)
+
+
+# one workgroup per tile, strips and super-squares; one slab and more; the full matrix, the triangle and the smaller tiles
+@pytest.mark.parametrize("n,d", [(1000, 64), (3000, 100), (7001, 64), (7001, 200), (17000, 64), (17000, 1088)])
+def test_contraction_alone_ends_and_finds_nothing(fasted, n, d, monkeypatch):
+    import torch
+    from fasted_amd import find_pairs as fp
+
+    ld = (d + 63) // 64 * 64
+    pts = torch.zeros((n, ld), dtype=torch.float16, device="cuda")
+    pairs = torch.full((64, 2), -1, dtype=torch.int32, device="cuda")
+    for rows in ("256", "128"):
+        monkeypatch.setenv("FASTED_TILE_ROWS", rows)
+        for flags in (0, fp.FASTED_SYMMETRIC, fp.FASTED_SORT_PAIRS, fp.FASTED_EVENT_TIMING):
+            st = fasted.self_join_device(pts.data_ptr(), n, d, ld, 1.0, pairs.data_ptr(), len(pairs), flags=flags | fp.FASTED_NO_EPILOGUE)
+            assert st.pairsFound == st.pairsStored == 0 and st.joinMs > 0
+    assert bool((pairs == -1).all())
