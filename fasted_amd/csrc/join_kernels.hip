@@ -1294,15 +1294,13 @@ hipError_t launch_join_grid(JoinParams p, bool rows128, bool squares, bool epilo
             default: join_kernel<true, false, 256, true, true, true, true, true><<<g, b, 0, stream>>>(p); break;
         }
     } else if (!epilogue) {
-        switch ((rows128 ? 4 : 0) + (squares ? 2 : 0) + (oneSlab ? 1 : 0)) {
+        switch (rows128 ? 4 + (oneSlab ? 1 : 0) : (squares ? 2 : 0) + (oneSlab ? 1 : 0)) {
             case 0: join_kernel<false, false, 256, false><<<g, b, 0, stream>>>(p); break;
             case 1: join_kernel<false, false, 256, true><<<g, b, 0, stream>>>(p); break;
             case 2: join_kernel<false, true, 256, false><<<g, b, 0, stream>>>(p); break;
             case 3: join_kernel<false, true, 256, true><<<g, b, 0, stream>>>(p); break;
             case 4: join_kernel<false, false, 128, false><<<g, b, 0, stream>>>(p); break;
-            case 5: join_kernel<false, false, 128, true><<<g, b, 0, stream>>>(p); break;
-            case 6: join_kernel<false, true, 128, false><<<g, b, 0, stream>>>(p); break;
-            default: join_kernel<false, true, 128, true><<<g, b, 0, stream>>>(p); break;
+            default: join_kernel<false, false, 128, true><<<g, b, 0, stream>>>(p); break;
         }
     } else if (p.symmetric) {
         switch ((squares ? 8 : 0) + variant) {
@@ -1318,13 +1316,10 @@ hipError_t launch_join_grid(JoinParams p, bool rows128, bool squares, bool epilo
             default: join_kernel<true, true, 256, true, true, true, true><<<g, b, 0, stream>>>(p); break;
         }
     } else if (rows128) {
-        switch ((squares ? 4 : 0) + k) {
+        switch (k) {
             case 0: join_kernel<true, false, 128, false><<<g, b, 0, stream>>>(p); break;
             case 1: join_kernel<true, false, 128, false, true><<<g, b, 0, stream>>>(p); break;
-            case 2: join_kernel<true, false, 128, true, true><<<g, b, 0, stream>>>(p); break;
-            case 4: join_kernel<true, true, 128, false><<<g, b, 0, stream>>>(p); break;
-            case 5: join_kernel<true, true, 128, false, true><<<g, b, 0, stream>>>(p); break;
-            default: join_kernel<true, true, 128, true, true><<<g, b, 0, stream>>>(p); break;
+            default: join_kernel<true, false, 128, true, true><<<g, b, 0, stream>>>(p); break;
         }
     } else {
         switch ((squares ? 8 : 0) + variant) {
@@ -1390,7 +1385,7 @@ hipError_t launch_join(const JoinLaunch& launch, hipStream_t stream, BitsLayout*
     const char* const forced = getenv("FASTED_TILE_ROWS");  // read at every launch: a test sets it per case
     const int forcedRows = forced ? atoi(forced) : 0;
     if (forcedRows == 256) rows128 = false;
-    if (forcedRows == 128) rows128 = true;
+    if (forcedRows == 128) rows128 = tiles128 >> 32 == 0;
     if (mayMirror && l.triangle == Triangle::kUpper) rows128 = false;
     p.symmetric = (mayMirror && !rows128) ? 1 : 0;
     const int tileRows = rows128 ? 128 : kTile;
@@ -1407,7 +1402,7 @@ hipError_t launch_join(const JoinLaunch& launch, hipStream_t stream, BitsLayout*
     const unsigned long long rowsOfTiles = ((unsigned long long)l.nQ + tileRows - 1) / tileRows;
     const unsigned long long tileCount = rowsOfTiles * (((unsigned long long)l.nC + kTile - 1) / kTile);
     const bool fewSkipped = !p.symmetric && (32 - rowsOfTiles % 32) % 32 * 16 <= rowsOfTiles;
-    const bool squares = !l.bits && rowsOfTiles >= kSquaresFrom &&
+    const bool squares = !l.bits && !rows128 && rowsOfTiles >= kSquaresFrom &&
                          (fewSkipped || (p.symmetric && rowsOfTiles > 128) || (unsigned long long)l.nQ * l.dPad * 2 > 32ull << 20 || tileCount >> 32);
     p.raster = make_raster(l.nQ, l.nC, p.symmetric != 0, tileRows);
     p.bits = l.bits;
