@@ -1,6 +1,7 @@
 """GPU parity of the row-major order of the stored pairs, at the counts and distributions where the sort takes another path:
 one workgroup, one and two levels of buckets, buckets too full for the LDS, crowded cells, keys of more than 32 bits, lists
-that a level breaks off, the radix sort behind them.  tests/test_sort_routes.py holds the lists to these paths."""
+that a level breaks off, the radix sort behind them.  tests/test_sort_routes.py holds the lists to these paths, and to more
+points than a join may have whose list is made in order without a sort."""
 import ctypes
 
 import numpy as np
@@ -22,6 +23,14 @@ def _coded(values):
     return pts, v
 
 
+MAX_BIT_ROWS = 20224  # points of either side up to which no sort follows the join
+
+
+def _to_be_sorted(q, c):
+    """The same pairs, in a join of enough candidates that they are sorted."""
+    return q, np.concatenate([c, 3000000 + np.arange(MAX_BIT_ROWS + 1 - len(c))])
+
+
 def _hub(n, row, share):
     q = np.arange(n) + 1
     q[row] = 0
@@ -36,15 +45,15 @@ def _rand(nq, nc, distinct):
 
 
 CASES = {
-    "two records": lambda: (np.array([7]), np.array([7, 7])),
-    "the last count of one workgroup": lambda: (np.zeros(64, int), np.zeros(128, int)),
-    "the first of one level": lambda: (np.zeros(1, int), np.zeros(8193, int)),
-    "the last of one level": lambda: (np.zeros(1024, int), np.zeros(1024, int)),
-    "the first of two levels": lambda: (np.zeros(1025, int), np.zeros(1024, int)),
-    "a small join of runs": lambda: (np.arange(1000) // 8, np.arange(1000) // 8),
-    "one level of runs": lambda: (np.arange(9000) // 90, np.arange(9000) // 90),
+    "two records": lambda: _to_be_sorted(np.array([7]), np.array([7, 7])),
+    "the last count of one workgroup": lambda: _to_be_sorted(np.zeros(64, int), np.zeros(128, int)),
+    "the first of one level": lambda: _to_be_sorted(np.zeros(1, int), np.zeros(8193, int)),
+    "the last of one level": lambda: _to_be_sorted(np.zeros(1024, int), np.zeros(1024, int)),
+    "the first of two levels": lambda: _to_be_sorted(np.zeros(1025, int), np.zeros(1024, int)),
+    "a small join of runs": lambda: _to_be_sorted(np.arange(1000) // 8, np.arange(1000) // 8),
+    "one level of runs": lambda: _to_be_sorted(np.arange(9000) // 90, np.arange(9000) // 90),
     "two levels of runs": lambda: (np.arange(40000) // 70, np.arange(40000) // 70),
-    "one level, a crowded row": lambda: _hub(20011, 4321, 0.7),
+    "one level, a crowded row": lambda: _to_be_sorted(*_hub(20011, 4321, 0.7)),
     "two levels, a crowded row": lambda: tuple(np.concatenate(x) for x in zip(_hub(30011, 20000, 0.9), _rand(5000, 30000, 100))),
     "a row too crowded for one workgroup": lambda: tuple(np.concatenate(x) for x in zip(_hub(300, 7, 1.0), ([], np.zeros(1000000, int)))),
     "few records, long keys": lambda: _rand(40000, 70001, 500000),
@@ -72,6 +81,7 @@ def _check(qv, cv, calls=2):
         assert st.pairsFound == st.pairsStored == len(want)
         assert torch.equal(pairs[:-1], want)
         assert int(pairs[-1].abs().sum()) == 0
+        assert st.sortMs > 0  # the list was sorted, not made in order
         sort_ms.append(st.sortMs)
     return min(sort_ms)
 
@@ -123,7 +133,7 @@ def test_crowded_lists_are_row_major_and_leave_the_sort_as_it_was(name):
     import fasted_amd as fasted
     from fasted_amd.find_pairs import FASTED_SORT_PAIRS
 
-    ordinary = _groups(20000, 10.0)
+    ordinary = _groups(30000, 10.0)
     for qv, cv in (sort_routes.CASES[name][0](), ordinary, sort_routes.CASES[name][0]()):
         want = torch.from_numpy(sort_routes.pairs_of(qv, cv)).cuda()
         (q, _), (c, _) = _coded(qv), _coded(cv)
@@ -133,6 +143,7 @@ def test_crowded_lists_are_row_major_and_leave_the_sort_as_it_was(name):
         assert st.pairsFound == st.pairsStored == len(want)
         assert torch.equal(pairs[:-1], want)
         assert int(pairs[-1].abs().sum()) == 0
+        assert st.sortMs > 0
 
 
 def test_crowded_rows_of_a_later_query_block_are_row_major():

@@ -30,6 +30,7 @@ LISTS = {**test_gpu_pair_sort.CASES, **test_gpu_pair_sort.SPARSE}
 
 def _route(qv, cv):
     qv, cv = np.asarray(qv).astype(np.int64), np.asarray(cv).astype(np.int64)
+    assert max(len(qv), len(cv)) > test_gpu_pair_sort.MAX_BIT_ROWS
     return sort_routes.route(sort_routes.pairs_of(qv, cv), len(qv), len(cv))
 
 
