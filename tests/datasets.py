@@ -53,3 +53,8 @@ def epsilon_for_neighbours(bits, mean_neighbours, sample=512, seed=99):
     flat = np.partition(d2.reshape(-1), k)[: k + 1]
     lo, hi = np.sort(flat)[-2:]
     return float(np.sqrt(max(0.5 * (lo + hi), 0.0)))
+
+
+def row_major(pairs):
+    """Pair records (a torch tensor of two columns) that came in any order, row-major."""
+    return pairs[(pairs[:, 0].long() << 32 | pairs[:, 1].long()).argsort()]

@@ -124,7 +124,7 @@ def test_native_epsilon_search_matches_the_python_procedure(lib):
 def test_count_only_probe_equals_the_full_join_count(lib, n, d):
     """The count-only probe computes the tiles on and above the diagonal only and doubles what it finds off the
     diagonal; a storing reRun computes the whole matrix.  The two counts must be equal at every epsilon (144 tiles
-    one per workgroup, and 6241 tiles through the queues in the tall order)."""
+    one per workgroup, and 6241 tiles through the queues)."""
     import fasted_amd
 
     assert lib.fasted_load_exponential_dataset(n, d, 40.0, 10.0) == 0

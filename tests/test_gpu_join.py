@@ -406,15 +406,16 @@ def test_join_is_deterministic_over_many_tiles_per_workgroup(fasted):
     assert int((rel > 1e-3).sum()) == 0, (int(diff.sum()), float(rel.max()))
 
 
-def test_tall_tile_order_exact_pair_sets(fasted):
-    """From 64 x 64 tiles on, the work queues walk super-squares of 32 x 8 tiles.  Integer coordinates make the
-    join exact, so on a ragged matrix of 65 x 65 tiles the full matrix, its upper triangle (upper part of
-    the tall super-squares, mirrored) and a rectangular two-set join (65 x 3 tiles: most super-square positions
+@pytest.mark.parametrize("n", [96 * 256 - 75, 129 * 256 + 37])
+def test_super_squares_exact_pair_sets(fasted, n):
+    """Matrices whose rows of tiles fill super-squares of 32 x 8 tiles (96 of them), and triangles of more than 128 rows of
+    tiles, are walked in those.  Integer coordinates make the join exact, so the full matrix, its upper triangle (upper
+    part of the super-squares, mirrored) and a rectangular two-set join (3 columns of tiles: most super-square positions
     are padding) must each give exactly the pair list of a blockwise FP64 computation."""
     import torch
     from fasted_amd import find_pairs as fp
 
-    n, d, nc = 64 * 256 + 37, 64, 600
+    d, nc = 64, 600
     bits = datasets.small_integers(n, d, high=3, seed=91)
     pts = torch.from_numpy(bits.view(np.int16).copy()).cuda()
     x = pts.view(torch.float16).double()
@@ -433,7 +434,7 @@ def test_tall_tile_order_exact_pair_sets(fasted):
 
     want = truth(n)
     cap = int(want.shape[0]) + 1024
-    for flags in (fp.FASTED_SORT_PAIRS | fp.FASTED_FULL_MATRIX, fp.FASTED_SORT_PAIRS | fp.FASTED_SYMMETRIC):
+    for flags in (fp.FASTED_SORT_PAIRS | fp.FASTED_FULL_MATRIX, fp.FASTED_SORT_PAIRS | fp.FASTED_SYMMETRIC, fp.FASTED_SORT_PAIRS):
         pairs = torch.empty((cap, 2), dtype=torch.int32, device="cuda")
         st = fasted.self_join_device(pts.data_ptr(), n, d, d, eps, pairs.data_ptr(), cap, flags=flags)
         assert st.pairsFound == st.pairsStored == want.shape[0]
@@ -450,8 +451,7 @@ def test_both_tile_heights_give_the_exact_pair_set(fasted, n, d, monkeypatch):
     """Matrices of few tiles are cut into tiles of 128 query rows instead of 256 (FASTED_TILE_ROWS forces either).
     Integer coordinates make the join exact: both heights, on a self-join, on a two-set join with a ragged
     query count and with non-finite points present, must give exactly the FP64 pair list.  The last shape has
-    65 tile rows of 128: the tall tile order with that height.  Self-joins with the library's choice and of the
-    full matrix."""
+    65 tile rows of 128.  Self-joins with the library's choice and of the full matrix, sorted (hit bits) and not."""
     import torch
     from fasted_amd import find_pairs as fp
 
@@ -466,9 +466,10 @@ def test_both_tile_heights_give_the_exact_pair_set(fasted, n, d, monkeypatch):
     pts = torch.from_numpy(bits.view(np.int16).copy()).cuda()
     for rows in ("256", "128"):
         monkeypatch.setenv("FASTED_TILE_ROWS", rows)
-        for flags in (fp.FASTED_SORT_PAIRS, fp.FASTED_SORT_PAIRS | fp.FASTED_FULL_MATRIX):
+        for flags in (fp.FASTED_SORT_PAIRS, fp.FASTED_SORT_PAIRS | fp.FASTED_FULL_MATRIX, 0, fp.FASTED_FULL_MATRIX):
             got, st, _ = device_join(fasted, bits, eps, flags=flags)
-            assert st.pairsFound == len(truth) and np.array_equal(got, truth), (rows, flags)
+            assert st.pairsFound == len(truth) and np.array_equal(oracle.sort_pairs(got), truth), (rows, flags)
+            assert not flags & fp.FASTED_SORT_PAIRS or np.array_equal(got, truth), (rows, flags)
         buf = torch.empty((len(truth2) + 64, 2), dtype=torch.int32, device="cuda")
         st2 = fasted.join_device(pts.data_ptr(), nq, d, pts.data_ptr(), nc, d, d, eps, buf.data_ptr(), buf.shape[0])
         assert st2.pairsFound == len(truth2) and np.array_equal(buf[: st2.pairsStored].cpu().numpy(), truth2), rows
@@ -480,9 +481,9 @@ def test_both_tile_heights_give_the_exact_pair_set(fasted, n, d, monkeypatch):
     want = want[np.lexsort((want[:, 1], want[:, 0]))]
     for rows in ("256", "128"):
         monkeypatch.setenv("FASTED_TILE_ROWS", rows)
-        for flags in (fp.FASTED_SORT_PAIRS, fp.FASTED_SORT_PAIRS | fp.FASTED_FULL_MATRIX):
+        for flags in (fp.FASTED_SORT_PAIRS, fp.FASTED_SORT_PAIRS | fp.FASTED_FULL_MATRIX, 0, fp.FASTED_FULL_MATRIX):
             got, st, _ = device_join(fasted, bad, eps, flags=flags)
-            assert np.array_equal(got, want), (rows, flags)
+            assert np.array_equal(oracle.sort_pairs(got), want), (rows, flags)
 
 
 def test_small_joins_time_themselves_with_the_device_clock(fasted):

@@ -1,6 +1,6 @@
 """GPU parity tests of mid-size matrices: more tiles than two rounds of the workgroups (so the tiles come from the
-per-XCD work queues, not one workgroup per tile), fewer than 64 tile rows (the 16 x 16 super-square order), several
-slabs per tile.  The size band of the reference's own sweep rows of 10 000 and 21 544 points
+per-XCD work queues, not one workgroup per tile), in strips and in super-squares, several slabs per tile.  A sorted join of
+up to 20 224 points leaves hit bits, an unsorted one stages its pairs: other kernels, so both are asked for.  The size band of the reference's own sweep rows of 10 000 and 21 544 points
 (results/speed_results/ExpoDataSpeedVsSize_OnDemandRasterizer.json); kernel counterpart
 source/findPairs.cuh:360-546 with source/rasterizer/onDemandRasterizer.cuh:78-108."""
 import numpy as np
@@ -32,9 +32,9 @@ def integer_case(n, d, seed, rank=10):
 
 @pytest.mark.parametrize("n,d", [(7000, 128), (7000, 320), (12000, 128), (12000, 320), (6000, 1088)])
 def test_queue_mode_exact_pair_lists(fasted, n, d, monkeypatch):
-    """784 and 2209 tiles of 256 rows (1540 and 4418 of 128 rows, the latter in the tall order), and 17 slabs (hit bits
-    behind the k-loop): the library's choice, the full matrix and the triangle, both tile heights, with and without
-    squared norms brought by the caller."""
+    """784 and 2209 tiles of 256 rows (1540 and 4418 of 128 rows), in strips, and 17 slabs (hit bits behind the k-loop):
+    the library's choice, the full matrix and the triangle, both tile heights, with and without squared norms brought by
+    the caller, sorted and not."""
     import torch
     from fasted_amd import find_pairs as fp
 
@@ -48,14 +48,15 @@ def test_queue_mode_exact_pair_lists(fasted, n, d, monkeypatch):
     fasted.sum_squared_device(pts.data_ptr(), n, d, d, sums.data_ptr())
     for rows in ("256", "128"):
         monkeypatch.setenv("FASTED_TILE_ROWS", rows)
-        for flags in (fp.FASTED_SORT_PAIRS, fp.FASTED_SORT_PAIRS | fp.FASTED_FULL_MATRIX,
-                      fp.FASTED_SORT_PAIRS | fp.FASTED_SYMMETRIC, fp.FASTED_SORT_PAIRS | fp.FASTED_SKIP_SUMS,
-                      fp.FASTED_SORT_PAIRS | fp.FASTED_FULL_MATRIX | fp.FASTED_SKIP_SUMS):
-            pairs.fill_(-1)
-            st = fasted.self_join_device(pts.data_ptr(), n, d, d, eps, pairs.data_ptr(), cap, sums_ptr=sums.data_ptr(),
-                                         flags=flags)
-            assert st.pairsFound == st.pairsStored == len(truth), (rows, flags)
-            assert np.array_equal(pairs[: st.pairsStored].cpu().numpy(), truth), (rows, flags)
+        for flags in (0, fp.FASTED_FULL_MATRIX, fp.FASTED_SYMMETRIC, fp.FASTED_SKIP_SUMS, fp.FASTED_FULL_MATRIX | fp.FASTED_SKIP_SUMS):
+            for order in (fp.FASTED_SORT_PAIRS, 0):
+                pairs.fill_(-1)
+                st = fasted.self_join_device(pts.data_ptr(), n, d, d, eps, pairs.data_ptr(), cap, sums_ptr=sums.data_ptr(),
+                                             flags=flags | order)
+                assert st.pairsFound == st.pairsStored == len(truth), (rows, flags, order)
+                got = pairs[: st.pairsStored] if order else datasets.row_major(pairs[: st.pairsStored])
+                assert np.array_equal(got.cpu().numpy(), truth), (rows, flags, order)
+                assert bool((pairs[st.pairsStored :] == -1).all())
 
 
 def test_queue_mode_two_set_exact_pair_list(fasted, monkeypatch):
@@ -79,12 +80,13 @@ def test_queue_mode_two_set_exact_pair_list(fasted, monkeypatch):
     fasted.sum_squared_device(c.data_ptr(), nc, d, d, sc.data_ptr())
     for rows in ("256", "128"):
         monkeypatch.setenv("FASTED_TILE_ROWS", rows)
-        for flags in (fp.FASTED_SORT_PAIRS, fp.FASTED_SORT_PAIRS | fp.FASTED_SKIP_SUMS):
+        for flags in (fp.FASTED_SORT_PAIRS, fp.FASTED_SORT_PAIRS | fp.FASTED_SKIP_SUMS, 0, fp.FASTED_SKIP_SUMS):
             pairs.fill_(-1)
             st = fasted.join_device(q.data_ptr(), nq, d, c.data_ptr(), nc, d, d, eps, pairs.data_ptr(), cap, flags=flags,
                                     sums_queries_ptr=sq.data_ptr(), sums_candidates_ptr=sc.data_ptr())
             assert st.pairsFound == st.pairsStored == len(want), (rows, flags)
-            assert np.array_equal(pairs[: st.pairsStored].cpu().numpy(), want), (rows, flags)
+            got = pairs[: st.pairsStored] if flags & fp.FASTED_SORT_PAIRS else datasets.row_major(pairs[: st.pairsStored])
+            assert np.array_equal(got.cpu().numpy(), want), (rows, flags)
 
 
 def test_queue_mode_band_check_exponential_10000x1024(fasted):
@@ -148,11 +150,14 @@ def test_skip_sums_needs_the_buffers_and_gives_the_same_list(fasted):
                                 flags=fp.FASTED_SKIP_SUMS)
 
 
-@pytest.mark.parametrize("d", [1, 32, 33, 65, 96, 97, 160, 992, 993])
-@pytest.mark.parametrize("n", [2900, 7001, 16500])
+# 2900: one workgroup per tile; 7001: the queues, in strips; 24500 (96 rows of tiles): the full matrix and all points against
+# some in super-squares, the triangle in strips; 33100 (130 rows): the triangle in super-squares, the full matrix in strips
+@pytest.mark.parametrize("n,d", [(n, d) for n in (2900, 7001) for d in (1, 32, 33, 65, 96, 97, 160, 992, 993)] +
+                         [(n, d) for n in (24500, 33100) for d in (24, 33, 65, 150)])
 def test_last_slab_with_one_and_two_steps(fasted, n, d):
-    """Dimensions that reach 32 columns or more into a tile's last slab, and fewer: one workgroup per tile, the queues, the
-    tall order; the triangle, the full matrix and two sets.  Integer coordinates: every sum is exact, the lists are equal."""
+    """Dimensions that reach 32 columns or more into a tile's last slab, and fewer: the triangle, the full matrix and two sets,
+    with hit bits (sorted joins of up to 20 224 points) and with staged pairs.  Integer coordinates: every sum is exact, the
+    lists are equal."""
     import torch
     from fasted_amd import find_pairs as fp
 
@@ -162,20 +167,35 @@ def test_last_slab_with_one_and_two_steps(fasted, n, d):
     pts[:, :d] = torch.randint(0, high, (n, d), generator=gen, device="cuda").to(torch.float16)
     x = pts.float()
     sq = (x * x).sum(1)
-    d2 = torch.cat([sq[r : r + 2048, None] + sq[None, :] - 2.0 * (x[r : r + 2048] @ x.T) for r in range(0, n, 2048)])
-    eps2 = float(torch.kthvalue(d2[:256].flatten(), 256 * 12).values) + 0.5
-    want = torch.nonzero(d2 <= eps2).to(torch.int32)
-    m = n // 3
+    blocks = [(r, sq[r : r + 2048, None] + sq[None, :] - 2.0 * (x[r : r + 2048] @ x.T)) for r in range(0, n, 2048)]
+    eps2 = float(torch.kthvalue(blocks[0][1][:256].flatten(), 256 * 12).values) + 0.5
+    want = torch.cat([torch.nonzero(d2 <= eps2) + torch.tensor([r, 0], device="cuda") for r, d2 in blocks]).to(torch.int32)
+    del blocks
+    assert len(want) > 2 * n
     cap = len(want) + 64
     pairs = torch.empty((cap, 2), dtype=torch.int32, device="cuda")
-    for flags in (0, fp.FASTED_FULL_MATRIX):
+
+    def check(st, expected, what):
+        assert st.pairsFound == st.pairsStored == len(expected), what
+        got = pairs[: st.pairsStored]
+        assert torch.equal(got if what[-1] else datasets.row_major(got), expected), what
+        assert bool((pairs[st.pairsStored :] == -1).all()), what
+
+    m, some = n // 3, 1000
+    lo = torch.tensor([0, m], dtype=torch.int32, device="cuda")
+    two = want[(want[:, 0] < m) & (want[:, 1] >= m)] - lo
+    against_some = want[want[:, 1] < some]
+    for order in (fp.FASTED_SORT_PAIRS, 0):
+        for flags in (0, fp.FASTED_FULL_MATRIX, fp.FASTED_SYMMETRIC):
+            pairs.fill_(-1)
+            st = fasted.self_join_device(pts.data_ptr(), n, d, ld, eps2**0.5, pairs.data_ptr(), cap, flags=flags | order)
+            check(st, want, (flags, order))
         pairs.fill_(-1)
-        st = fasted.self_join_device(pts.data_ptr(), n, d, ld, eps2**0.5, pairs.data_ptr(), cap, flags=flags | fp.FASTED_SORT_PAIRS)
-        assert st.pairsFound == len(want) and torch.equal(pairs[: len(want)], want), flags
-    st = fasted.join_device(pts.data_ptr(), m, ld, pts[m:].data_ptr(), n - m, ld, d, eps2**0.5, pairs.data_ptr(), cap,
-                            flags=fp.FASTED_SORT_PAIRS)
-    two = want[(want[:, 0] < m) & (want[:, 1] >= m)] - torch.tensor([0, m], dtype=torch.int32, device="cuda")
-    assert st.pairsFound == len(two) and torch.equal(pairs[: len(two)], two)
+        st = fasted.join_device(pts.data_ptr(), m, ld, pts[m:].data_ptr(), n - m, ld, d, eps2**0.5, pairs.data_ptr(), cap, flags=order)
+        check(st, two, ("two sets", order))
+        pairs.fill_(-1)
+        st = fasted.join_device(pts.data_ptr(), n, ld, pts.data_ptr(), some, ld, d, eps2**0.5, pairs.data_ptr(), cap, flags=order)
+        check(st, against_some, ("all against some", order))
 
 
 # one workgroup per tile, strips and super-squares; one slab and more; the full matrix, the triangle and the smaller tiles

@@ -11,7 +11,7 @@ pytestmark = pytest.mark.gpu
 
 # one tile; the last size of 128-row tiles in one round (11 x 23 of 256 workgroups) and the next; one round of the full
 # matrix in 256-row tiles and the next; 31 tile rows (496 tiles above the diagonal: one workgroup each) and 32 (528: the
-# work queues); 64 tile rows (the tall order)
+# work queues); 64 tile rows and 65.  Sorted joins of this size leave hit bits, unsorted ones stage their pairs.
 @pytest.mark.parametrize("n,d", [(1, 3), (256, 64), (2816, 64), (2817, 130), (4096, 64), (4097, 130), (7936, 64),
                                  (7937, 100), (16384, 64), (16385, 65)])
 def test_every_part_of_the_matrix_gives_the_same_pairs(n, d):
@@ -30,12 +30,13 @@ def test_every_part_of_the_matrix_gives_the_same_pairs(n, d):
     pts = torch.from_numpy(bits.view(np.int16).copy()).cuda()
     cap = 200 * n + 1024
     got = []
-    for flags in (fp.FASTED_FULL_MATRIX, 0, fp.FASTED_SYMMETRIC):
-        pairs = torch.full((cap, 2), -1, dtype=torch.int32, device="cuda")
-        st = fasted.self_join_device(pts.data_ptr(), n, d, ld, eps, pairs.data_ptr(), cap, flags=flags | fp.FASTED_SORT_PAIRS)
-        assert st.pairsFound == st.pairsStored
-        got.append(pairs[: st.pairsStored].cpu().numpy())
-    assert np.array_equal(got[0], got[1]) and np.array_equal(got[0], got[2])
+    for order in (fp.FASTED_SORT_PAIRS, 0):
+        for flags in (fp.FASTED_FULL_MATRIX, 0, fp.FASTED_SYMMETRIC):
+            pairs = torch.full((cap, 2), -1, dtype=torch.int32, device="cuda")
+            st = fasted.self_join_device(pts.data_ptr(), n, d, ld, eps, pairs.data_ptr(), cap, flags=flags | order)
+            assert st.pairsFound == st.pairsStored
+            got.append((pairs[: st.pairsStored] if order else datasets.row_major(pairs[: st.pairsStored])).cpu().numpy())
+    assert all(np.array_equal(got[0], g) for g in got[1:])
     if n <= 4097:
         assert np.array_equal(got[0], oracle.self_join_f64(bits, eps))
 
