@@ -168,7 +168,7 @@ def test_listed_distances_match_fp64(n, d, count):
     for r in range(0, len(i), step):
         j = i[r : r + step]
         want = (pts[j[:, 0], :d].double() - other[j[:, 1], :d].double()).norm(dim=1)
-        bound = 1e-7 + 0.5 * (ld / 8 + 20) * 2.0**-24  # as above, with 8 lanes to a row
+        bound = 1e-7 + 0.5 * (ld / 16 + 20) * 2.0**-24  # as above; no kernel adds more than ld / 16 products to one partial sum
         assert bool(((mine[r : r + step] - want).abs() <= bound * want).all())
 
 
@@ -203,5 +203,5 @@ def test_smallest_sliced_lists_match_fp64(d):
         ok = (i >= 0).all(1) & (i < n).all(1)
         i = i[ok]
         want = (pts[i[:, 0]].double() - pts[i[:, 1]].double()).norm(dim=1)
-        bound = 1e-7 + 0.5 * (ld / 8 + 20) * 2.0**-24  # as above, with 8 lanes to a row
+        bound = 1e-7 + 0.5 * (ld / 16 + 20) * 2.0**-24  # as above; no kernel adds more than ld / 16 products to one partial sum
         assert bool(((got[r : r + step][: len(ok)][ok].double() - want).abs() <= bound * want).all())
