@@ -359,7 +359,33 @@ void check_lists_come_down_without_pinned_memory() {
     for (unsigned long long i = 0; i < cap && failures == 0; ++i) CHECK(pairs[i].QueryPoint == (int)(i / 2) && pairs[i].CandidatePoint == (int)(i % 2));
 }
 
+// Without memory for the hit bits a sorted join of few points stages its pairs and sorts them; with it again, it leaves bits.
+void check_without_memory_for_hit_bits_the_pairs_are_sorted() {
+    alignas(16) static char points[64];
+    FastedPair pairs[4];
+    world.found = 4;
+    auto join = [&](long long n, bool inBits) {
+        const int lists = world.lists, sorts = world.sorts;
+        FastedJoinStats st{};
+        std::fill(pairs, pairs + 4, FastedPair{-1, -1});
+        CHECK(fasted_self_join_device(points, n, 64, 64, 1.0, nullptr, pairs, 4, FASTED_SORT_PAIRS, nullptr, &st) == 0);
+        CHECK(st.pairsFound == 4 && st.pairsStored == 4 && pairs[3].QueryPoint == 1 && pairs[3].CandidatePoint == 1);
+        CHECK(world.lists - lists == (inBits ? 1 : 0) && world.sorts - sorts == (inBits ? 0 : 1));
+        CHECK((world.joins.back().bits != nullptr) == inBits);
+        CHECK(std::fabs(st.joinMs - (inBits ? kJoinMs + kDispatchMs + kListMs : kJoinMs)) < 1e-3);
+    };
+    join(1000, true);
+    world.refuseFrom = (size_t)1 << 20;
+    join(1000, true);  // (the megabyte that is there does)
+    join(8000, false);
+    join(1000, false);  // (it has been given back)
+    world.refuseFrom = ~(size_t)0;
+    join(8000, true);
+    join(20224, true);
+}
+
 const std::map<std::string, std::function<void()>> kChecks = {
+    {"without_memory_for_hit_bits_the_pairs_are_sorted", check_without_memory_for_hit_bits_the_pairs_are_sorted},
     {"lists_come_down_without_pinned_memory", check_lists_come_down_without_pinned_memory},
     {"a_failed_download_gives_up_its_pieces", check_a_failed_download_gives_up_its_pieces},
     {"every_join_is_told_the_dimensionality", check_every_join_is_told_the_dimensionality},

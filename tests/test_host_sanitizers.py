@@ -31,7 +31,7 @@ def test_host_code_is_clean_under_address_and_ub_sanitizers():
 @pytest.mark.parametrize("check", ["norms_of_two_large_sets", "sorted_joins_drain_the_stream",
                                    "join_time_spans_the_writing_of_the_pairs", "results_are_timed_with_events",
                                    "every_join_is_told_the_dimensionality", "a_failed_download_gives_up_its_pieces",
-                                   "lists_come_down_without_pinned_memory"])
+                                   "lists_come_down_without_pinned_memory", "without_memory_for_hit_bits_the_pairs_are_sorted"])
 def test_host_orchestration(check):
     build = subprocess.run(["make", "-C", os.path.join(ROOT, "oracle"), "_asan/api_check"], capture_output=True, text=True, timeout=600)
     assert build.returncode == 0, build.stdout[-2000:] + build.stderr[-2000:]
