@@ -154,7 +154,7 @@ struct Workspace {
 // array instead of hipMalloc'ed memory; each GPU the library runs on holds its own copy at its own address,
 // looked up once per device.  Host code never uses the array's name as an address: only `base`.
 constexpr size_t kNoAllocMaxPoints = (size_t)1 << 22;  // 4 Mi points: 2 x 16 MiB (squared norms, accumulator start values)
-constexpr size_t kNoAllocCounterBytes = 4096;          // counter block (1152 bytes used)
+constexpr size_t kNoAllocCounterBytes = 4096;          // counter block (1280 bytes used)
 constexpr size_t kNoAllocScratchBytes = kNoAllocCounterBytes + 2 * kNoAllocMaxPoints * sizeof(float);  // norms, halves
 static __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
 

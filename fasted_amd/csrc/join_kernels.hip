@@ -1396,9 +1396,13 @@ hipError_t launch_join(const JoinLaunch& launch, hipStream_t stream, BitsLayout*
     // tiles, or 32 MB of queries (and a number of tiles that fits 32 bits) unless the squares have next to no padding, and
     // triangles of up to 128 rows.  Join kernel, squares -> strips: 9733 x 257 47.7 -> 43.4 us, 16000 x 1024 218 -> 201, 22000 x
     // 300 150 -> 143, 30000 x 200 203 -> 188, 10007 x 250000 x 200 (40 rows) 912 -> 868, 20000 x 60000 x 200 (79) 465 -> 446; but
-    // 16384 x 200000 x 384 (64 rows, two squares) 1.85 -> 1.87 ms, 100000 x 128 (391 rows) 1124 -> 1110 us on one card and 2 %
-    // slower on another, 200000 x 384, 154 MB, 12.73 -> 12.80 ms, 100000 x 4096, 819 MB, 29.8 -> 30.6.  (Strips of eight rows
-    // instead of four columns, whose queries stay in the L2: the same within 2 %, 16000 x 128 50.6 against 53.9 us.)
+    // 16384 x 200000 x 384 (64 rows, two squares) 1.85 -> 1.87 ms, 200000 x 384, 154 MB, 12.73 -> 12.80, 100000 x 4096, 819 MB,
+    // 29.8 -> 30.6.  (Strips of eight rows instead of four columns, whose queries stay in the L2: the same within 2 %, 16000 x
+    // 128 50.6 against 53.9 us.)
+    // The line for triangles lies on the safe side: one card took 2 % longer for 100000 x 128 (391 rows) in strips.  Three runs
+    // since, both orders in turn, have strips ahead up to there: 25000 x 64 (98 rows) 82 -> 73 us, 32768 x 128 (128) 163 -> 157,
+    // 33000 x 128 (129) 171 -> 161, 46416 x 128 (182) 304 -> 295, 66000 x 128 (258) 564 -> 550, 82000 x 128 (321) 819 -> 793,
+    // 100000 x 128 1155 -> 1136.  Sorted calls with 64 neighbours gain 3 % at 129 rows, 1.4 at 182, 3 at 321, and lose 0.5 at 391.
     const unsigned long long rowsOfTiles = ((unsigned long long)l.nQ + tileRows - 1) / tileRows;
     const unsigned long long tileCount = rowsOfTiles * (((unsigned long long)l.nC + kTile - 1) / kTile);
     const bool fewSkipped = !p.symmetric && (32 - rowsOfTiles % 32) % 32 * 16 <= rowsOfTiles;

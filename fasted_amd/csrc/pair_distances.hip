@@ -126,7 +126,7 @@ __global__ void __launch_bounds__(kDistThreads, kChunks <= 6 ? 6 : 5) listed_dis
 // Where the candidates fit the eight L2 caches together but not one of them: the candidates are cut into 8 slices (or a
 // multiple), and the workgroups of one XCD -- workgroups are dealt to the XCDs in turn; nothing but time depends on it --
 // look through all pairs for those of one slice, whose rows then stay in that XCD's L2.  Bound by what still misses the L2
-// (50021 x 384 with 5 million pairs, 4.8 MB to a slice: a third of the row fetches).  With a candidate row in registers ahead
+// (50021 x 384 with 5 million pairs, 4.8 MB to a slice: 16.4 of 38.6 million requests).  With a candidate row in registers ahead
 // of its turn, 16 lanes for such rows and a root per pair, of 175 million vector instructions 61 were the arithmetic: 354 -> 291
 // us; 20000 x 300 with 2 million 155 (not in slices) -> 92, 60000 x 192 with 3 million 174 (not in slices) -> 108, 5000 x 1000
 // with 500 thousand 104 (not in slices) -> 67.  Pairs put in the order of the slices first, by a kernel of its own, so that

@@ -199,7 +199,7 @@ def test_last_slab_with_one_and_two_steps(fasted, n, d):
 
 
 # one workgroup per tile, strips and super-squares; one slab and more; the full matrix, the triangle and the smaller tiles
-@pytest.mark.parametrize("n,d", [(1000, 64), (3000, 100), (7001, 64), (7001, 200), (17000, 64), (17000, 1088)])
+@pytest.mark.parametrize("n,d", [(1000, 64), (3000, 100), (7001, 64), (7001, 200), (24500, 64), (17000, 1088)])
 def test_contraction_alone_ends_and_finds_nothing(fasted, n, d, monkeypatch):
     import torch
     from fasted_amd import find_pairs as fp
