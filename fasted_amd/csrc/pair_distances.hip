@@ -266,7 +266,11 @@ hipError_t launch_pair_distances(const void* queries, long long ldQ, int nQ, con
     // 2048 with 24 700 and 975).  Less than 100 thousand pairs leave too little for every XCD (2000 x 2500 with 60 thousand 37
     // and 41; 3000 x 2000 with 120 thousand 55 and 47).  Slices of up to 5 MB: 50021 x 384 in 8 of 4.8 MB 291 us, in 16 of
     // 2.4 313; 12000 x 2048 with 1.2 million in 8 of 6.1 MB 354, in 16 of 3.1 285.
-    const bool sliced = rowBytes >= 256 && bytes >= 8ull << 20 && slices * 32 <= rowBytes &&
+    // Between 4 and 8 MB the rows that pass the L2 are few; rows of 1 KB and more pay all the same where there is much to fetch (in
+    // the order of the list, sliced: 2000 x 2000, 8.2 MB, with 400 thousand pairs 117 and 93 us, 1 million 266 and 191, in no order
+    // 509 and 357; 4000 x 800 with 1.2 million 136 and 130; but 3000 x 1000 with 600 thousand 82 and 73, near candidates 73 and 87).
+    const bool large = bytes >= 8ull << 20 || (rowBytes >= 1024 && bytes > 4ull << 20 && count * rowBytes >= 3ull << 29);
+    const bool sliced = rowBytes >= 256 && large && slices * 32 <= rowBytes &&
                         count / ((rowBytes < 1024 ? 3 : 2) * slices) >= (u64)nQ && batches >= 96 && batches * slices <= maxGroups && chunks <= 64 * 8 && addressable;
     // In the order of the list, rows of more than 192 chunks are walked by 16 lanes as well as held by 64 (50000 x 2048 with 1.2
     // million pairs 696 and 740 us, near candidates 302 and 277; 6000 x 3000 with 180 thousand 128 and 157).
