@@ -135,11 +135,11 @@ template <int kLanes, int kChunks>
 __global__ void __launch_bounds__(kDistThreads, kChunks <= 6 ? 6 : 5) sliced_distances_kernel(const u32x4* __restrict__ ptsQ, u32 ldQ16, int nQ,
                                                                       const u32x4* __restrict__ ptsC, u32 ldC16, int nC,
                                                                       int chunksPerRow, const int2* __restrict__ pairs,
-                                                                      u32 count, float* __restrict__ out,
+                                                                      u32 count, float* __restrict__ out, u32 batchPairs,
                                                                       u32 slices, int sliceRows, u32 stretch) {
-    constexpr u32 kBatch = kListCap, kPer = kBatch / kDistThreads;  // pairs a workgroup looks through
-    __shared__ RowPair found[kBatch];
-    __shared__ unsigned short where[kBatch];
+    constexpr u32 kWaves = kDistThreads / 64, kPer = kListCap / kDistThreads;
+    __shared__ RowPair found[kListCap];  // a workgroup looks through batchPairs <= kListCap pairs
+    __shared__ unsigned short where[kListCap];
     __shared__ u32 total;
     // workgroup number = ((pass * batches) + batch) * 8 + XCD, slice = pass * 8 + XCD; the XCDs go through every `stretch`
     // batches from different ones on, each from where its slice lies in a list whose candidates ascend
@@ -150,13 +150,14 @@ __global__ void __launch_bounds__(kDistThreads, kChunks <= 6 ? 6 : 5) sliced_dis
         const u32 start = batch / stretch * stretch, length = min(stretch, batches - start);
         batch = start + (batch - start + slice * length / slices) % length;
     }
-    const u32 first = batch * kBatch;
-    const u32 here = min(kBatch, count - first);
+    const u32 first = batch * batchPairs;
+    const u32 here = min(batchPairs, count - first);
     const int lane = threadIdx.x & 63;
     if (threadIdx.x == 0) total = 0;
     __syncthreads();
     {
-        const u32 waveFirst = threadIdx.x / 64 * (kBatch / (kDistThreads / 64)) + lane;
+        const u32 perWave = batchPairs / kWaves, waveFirst = threadIdx.x / 64 * perWave + lane;
+        const u32 waveEnd = min(threadIdx.x / 64 * perWave + perWave, here);
         int2 pr[kPer];
 #pragma unroll
         for (u32 e = 0; e < kPer; ++e) pr[e] = pairs[first + min(waveFirst + e * 64, here - 1)];
@@ -166,7 +167,7 @@ __global__ void __launch_bounds__(kDistThreads, kChunks <= 6 ? 6 : 5) sliced_dis
 #pragma unroll
         for (u32 e = 0; e < kPer; ++e) {
             const bool valid = pr[e].x >= 0 && pr[e].x < nQ && pr[e].y >= 0 && pr[e].y < nC;
-            const bool real = waveFirst + e * 64 < here;
+            const bool real = waveFirst + e * 64 < waveEnd;
             if (!valid && real && slice == 0) out[first + waveFirst + e * 64] = __builtin_nanf("");
             take[e] = __builtin_amdgcn_ballot_w64(real && valid && (u32)pr[e].y - slice * (u32)sliceRows < (u32)sliceRows);
             mine += __builtin_popcountll(take[e]);
@@ -288,8 +289,18 @@ hipError_t launch_pair_distances(const void* queries, long long ldQ, int nQ, con
             // whose batches take long, the XCDs then start in different places.
             const bool turned = kLanes >= 16 && count / (16 * slices) < (u64)nQ;
             const int sliceRows = (int)(((u64)nC + slices - 1) / slices);
-            sliced_distances_kernel<kLanes, kChunks><<<dim3((unsigned)(batches * slices)), dim3(kDistThreads), 0, stream>>>(
-                q, ldQ16, nQ, c, ldC16, nC, chunks, list, (u32)count, out, (u32)slices, sliceRows, turned ? kTurnPairs / kListCap : 0u);
+            // Where candidates are the query's neighbours in the set, the pairs of a slice are one piece of the list, and its
+            // batches are all the workgroups that its XCD has: less than 50 are halved, and of longer rows less than 20 again.
+            // Near candidates, batches of 1024 / 512 / 256 pairs: 3000 x 2000 with 120 thousand pairs (15 batches of 1024 to a
+            // slice) 117 / 67 / 46 us, 5000 x 4096 with 150 thousand (18) 176 / 117 / 85, 11000 x 2048 with 396 thousand (24) 197 /
+            // 140 / 115, 25000 x 2048 with 1.2 million (51) 505 / 348 / 307, 25000 x 2048 with 2 million (81) 587 / 425 / 480.
+            // Others: 47 / 45 / 44, 128 / 130 / 134, 165 / 167 / 172, 637 / 660 / 642, 823 / 865 / 797; 16000 x 384 with 800
+            // thousand (98) 57 / 61 / 74.
+            const u32 batchPairs = count >= 50ull * kListCap * slices ? kListCap
+                                   : kLanes < 32 || count >= 20ull * kListCap * slices ? kListCap / 2 : kListCap / 4;
+            const u64 groups = (count + batchPairs - 1) / batchPairs * slices;
+            sliced_distances_kernel<kLanes, kChunks><<<dim3((unsigned)groups), dim3(kDistThreads), 0, stream>>>(
+                q, ldQ16, nQ, c, ldC16, nC, chunks, list, (u32)count, out, batchPairs, (u32)slices, sliceRows, turned ? kTurnPairs / batchPairs : 0u);
         } else if constexpr (kLanes < 64) {
             // Up to four pairs to a group of 8 lanes, two to a larger one, fewer where that leaves less than 8192 waves (4000 x 64
             // with 32 thousand pairs 14.1 us with one, 14.8 with four; 60000 x 64 with 1.2 million 41 with one, 29 with four;

@@ -207,6 +207,39 @@ def test_smallest_sliced_lists_match_fp64(d):
         assert bool(((got[r : r + step][: len(ok)][ok].double() - want).abs() <= bound * want).all())
 
 
+# lists on both sides of the lines between batches of 256, 512 and 1024 pairs: rows of each number of lanes (8 to 64; up to 16 have
+# no batches of 256), candidates near the query, so that whole batches belong to a slice, and a stretch of the list in no order
+@pytest.mark.parametrize("d,count", [(d, c) for d in (300, 640, 1000, 2048) for c in (20 * 8192 - 1, 20 * 8192, 50 * 8192 - 1, 50 * 8192)])
+def test_batches_of_sliced_lists_match_fp64(d, count):
+    import torch
+
+    import fasted_amd as fasted
+
+    gen = torch.Generator(device="cuda").manual_seed(d + count)
+    ld = (d + 63) // 64 * 64
+    n = (8 << 20) // (2 * ld) + 1
+    if count < 24 * n:  # (too few for slices of short rows)
+        n = -(-count // 24)
+    pts = torch.zeros((n, ld), dtype=torch.float16, device="cuda")
+    pts[:, :d] = torch.randn((n, d), generator=gen, device="cuda").to(torch.float16)
+    q = torch.arange(count, device="cuda") * n // count
+    pairs = torch.stack([q, (q + torch.randint(-20, 21, (count,), generator=gen, device="cuda")) % n], 1).to(torch.int32)
+    pairs[2000:6000] = pairs[2000:6000][torch.randperm(4000, generator=gen, device="cuda")]
+    bad = torch.tensor([0, 255, 256, count - 2], device="cuda")
+    pairs[bad] = torch.tensor([[-1, 0], [0, n], [n, 0], [0, -1]], dtype=torch.int32, device="cuda")
+    got = torch.full((count + 1,), -2.0, dtype=torch.float32, device="cuda")
+    fasted.pair_distances_device(pts.data_ptr(), n, ld, pts.data_ptr(), n, ld, d, pairs.data_ptr(), count, got.data_ptr())
+    assert float(got[-1]) == -2.0
+    assert torch.isnan(got[bad]).all()
+    for r in range(0, count, 1 << 16):
+        i = pairs[r : r + (1 << 16)].long()
+        ok = (i >= 0).all(1) & (i < n).all(1)
+        i = i[ok]
+        want = (pts[i[:, 0]].double() - pts[i[:, 1]].double()).norm(dim=1)
+        bound = 1e-7 + 0.5 * (ld / 16 + 20) * 2.0**-24  # as above
+        assert bool(((got[r : r + (1 << 16)][: len(ok)][ok].double() - want).abs() <= bound * want).all())
+
+
 def _shortest_call(n, d, per, kind):
     """Seconds of the shortest of 20 calls for `per` pairs a query, candidates anywhere or near the query, row-major or shuffled."""
     import time
@@ -230,6 +263,12 @@ def _shortest_call(n, d, per, kind):
         fasted.pair_distances_device(pts.data_ptr(), n, ld, pts.data_ptr(), n, ld, d, pairs.data_ptr(), len(q), out.data_ptr())
         best = min(best, time.perf_counter() - t0)
     return best
+
+
+@pytest.mark.parametrize("n,d,per", [(5000, 1000, 30), (3000, 2000, 40), (5000, 4096, 30), (11000, 2048, 36)])
+def test_near_candidates_of_short_lists_take_no_longer_than_others(n, d, per):
+    # 1.2 to 2.5 times as long when a batch had 1024 pairs whatever the list
+    assert _shortest_call(n, d, per, "near") < 1.1 * _shortest_call(n, d, per, "anywhere")
 
 
 def test_long_lists_of_sets_below_8_mb_are_sliced_where_rows_are_long():
